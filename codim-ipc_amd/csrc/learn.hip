@@ -560,7 +560,6 @@ __global__ __launch_bounds__(BS) void k_lp_spmv_bf16(int nrow, int rowsPerXcd, c
                                                      V* __restrict__ y, const V* __restrict__ r, double* __restrict__ part,
                                                      const int* __restrict__ done, const int* __restrict__ cgAgg,
                                                      const double* __restrict__ cgD, const double* __restrict__ cgZ) {
-    if (done && *done) return;   // the PCG has converged: later iterations of the chunk do nothing
     __shared__ double lds[BS / 64];
     constexpr int RPG = BS / LANES;
     const int xb = blockIdx.x % 8, jb = blockIdx.x / 8, nj = gridDim.x / 8;
@@ -569,7 +568,9 @@ __global__ __launch_bounds__(BS) void k_lp_spmv_bf16(int nrow, int rowsPerXcd, c
     int g = jb;
     int row = rowBase + g * RPG;
     bool live = g * RPG < rowsPerXcd && row < nrow;
+    const int isDone = done ? *done : 0;
     int beg = live ? rp[row] : 0, end = live ? rp[row + 1] : 0;
+    if (isDone) return;   // the PCG has converged: later iterations of the chunk do nothing
     double dot = 0;
     for (; g * RPG < rowsPerXcd; g += nj) {
         const int gn = g + nj, rowN = rowBase + gn * RPG;
@@ -1139,7 +1140,12 @@ void lp_prepare(Ctx& c) {
 }
 
 constexpr int kLpSpmvBlock = 256;
-int lp_apply_partials(const Ctx& c) { return c.lpGrid; }
+// workgroups of the factor products: c.lpGrid, but no more than there are row groups (the
+// rest would only lengthen the partial sums that the SpMV's workgroups each add up)
+int lp_apply_partials(const Ctx& c) {
+    const int rpg = kLpSpmvBlock / c.lpLanes, perXcd = (c.nV + 7) / 8;
+    return std::min(c.lpGrid, 8 * ((perXcd + rpg - 1) / rpg));
+}
 
 template <int LANES, class V>
 static void lp_spmv_go(Ctx& c, const int* rp, const int* col, const uint32_t* val, int nnz, const V* x, V* y, const V* r, double* part,
@@ -1149,7 +1155,7 @@ static void lp_spmv_go(Ctx& c, const int* rp, const int* col, const uint32_t* va
     int rpx = (nV + 7) / 8;
     rpx = (rpx + RPG - 1) / RPG * RPG;
     const CoarseSpace& g = c.cg;
-    hipLaunchKernelGGL((k_lp_spmv_bf16<LANES, kLpSpmvBlock, V>), dim3(c.lpGrid), dim3(kLpSpmvBlock), 0, c.s, nV, rpx, rp, col, val, nnz,
+    hipLaunchKernelGGL((k_lp_spmv_bf16<LANES, kLpSpmvBlock, V>), dim3(lp_apply_partials(c)), dim3(kLpSpmvBlock), 0, c.s, nV, rpx, rp, col, val, nnz,
                        x, y, r, part, done, coarse ? (const int*)g.agg.p : nullptr, coarse ? (const double*)g.d.p : nullptr,
                        coarse ? (const double*)g.zc.p : nullptr);
 }
@@ -1178,7 +1184,7 @@ int lp_apply(Ctx& c, const V* r, V* z, V* tmp, double* part, bool coarse) {
     lp_spmv<V>(c, (const int*)lp.gLrp.p, (const int*)lp.gLcol.p, (const uint32_t*)lp.FL.p, lp.nLow, r, tmp, (const V*)nullptr, nullptr);
     lp_spmv<V>(c, (const int*)lp.gUrp.p, (const int*)lp.gUcol.p, (const uint32_t*)lp.FU.p, lp.nLow, (const V*)tmp, z, r, part, nullptr, coarse);
     CIPC_LAUNCH_CHECK();
-    return c.lpGrid;
+    return lp_apply_partials(c);
 }
 template int lp_apply<double>(Ctx&, const double*, double*, double*, double*, bool);
 template int lp_apply<float>(Ctx&, const float*, float*, float*, double*, bool);

@@ -70,6 +70,26 @@ __device__ __forceinline__ double block_allsum(double v, double* lds) {
     return r;
 }
 
+// A thread's share (entries i, i + BS, ...) of up to four per-workgroup partials per batch,
+// every load of a batch issued before the first add.  The adds run in index order, so the
+// sum has the same bits as a plain loop.
+template <int BS>
+struct PartialHead {
+    double v[4];
+    __device__ __forceinline__ void load(const double* __restrict__ p, int n) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = (int)threadIdx.x + k * BS < n ? p[threadIdx.x + k * BS] : 0.0;
+    }
+    __device__ __forceinline__ double finish(const double* __restrict__ p, int n) const {
+        double a = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a += v[k];
+#pragma unroll 4
+        for (int i = threadIdx.x + 4 * BS; i < n; i += BS) a += p[i];
+        return a;
+    }
+};
+
 // rows per XCD, rounded up to whole groups of `rowsPerGroup`
 inline int rows_per_xcd(int nrow, int rowsPerGroup) {
     int r = (nrow + kXcd - 1) / kXcd;
@@ -134,17 +154,19 @@ __device__ __forceinline__ void bsr_row(int beg, int end, const int* __restrict_
 // pattern's arrays per position), so the lanes of a row fill up across both patterns and
 // no second dependent row-bound load follows the elastic pass.  The diagonal block that
 // fills `own` is the elastic one (contact rows also hold diagonal blocks).
+// RowPass holds one lane pass (UNR positions): load() issues its column, block and vector
+// loads, use() adds its products.  The loads do not depend on beta, so the kernel issues a
+// row's first pass before it reduces the previous kernel's partials.
 template <class M, class V, int LANES, bool WITHP, int UNR>
-__device__ __forceinline__ void bsr_row_ek(int lane, int eb, int ee, int cb, int ce, const int* __restrict__ ecol,
-                                           const M* __restrict__ ev, long enz, const int* __restrict__ ccol, const M* __restrict__ cv,
-                                           long cnz, int row, const V* __restrict__ z, const V* __restrict__ p, V beta, V* s, V* own,
-                                           bool& hasOwn) {
+struct RowPass {
     static_assert(UNR == 1 || UNR == 2, "");
-    const int nE = ee - eb, nT = nE + (ce - cb);
-    for (int j = lane; j < nT; j += UNR * LANES) {
-        int c[UNR];
-        bool on[UNR], el[UNR];
-        V a[UNR][9], x[UNR][3];
+    int c[UNR];
+    bool on[UNR], el[UNR];
+    M a[UNR][9];
+    V x[UNR][3], pv[UNR][3];
+    __device__ __forceinline__ void load(int j, int nT, int nE, int eb, int cb, const int* __restrict__ ecol, const M* __restrict__ ev,
+                                         long enz, const int* __restrict__ ccol, const M* __restrict__ cv, long cnz,
+                                         const V* __restrict__ z, const V* __restrict__ p) {
 #pragma unroll
         for (int u = 0; u < UNR; ++u) {
             const int ju = u == 0 || j + u * LANES < nT ? j + u * LANES : j;
@@ -156,33 +178,34 @@ __device__ __forceinline__ void bsr_row_ek(int lane, int eb, int ee, int cb, int
             const long nz = el[u] ? enz : cnz;
             c[u] = cp[b];
 #pragma unroll
-            for (int k = 0; k < 9; ++k) a[u][k] = (V)vp[k * nz + b];
+            for (int k = 0; k < 9; ++k) a[u][k] = vp[k * nz + b];
         }
 #pragma unroll
         for (int u = 0; u < UNR; ++u) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) x[u][k] = z[3 * c[u] + k];
-            if (WITHP) {
-                V pv[3];
+            if (WITHP)
 #pragma unroll
-                for (int k = 0; k < 3; ++k) pv[k] = p[3 * c[u] + k];
-#pragma unroll
-                for (int k = 0; k < 3; ++k) x[u][k] += beta * pv[k];
-            }
+                for (int k = 0; k < 3; ++k) pv[u][k] = p[3 * c[u] + k];
         }
+    }
+    __device__ __forceinline__ void use(int row, V beta, V* s, V* own, bool& hasOwn) {
 #pragma unroll
         for (int u = 0; u < UNR; ++u) {
+            if (WITHP)
+#pragma unroll
+                for (int k = 0; k < 3; ++k) x[u][k] += beta * pv[u][k];
             if (on[u] && el[u] && c[u] == row) {
                 own[0] = x[u][0]; own[1] = x[u][1]; own[2] = x[u][2];
                 hasOwn = true;
             }
             if (!on[u]) x[u][0] = x[u][1] = x[u][2] = 0;
-            s[0] += a[u][0] * x[u][0] + a[u][1] * x[u][1] + a[u][2] * x[u][2];
-            s[1] += a[u][3] * x[u][0] + a[u][4] * x[u][1] + a[u][5] * x[u][2];
-            s[2] += a[u][6] * x[u][0] + a[u][7] * x[u][1] + a[u][8] * x[u][2];
+            s[0] += (V)a[u][0] * x[u][0] + (V)a[u][1] * x[u][1] + (V)a[u][2] * x[u][2];
+            s[1] += (V)a[u][3] * x[u][0] + (V)a[u][4] * x[u][1] + (V)a[u][5] * x[u][2];
+            s[2] += (V)a[u][6] * x[u][0] + (V)a[u][7] * x[u][1] + (V)a[u][8] * x[u][2];
         }
     }
-}
+};
 
 // Iteration `it`: convergence of the residual left by the previous update is decided
 // first; then p_new = z + beta p_old (p_new = z at it = 0, WITHP = false), q = A p_new,
@@ -207,19 +230,24 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv(const int* __restrict__ itDev, 
     bool live = g * RPG < rowsPerXcd && row < nrow;
     int beg = live ? erp[row] : 0, end = live ? erp[row + 1] : 0;
     int cbeg = live && cnz > 0 ? crp[row] : 0, cend = live && cnz > 0 ? crp[row + 1] : 0;
-    if (flags[F_DONE]) return;
-    const int it = itDev ? *itDev + itArg : itArg;   // a captured chunk reads its base iteration
-
-    double arz = 0, arr = 0;
-#pragma unroll 4
-    for (int i = threadIdx.x; i < nRZ; i += BS) arz += partRZ[i];
-#pragma unroll 4
-    for (int i = threadIdx.x; i < nRR; i += BS) arr += partRR[i];
-    const double rz = block_allsum<BS>(arz, lds);
-    const double rr = block_allsum<BS>(arr, lds);
-    const double bb = it == 0 ? rr : sc[S_BB];
+    // everything the prologue needs is loaded before the first branch waits on any of it:
+    // the flag, the iteration, the scalars, the partials and the first row's first pass
+    const int done = flags[F_DONE];
+    const int itBase = itDev ? *itDev : 0;   // a captured chunk reads its base iteration
+    const double scBB = sc[S_BB], scTol = sc[S_TOL2], scRZ[2] = {sc[S_RZ0], sc[S_RZ1]};
+    PartialHead<BS> hz, hr;
+    hz.load(partRZ, nRZ);
+    hr.load(partRR, nRR);
+    RowPass<M, V, LANES, WITHP, UNR> pass;
+    int nE = end - beg, nT = nE + (cend - cbeg);
+    if (lane < nT) pass.load(lane, nT, nE, beg, cbeg, ecol, ev, enz, ccol, cv, cnz, z, pold);
+    if (done) return;
+    const int it = itBase + itArg;
+    const double rz = block_allsum<BS>(hz.finish(partRZ, nRZ), lds);
+    const double rr = block_allsum<BS>(hr.finish(partRR, nRR), lds);
+    const double bb = it == 0 ? rr : scBB;
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    if (rr <= sc[S_TOL2] * bb || it >= maxIt) {
+    if (rr <= scTol * bb || it >= maxIt) {
         if (lead) {
             if (it == 0) sc[S_BB] = rr;
             sc[S_RR] = rr;
@@ -228,7 +256,7 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv(const int* __restrict__ itDev, 
         }
         return;
     }
-    const V beta = WITHP ? (V)(rz / sc[S_RZ0 + ((it - 1) & 1)]) : (V)0;
+    const V beta = WITHP ? (V)(rz / ((it - 1) & 1 ? scRZ[1] : scRZ[0])) : (V)0;
 
     double pq = 0;
     for (; g * RPG < rowsPerXcd; g += nj) {
@@ -239,9 +267,10 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv(const int* __restrict__ itDev, 
         const int cbegN = liveN && cnz > 0 ? crp[rowN] : 0, cendN = liveN && cnz > 0 ? crp[rowN + 1] : 0;
         V s[3] = {0, 0, 0}, own[3] = {0, 0, 0};
         bool hasOwn = false;
-        if (row < nrow)
-            bsr_row_ek<M, V, LANES, WITHP, UNR>(lane, beg, end, cbeg, cend, ecol, ev, enz, ccol, cv, cnz, row, z, pold, beta, s, own,
-                                                hasOwn);
+        for (int j = lane; j < nT; j += UNR * LANES) {
+            if (j != lane || g != jb) pass.load(j, nT, nE, beg, cbeg, ecol, ev, enz, ccol, cv, cnz, z, pold);
+            pass.use(row, beta, s, own, hasOwn);
+        }
 #pragma unroll
         for (int o = LANES / 2; o > 0; o >>= 1)
 #pragma unroll
@@ -259,6 +288,8 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv(const int* __restrict__ itDev, 
         end = endN;
         cbeg = cbegN;
         cend = cendN;
+        nE = end - beg;
+        nT = nE + (cend - cbeg);
     }
     const double bpq = block_allsum<BS>(pq, lds);
     if (threadIdx.x == 0) partS[blockIdx.x] = bpq;
@@ -290,11 +321,12 @@ __global__ __launch_bounds__(BS) void k_pcg_update(const int* __restrict__ itDev
                                                    V* __restrict__ r, V* __restrict__ z, const V* __restrict__ p, const V* __restrict__ q,
                                                    const V* __restrict__ dinv, const double* __restrict__ partS, int nS,
                                                    double* __restrict__ partU, double* __restrict__ sc, int* __restrict__ flags) {
-    if (flags[F_DONE]) return;
-    const int it = itDev ? *itDev + itArg : itArg;
     __shared__ double lds[BS / 64];
-    double a = 0;
-    for (int i = threadIdx.x; i < nS; i += BS) a += partS[i];
+    const int done = flags[F_DONE];
+    const int itBase = itDev ? *itDev : 0;
+    const double scRZ[2] = {sc[S_RZ0], sc[S_RZ1]};
+    PartialHead<BS> hs;
+    hs.load(partS, nS);
     const int row = (int)(blockIdx.x % kXcd) * rowsPerXcd + (int)(blockIdx.x / kXcd) * BS + (int)threadIdx.x;
     const bool valid = row < nrow;
     V pv[3] = {0, 0, 0}, qv[3] = {0, 0, 0}, xv[3] = {0, 0, 0}, rv[3] = {0, 0, 0}, D[9];
@@ -308,7 +340,9 @@ __global__ __launch_bounds__(BS) void k_pcg_update(const int* __restrict__ itDev
 #pragma unroll
             for (int k = 0; k < 9; ++k) D[k] = dinv[9l * row + k];
     }
-    const double pq = block_allsum<BS>(a, lds);
+    if (done) return;
+    const int it = itBase + itArg;
+    const double pq = block_allsum<BS>(hs.finish(partS, nS), lds);
     if (!(pq > 0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             flags[F_FAIL] = 1;
@@ -317,7 +351,7 @@ __global__ __launch_bounds__(BS) void k_pcg_update(const int* __restrict__ itDev
         }
         return;
     }
-    const V alpha = (V)(sc[S_RZ0 + (it & 1)] / pq);
+    const V alpha = (V)((it & 1 ? scRZ[1] : scRZ[0]) / pq);
     double rz = 0, rr = 0;
     if (valid) {
 #pragma unroll
@@ -357,8 +391,6 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
                                                          const V* __restrict__ rOld, V* __restrict__ rNew, V* __restrict__ y,
                                                          const double* __restrict__ partS, int nS, double* __restrict__ partRR,
                                                          double* __restrict__ sc, int* __restrict__ flags) {
-    if (flags[F_DONE]) return;
-    const int it = itDev ? *itDev + itArg : itArg;
     __shared__ double lds[BS / 64];
     constexpr int RPG = BS / LANES;
     const int xb = blockIdx.x % kXcd, jb = blockIdx.x / kXcd, nj = gridDim.x / kXcd;
@@ -368,9 +400,26 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
     int row = rowBase + g * RPG;
     bool live = g * RPG < rowsPerXcd && row < nrow;
     int beg = live ? rp[row] : 0, end = live ? rp[row + 1] : 0;
-    double a = 0;
-    for (int i = threadIdx.x; i < nS; i += BS) a += partS[i];
-    const double pq = block_allsum<BS>(a, lds);
+    const int done = flags[F_DONE];
+    const int itBase = itDev ? *itDev : 0;
+    const double scRZ[2] = {sc[S_RZ0], sc[S_RZ1]};
+    PartialHead<BS> hs;
+    hs.load(partS, nS);
+    // the first block of the lane's first row, which does not depend on alpha
+    int c0 = 0;
+    V r0[3] = {0, 0, 0}, q0[3] = {0, 0, 0}, f0[9];
+    if (beg + lane < end) {
+        c0 = col[beg + lane];
+        lp_unpack9<V>(val, nnz, beg + lane, f0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            r0[k] = rOld[3 * c0 + k];
+            q0[k] = q[3 * c0 + k];
+        }
+    }
+    if (done) return;
+    const int it = itBase + itArg;
+    const double pq = block_allsum<BS>(hs.finish(partS, nS), lds);
     if (!(pq > 0)) {
         if (blockIdx.x == 0 && threadIdx.x == 0) {
             flags[F_FAIL] = 1;
@@ -379,7 +428,7 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
         }
         return;
     }
-    const V alpha = (V)(sc[S_RZ0 + (it & 1)] / pq);
+    const V alpha = (V)((it & 1 ? scRZ[1] : scRZ[0]) / pq);
     double rr = 0;
     for (; g * RPG < rowsPerXcd; g += nj) {
         const int gn = g + nj, rowN = rowBase + gn * RPG;
@@ -387,16 +436,22 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
         const int begN = liveN ? rp[rowN] : 0, endN = liveN ? rp[rowN + 1] : 0;
         V acc[3] = {0, 0, 0};
         for (int b = beg + lane; b < end; b += LANES) {
-            const int c = col[b];
+            if (b != beg + lane || g != jb) {
+                c0 = col[b];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    r0[k] = rOld[3 * c0 + k];
+                    q0[k] = q[3 * c0 + k];
+                }
+                lp_unpack9<V>(val, nnz, b, f0);
+            }
             V rv[3];
 #pragma unroll
-            for (int k = 0; k < 3; ++k) rv[k] = rOld[3 * c + k] - alpha * q[3 * c + k];
-            V f[9];
-            lp_unpack9<V>(val, nnz, b, f);
-            acc[0] += f[0] * rv[0] + f[1] * rv[1] + f[2] * rv[2];
-            acc[1] += f[3] * rv[0] + f[4] * rv[1] + f[5] * rv[2];
-            acc[2] += f[6] * rv[0] + f[7] * rv[1] + f[8] * rv[2];
-            if (c == row) {
+            for (int k = 0; k < 3; ++k) rv[k] = r0[k] - alpha * q0[k];
+            acc[0] += f0[0] * rv[0] + f0[1] * rv[1] + f0[2] * rv[2];
+            acc[1] += f0[3] * rv[0] + f0[4] * rv[1] + f0[5] * rv[2];
+            acc[2] += f0[6] * rv[0] + f0[7] * rv[1] + f0[8] * rv[2];
+            if (c0 == row) {
 #pragma unroll
                 for (int k = 0; k < 3; ++k) {
                     rNew[3 * row + k] = rv[k];
@@ -653,6 +708,10 @@ static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V*
             nS = T.spmvCand[cand][0]; sLanes = T.spmvCand[cand][1]; sUnroll = T.spmvCand[cand][2];
         }
         const int rpxS = rows_per_xcd(nV, kSpmvBlock / sLanes);
+        // no more workgroups than row groups: the rest would only sum the partials and add
+        // zeros to the next kernel's (a 4,247-vertex scene has 272 groups of 16 rows for the
+        // default 1024 workgroups)
+        nS = std::min(nS, kXcd * (rpxS / (kSpmvBlock / sLanes)));
         // a whole chunk after the first, with no launch timed, replays one captured graph of
         // its 16 iterations (launch arguments identical from chunk to chunk: the iteration
         // number comes from the device counter, the buffer parities repeat every 16)
