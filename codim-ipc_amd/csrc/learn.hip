@@ -595,9 +595,7 @@ __global__ __launch_bounds__(BS) void k_lp_spmv_bf16(int nrow, int rowsPerXcd, c
             acc[2] += a[6] * x0 + a[7] * x1 + a[8] * x2;
         }
 #pragma unroll
-        for (int o = LANES / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) acc[k] += __shfl_xor(acc[k], o, LANES);
+        for (int k = 0; k < 3; ++k) acc[k] = lane_sum<LANES>(acc[k]);
         if (row < nrow && lane == 0) {
             // two-level correction: y_i += T_i zc = t_a + w_a x d_i (rows of the coarse space)
             const int ca = cgZ ? cgAgg[row] : -1;
@@ -663,9 +661,7 @@ __global__ void k_lp_apply_upper(int nV, const int* __restrict__ rp, const int* 
             }
         }
 #pragma unroll
-        for (int o = LANES / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) acc[k] += __shfl_xor(acc[k], o, LANES);
+        for (int k = 0; k < 3; ++k) acc[k] = lane_sum<LANES>(acc[k]);
         if (row < nV && lane == 0) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {

@@ -15,15 +15,19 @@
 // The refinement (x += d, r = b - H x with the FP64 blocks) repeats the inner solve on
 // the FP64 residual until ||r|| <= tol ||b|| holds in FP64.
 //
-// One CG iteration is two kernels and no atomics:
-//   k_pcg_spmv   beta from the previous update's partial sums, p = z + beta p_old formed
-//                on the fly, q = A p, p written, partial sums of p.q per workgroup;
-//   k_pcg_update x += alpha p, r -= alpha q, z = Dinv r, partial sums of r.z and r.r.
+// One CG iteration has no atomics.  Block Jacobi, two kernels:
+//   k_pcg_spmv_p    q = A p, partial sums of p.q and q.Dinv q per workgroup;
+//   k_pcg_update_p  alpha and beta from those sums, x += alpha p, r -= alpha q, z = Dinv r,
+//                   p = z + beta p, partial sums of r.r and r.z.
+// The learned preconditioner: the SpMV, then the kernels of the factor products,
+//   k_pcg_spmv      beta from the previous partial sums, p = z + beta p_old formed on the
+//                   fly, q = A p, p written, partial sums of p.q per workgroup;
+//   k_pcg_update_lower and k_lp_spmv_bf16 (learn.hip).
 // Each kernel starts by summing the previous kernel's per-workgroup partials itself
 // (every workgroup in the same fixed order, so all hold the identical scalar); kernel
 // boundaries on the one stream order those writes before the reads, so no fence or
-// ticket counter is needed.  The SpMV runs a fixed grid (Ctx::spmvGrid workgroups) so the
-// update kernel has few partials to sum.
+// ticket counter is needed.  The SpMV runs a fixed grid (Ctx::spmvGrid workgroups at
+// most) so the next kernel has few partials to sum.
 //
 // Matrix blocks are stored structure-of-arrays (entry k of all blocks contiguous);
 // LANES lanes share a block row and stride over its blocks, so the lanes of a wave read
@@ -48,7 +52,10 @@ enum { S_RZ0 = 0, S_RZ1, S_BB, S_RR, S_TOL2 };   // S_TOL2: the squared relative
 enum { F_DONE = 0, F_ITERS, F_FAIL };
 
 constexpr int kSpmvBlock = 256;
-constexpr int kUpdBlock = 256;
+constexpr int kInitBlock = 256;
+// block-Jacobi update: vertices per group (the small one up to kSmallRows vertices) and
+// workgroups at most (a multiple of kXcd)
+constexpr int kUpdRowsSmall = 64, kUpdRows = 128, kSmallRows = 16384, kUpdGrid = 512;
 constexpr int kXcd = 8;
 // with profiling on, every kProfEvery-th SpMV launch is bracketed by timing events (events
 // on every launch slow the solve by about 10%), starting at launch kProfFirst of each
@@ -78,7 +85,11 @@ struct PartialHead {
     double v[4];
     __device__ __forceinline__ void load(const double* __restrict__ p, int n) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) v[k] = (int)threadIdx.x + k * BS < n ? p[threadIdx.x + k * BS] : 0.0;
+        for (int k = 0; k < 4; ++k) {
+            const int i = (int)threadIdx.x + k * BS;
+            const double w = p[i < n ? i : 0];   // always a load: no branch between the batch's issues
+            v[k] = i < n ? w : 0.0;
+        }
     }
     __device__ __forceinline__ double finish(const double* __restrict__ p, int n) const {
         double a = 0;
@@ -155,8 +166,9 @@ __device__ __forceinline__ void bsr_row(int beg, int end, const int* __restrict_
 // no second dependent row-bound load follows the elastic pass.  The diagonal block that
 // fills `own` is the elastic one (contact rows also hold diagonal blocks).
 // RowPass holds one lane pass (UNR positions): load() issues its column, block and vector
-// loads, use() adds its products.  The loads do not depend on beta, so the kernel issues a
-// row's first pass before it reduces the previous kernel's partials.
+// loads, use() adds its products.  The loads do not depend on alpha and beta, so the kernel
+// issues a row's first pass before it reduces the previous kernel's partials.
+// WITHP: the product's vector is z + beta p, else z alone.
 template <class M, class V, int LANES, bool WITHP, int UNR>
 struct RowPass {
     static_assert(UNR == 1 || UNR == 2, "");
@@ -195,7 +207,7 @@ struct RowPass {
             if (WITHP)
 #pragma unroll
                 for (int k = 0; k < 3; ++k) x[u][k] += beta * pv[u][k];
-            if (on[u] && el[u] && c[u] == row) {
+            if (own && on[u] && el[u] && c[u] == row) {
                 own[0] = x[u][0]; own[1] = x[u][1]; own[2] = x[u][2];
                 hasOwn = true;
             }
@@ -272,9 +284,7 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv(const int* __restrict__ itDev, 
             pass.use(row, beta, s, own, hasOwn);
         }
 #pragma unroll
-        for (int o = LANES / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) s[k] += __shfl_xor(s[k], o, LANES);
+        for (int k = 0; k < 3; ++k) s[k] = lane_sum<LANES>(s[k]);
         if (row < nrow && hasOwn) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
@@ -314,68 +324,218 @@ static auto spmv_kernel(int lanes, int unr, bool withP) -> decltype(&k_pcg_spmv<
     return nullptr;
 }
 
-// Iteration `it`: alpha = r.z / p.q, x += alpha p, r -= alpha q, z = Dinv r, partials
-// of r.z and r.r (written as partU[block], partU[nU + block]).
-template <class V, int BS, bool JAC>
-__global__ __launch_bounds__(BS) void k_pcg_update(const int* __restrict__ itDev, int itArg, int nrow, int rowsPerXcd, V* __restrict__ x,
-                                                   V* __restrict__ r, V* __restrict__ z, const V* __restrict__ p, const V* __restrict__ q,
-                                                   const V* __restrict__ dinv, const double* __restrict__ partS, int nS,
-                                                   double* __restrict__ partU, double* __restrict__ sc, int* __restrict__ flags) {
-    __shared__ double lds[BS / 64];
+// Block Jacobi.  The direction p is formed once per vertex by the update kernel, so that
+// the SpMV gathers one vector per block instead of z and p and has no scalar to wait for.
+// For that the update needs beta before r'.z' of the new residual is summed; with
+// z' = z - alpha u, u = Dinv q, and q.z = q.p (p is conjugate to the previous direction) it is
+//   r'.z' = r.z - 2 alpha q.z + alpha^2 q.u = alpha^2 q.u - r.z
+// (Meurant's form), q.u from the SpMV's row owners; r.z itself is summed anew from the
+// vectors every iteration, so the recurrence never spans more than one.
+// Bound: the block stream on large systems, the chain row bounds -> columns -> vectors ->
+// partials on small ones.  Measured (us per iteration, against forming p = z + beta p_old
+// in the gathers and one vertex per update thread): 4,247 vertices FP64 11.3 -> 7.9, 6,166
+// vertices FP32 11.0 -> 8.2, 33,169 vertices with 183,968 constraints FP64 27.1 -> 23.8 and
+// FP32 blocks 22.1 -> 18.8, 164,170 vertices with 1.25 million constraints 126.6 -> 114.3
+// and 66.4 -> 54.9.  (A single kernel per iteration, with the neighbours' p formed from z,
+// u and p_old in the gathers, was faster below 5,000 vertices only: three gathered vectors
+// per block cost more than the second launch.)
+// Partials: partS = [2][workgroups] of p.q, q.u; partU = [2][workgroups] of r.z, r.r,
+// double-buffered (an update reads the previous one's while it writes its own).
+template <class M, class V, int LANES, int BS, int UNR>
+__global__ __launch_bounds__(BS) void k_pcg_spmv_p(const int* __restrict__ erp, const int* __restrict__ ecol, const M* __restrict__ ev,
+                                                   int enz, const int* __restrict__ crp, const int* __restrict__ ccol,
+                                                   const M* __restrict__ cv, int cnz, int nrow, int rowsPerXcd,
+                                                   const V* __restrict__ p, const V* __restrict__ dinv, V* __restrict__ q,
+                                                   double* __restrict__ partS, const int* __restrict__ flags) {
+    static_assert(LANES >= 4, "");
+    constexpr int RPG = BS / LANES, NW = BS / 64;
+    __shared__ double lds[2][NW];
+    const int xb = blockIdx.x % kXcd, jb = blockIdx.x / kXcd, nj = gridDim.x / kXcd;
+    const int lane = threadIdx.x % LANES;
+    const int rowBase = xb * rowsPerXcd + (int)threadIdx.x / LANES;
+    int g = jb;
+    int row = rowBase + g * RPG;
+    const bool live = g * RPG < rowsPerXcd && row < nrow;
+    const int done = flags[F_DONE];
+    int beg = live ? erp[row] : 0, end = live ? erp[row + 1] : 0;
+    int cbeg = live && cnz > 0 ? crp[row] : 0, cend = live && cnz > 0 ? crp[row + 1] : 0;
+    if (done) return;
+    double sum[2] = {0, 0};
+    for (; g * RPG < rowsPerXcd; g += nj) {
+        const int gn = g + nj;
+        const int rowN = rowBase + gn * RPG;
+        const bool liveN = gn * RPG < rowsPerXcd && rowN < nrow;
+        const int begN = liveN ? erp[rowN] : 0, endN = liveN ? erp[rowN + 1] : 0;
+        const int cbegN = liveN && cnz > 0 ? crp[rowN] : 0, cendN = liveN && cnz > 0 ? crp[rowN + 1] : 0;
+        // lanes 0..2 own one component of the row each; their loads are in flight during
+        // the row's products
+        const bool owner = row < nrow && lane < 3;
+        V pk = 0, D[3] = {0, 0, 0};
+        if (owner) {
+            pk = p[3 * row + lane];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) D[m] = dinv[9l * row + 3 * lane + m];
+        }
+        V s[3] = {0, 0, 0};
+        bool unused = false;
+        const int nE = end - beg, nT = nE + (cend - cbeg);
+        for (int j = lane; j < nT; j += UNR * LANES) {
+            RowPass<M, V, LANES, false, UNR> pass;
+            pass.load(j, nT, nE, beg, cbeg, ecol, ev, enz, ccol, cv, cnz, p, nullptr);
+            pass.use(row, (V)0, s, (V*)nullptr, unused);
+        }
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s[k] = lane_sum<LANES>(s[k]);
+        if (owner) {
+            const V sk = lane == 0 ? s[0] : lane == 1 ? s[1] : s[2];
+            const V uk = D[0] * s[0] + D[1] * s[1] + D[2] * s[2];
+            q[3 * row + lane] = sk;
+            sum[0] += (double)pk * (double)sk;
+            sum[1] += (double)sk * (double)uk;
+        }
+        row = rowN;
+        beg = begN;
+        end = endN;
+        cbeg = cbegN;
+        cend = cendN;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        sum[k] = wave_sum(sum[k]);
+        if ((threadIdx.x & 63) == 0) lds[k][threadIdx.x >> 6] = sum[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double t = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) t += lds[threadIdx.x][w];
+        partS[(long)threadIdx.x * gridDim.x + blockIdx.x] = t;
+    }
+}
+template <class M, class V>
+static auto spmv_p_kernel(int lanes, int unr) -> decltype(&k_pcg_spmv_p<M, V, 16, kSpmvBlock, 1>) {
+#define CIPC_SPMV_P_PICK(L, U) \
+    if (lanes == L && unr == U) return k_pcg_spmv_p<M, V, L, kSpmvBlock, U>;
+    CIPC_SPMV_P_PICK(8, 1)
+    CIPC_SPMV_P_PICK(8, 2)
+    CIPC_SPMV_P_PICK(4, 1)
+    CIPC_SPMV_P_PICK(4, 2)
+    CIPC_SPMV_P_PICK(16, 2)
+    CIPC_SPMV_P_PICK(16, 1)
+#undef CIPC_SPMV_P_PICK
+    return nullptr;
+}
+
+// Iteration `it` after its SpMV: convergence of r_it is decided first (its r.r was summed by
+// the previous update), then x, r, z and the next direction.  One thread per component:
+// consecutive lanes read consecutive addresses, where one thread per vertex took 33
+// accesses of stride 24 bytes each; r' crosses to the vertex's other components through
+// LDS.  Workgroups of VB = 128 vertices spread small systems over the CUs; large ones walk
+// several such groups (at most kUpdGrid workgroups, so that the partials every workgroup
+// adds up stay few).  Measured (us per iteration with groups of 64 / 128 / 256 vertices): 8.5 /
+// 9.1 / 10.7 on 4,247 vertices, 25.3 / 24.1 / 24.7 on 33,169 (FP64 blocks).
+template <class V, int VB>
+__global__ __launch_bounds__(3 * VB) void k_pcg_update_p(const int* __restrict__ itDev, int itArg, int maxIt, int nrow, int rowsPerXcd,
+                                                         V* __restrict__ x, V* __restrict__ r, V* __restrict__ z, V* __restrict__ p,
+                                                         const V* __restrict__ q, const V* __restrict__ dinv,
+                                                         const double* __restrict__ partS, int nS, const double* __restrict__ partU, int nIn,
+                                                         double* __restrict__ partUN, double* __restrict__ sc, int* __restrict__ flags) {
+    constexpr int BS = 3 * VB, NW = BS / 64;
+    __shared__ double lds[4][NW], ldsN[2][NW];
+    __shared__ V rbuf[BS];
     const int done = flags[F_DONE];
     const int itBase = itDev ? *itDev : 0;
-    const double scRZ[2] = {sc[S_RZ0], sc[S_RZ1]};
-    PartialHead<BS> hs;
-    hs.load(partS, nS);
-    const int row = (int)(blockIdx.x % kXcd) * rowsPerXcd + (int)(blockIdx.x / kXcd) * BS + (int)threadIdx.x;
-    const bool valid = row < nrow;
-    V pv[3] = {0, 0, 0}, qv[3] = {0, 0, 0}, xv[3] = {0, 0, 0}, rv[3] = {0, 0, 0}, D[9];
-    if (valid) {
+    const double scBB = sc[S_BB], scTol = sc[S_TOL2];
+    const int nU = gridDim.x;
+    PartialHead<BS> head[4];   // p.q, q.u, r.z, r.r
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            pv[k] = p[3 * row + k]; qv[k] = q[3 * row + k];
-            xv[k] = x[3 * row + k]; rv[k] = r[3 * row + k];
-        }
-        if (JAC)
-#pragma unroll
-            for (int k = 0; k < 9; ++k) D[k] = dinv[9l * row + k];
+    for (int k = 0; k < 2; ++k) {
+        head[k].load(partS + (long)k * nS, nS);
+        head[2 + k].load(partU + (long)k * nIn, nIn);
     }
+    const int t = threadIdx.x, vtx = t / 3, comp = t - 3 * vtx;
+    const int xb = blockIdx.x % kXcd, nj = gridDim.x / kXcd;
+    int g = blockIdx.x / kXcd;
+    V pv = 0, qv = 0, xv = 0, rv = 0, D[3] = {0, 0, 0};
+    long o = 0;
+    bool valid = false;
+    auto load = [&]() {
+        const int row0 = xb * rowsPerXcd + g * VB;
+        o = 3l * row0 + t;
+        valid = g * VB < rowsPerXcd && row0 + vtx < nrow;
+        pv = qv = xv = rv = D[0] = D[1] = D[2] = 0;   // rows beyond nrow hold zeros and add nothing
+        if (valid) {
+            pv = p[o]; qv = q[o]; xv = x[o]; rv = r[o];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) D[m] = dinv[3 * o + m];
+        }
+    };
+    load();
     if (done) return;
     const int it = itBase + itArg;
-    const double pq = block_allsum<BS>(hs.finish(partS, nS), lds);
-    if (!(pq > 0)) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            flags[F_FAIL] = 1;
+    double tot[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        tot[k] = wave_sum(k < 2 ? head[k].finish(partS + (long)k * nS, nS) : head[k].finish(partU + (long)(k - 2) * nIn, nIn));
+        if ((t & 63) == 0) lds[k][t >> 6] = tot[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        tot[k] = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) tot[k] += lds[k][w];
+    }
+    const double pq = tot[0], rz = tot[2], rr = tot[3];
+    const double bb = it == 0 ? rr : scBB;
+    const bool lead = blockIdx.x == 0 && t == 0;
+    const bool stop = rr <= scTol * bb || it >= maxIt;
+    if (stop || !(pq > 0)) {
+        if (lead) {
+            if (it == 0) sc[S_BB] = rr;
+            sc[S_RR] = rr;
             flags[F_ITERS] = it;
+            if (!stop) flags[F_FAIL] = 1;
             flags[F_DONE] = 1;
         }
         return;
     }
-    const V alpha = (V)((it & 1 ? scRZ[1] : scRZ[0]) / pq);
-    double rz = 0, rr = 0;
-    if (valid) {
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            x[3 * row + k] = xv[k] + alpha * pv[k];
-            rv[k] = rv[k] - alpha * qv[k];
-            r[3 * row + k] = rv[k];
+    const double al = rz / pq, rzN = al * (al * tot[1]) - rz;
+    const V alpha = (V)al, beta = (V)(rzN > 0 ? rzN / rz : 0.0);
+    double srz = 0, srr = 0;
+    const int v0 = t - comp;
+    for (;;) {
+        rv = rv - alpha * qv;
+        rbuf[t] = rv;
+        __syncthreads();
+        const V zk = D[0] * rbuf[v0] + D[1] * rbuf[v0 + 1] + D[2] * rbuf[v0 + 2];
+        if (valid) {
+            x[o] = xv + alpha * pv;
+            r[o] = rv;
+            z[o] = zk;
+            p[o] = zk + beta * pv;
         }
+        srz += (double)rv * (double)zk;
+        srr += (double)rv * (double)rv;
+        g += nj;
+        if (g * VB >= rowsPerXcd) break;
+        load();
+        __syncthreads();   // rbuf is read by all before the next group overwrites it
+    }
+    srz = wave_sum(srz);
+    srr = wave_sum(srr);
+    if ((t & 63) == 0) {
+        ldsN[0][t >> 6] = srz;
+        ldsN[1][t >> 6] = srr;
+    }
+    __syncthreads();
+    if (t < 2) {
+        double a = 0;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            if (JAC) {
-                const V zk = D[3 * k] * rv[0] + D[3 * k + 1] * rv[1] + D[3 * k + 2] * rv[2];
-                z[3 * row + k] = zk;
-                rz += (double)rv[k] * (double)zk;
-            }
-            rr += (double)rv[k] * (double)rv[k];
-        }
+        for (int w = 0; w < NW; ++w) a += ldsN[t][w];
+        partUN[(long)t * nU + blockIdx.x] = a;
     }
-    const double brz = block_allsum<BS>(rz, lds);
-    const double brr = block_allsum<BS>(rr, lds);
-    if (threadIdx.x == 0) {
-        partU[blockIdx.x] = brz;
-        partU[gridDim.x + blockIdx.x] = brr;
-    }
+    if (it == 0 && lead) sc[S_BB] = rr;
 }
 
 // Learned form, iteration `it`, fused with the first factor product: alpha = r.z / p.q,
@@ -461,9 +621,7 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
             }
         }
 #pragma unroll
-        for (int o = LANES / 2; o > 0; o >>= 1)
-#pragma unroll
-            for (int k = 0; k < 3; ++k) acc[k] += __shfl_xor(acc[k], o, LANES);
+        for (int k = 0; k < 3; ++k) acc[k] = lane_sum<LANES>(acc[k]);
         if (row < nrow && lane == 0) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) y[3 * row + k] = acc[k];
@@ -476,12 +634,12 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
     if (threadIdx.x == 0) partRR[blockIdx.x] = brr;
 }
 
-// r = b, x = 0, z = Dinv r; partials of r.z and r.r in the update kernel's layout;
-// the solver flags are cleared.
+// r = b, x = 0, z = Dinv r and, when p is given, p = z; partials of r.z and r.r in the
+// update kernel's layout; the solver flags are cleared.
 template <class V, int BS>
 __global__ __launch_bounds__(BS) void k_pcg_init(int nrow, int rowsPerXcd, const V* __restrict__ b, V* __restrict__ x, V* __restrict__ r,
-                                                 V* __restrict__ z, const V* __restrict__ dinv, double* __restrict__ partU,
-                                                 int* __restrict__ flags) {
+                                                 V* __restrict__ z, V* __restrict__ p, const V* __restrict__ dinv,
+                                                 double* __restrict__ partU, int* __restrict__ flags) {
     __shared__ double lds[BS / 64];
     const int row = (int)(blockIdx.x % kXcd) * rowsPerXcd + (int)(blockIdx.x / kXcd) * BS + (int)threadIdx.x;
     double rz = 0, rr = 0;
@@ -498,6 +656,7 @@ __global__ __launch_bounds__(BS) void k_pcg_init(int nrow, int rowsPerXcd, const
         for (int k = 0; k < 3; ++k) {
             const V zk = dinv[9l * row + 3 * k] * rv[0] + dinv[9l * row + 3 * k + 1] * rv[1] + dinv[9l * row + 3 * k + 2] * rv[2];
             z[3 * row + k] = zk;
+            if (p) p[3 * row + k] = zk;
             rz += (double)rv[k] * (double)zk;
         }
     }
@@ -576,9 +735,7 @@ __global__ __launch_bounds__(kBlock) void k_residual(const int* __restrict__ erp
         if (cnz > 0) bsr_row<double, double, LANES, false>(crp[row] + lane, crp[row + 1], ccol, cv, cnz, -1, x, x, 0.0, s, own, hasOwn);
     }
 #pragma unroll
-    for (int o = LANES / 2; o > 0; o >>= 1)
-#pragma unroll
-        for (int k = 0; k < 3; ++k) s[k] += __shfl_xor(s[k], o, LANES);
+    for (int k = 0; k < 3; ++k) s[k] = lane_sum<LANES>(s[k]);
     double rr = 0;
     if (row < nrow && lane == 0) {
 #pragma unroll
@@ -604,8 +761,8 @@ __global__ void k_it_advance(int* itDev, int by) {
 // ---- one preconditioned CG solve in precision V; returns 0 converged, 1 not SPD
 // (p^T A p <= 0), 2 iteration limit
 template <class M, class V>
-static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V* r, V* z, V* pbuf, V* q, const V* dinv, double tol, int maxIter,
-                   int* iters, double* relres, bool learned = false) {
+static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V* r, V* z, V* pbuf, V* q, const V* dinv, double tol,
+                   int maxIter, int* iters, double* relres, bool learned = false) {
     const int nV = c.nV, n = 3 * nV;
     BSR& E = c.Ael;
     BSR& K = c.Acon;
@@ -618,21 +775,25 @@ static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V*
     int nSmax = c.spmvGrid;
     if (spmvTuning)
         for (const auto& k : T.spmvCand) nSmax = std::max(nSmax, k[0]);
-    const int rpxU = rows_per_xcd(nV, kUpdBlock), nU = kXcd * (rpxU / kUpdBlock);
+    const int rpxI = rows_per_xcd(nV, kInitBlock), nI = kXcd * (rpxI / kInitBlock);
+    const int updRows = nV <= kSmallRows ? kUpdRowsSmall : kUpdRows;
+    const int rpxU = rows_per_xcd(nV, updRows), nU = std::min(kUpdGrid, kXcd * (rpxU / updRows));
     const int nP = lp_apply_partials(c);
-    double* partS = c.dscr.ensure((size_t)nSmax + 2l * nU + 2l * nP);
-    double* partU = partS + nSmax;
-    double* partP = partU + 2l * nU;
+    double* partS = c.dscr.ensure(2l * nSmax + 4l * nU + 2l * nI + 2l * nP);
+    double* partU = partS + 2l * nSmax;
+    double* partI = partU + 4l * nU;          // the init kernel's r.z and r.r
+    double* partP = partI + 2l * nI;
     double* partF = partP + nP;               // r.r partials of the fused learned update
-    // r.z partials: the update kernel's (block Jacobi) or the preconditioner product's
-    const double* partRZ = learned ? partP : partU;
-    const int nRZ = learned ? nP : nU;
+    // learned form: r.z partials of the preconditioner product
+    const double* partRZ = partP;
+    const int nRZ = nP;
     // two-level correction of the learned preconditioner (coarse.hip)
     const bool coarse = learned && c.coarseOn && c.cg.ready;
     V* ltmp = nullptr;
     V* rb[2] = {r, r};                        // learned form: r ping-pongs between r and a second buffer
 
-    hipLaunchKernelGGL((k_pcg_init<V, kUpdBlock>), dim3(nU), dim3(kUpdBlock), 0, c.s, nV, rpxU, b, xsol, r, z, dinv, partU, flags);
+    hipLaunchKernelGGL((k_pcg_init<V, kInitBlock>), dim3(nI), dim3(kInitBlock), 0, c.s, nV, rpxI, b, xsol, r, z,
+                       learned ? (V*)nullptr : pbuf, dinv, partI, flags);
     CIPC_LAUNCH_CHECK();
     if (learned) {
         static_assert(sizeof(double) >= sizeof(V), "");
@@ -662,28 +823,37 @@ static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V*
     c.hScal[36] = tol2;
     CIPC_HIP(hipMemcpyAsync(sc + S_TOL2, c.hScal + 36, sizeof(double), hipMemcpyHostToDevice, c.s));
     const double mb = (double)sizeof(M), vb = (double)sizeof(V);
-    const double spmvBytes = (9 * mb + 4) * ((double)E.nnzb + K.nnzb) + 4.0 * (nV + 1) * (K.nnzb > 0 ? 2 : 1) + 4 * 3 * vb * nV;
+    // learned: z, p_old read, p, q written; block Jacobi: p, Dinv read, q written
+    const double spmvBytes = (9 * mb + 4) * ((double)E.nnzb + K.nnzb) + 4.0 * (nV + 1) * (K.nnzb > 0 ? 2 : 1) +
+                             (learned ? 4 * 3 : 2 * 3 + 9) * vb * nV;
     int* itDev = (int*)(c.counters.p + 24);   // base iteration of a captured chunk
     // one iteration's launches: iteration `it` (itDev == nullptr) or base + k (captured)
     auto launch_iteration = [&](int it, int k, const int* itd, int nS, int sLanes, int sUnroll, int rpxS, bool timed) {
         const V* pold = pbuf + (size_t)((it + 1) & 1) * n;
         V* pnew = pbuf + (size_t)(it & 1) * n;
         const int itArg = itd ? k : it;
-        auto kern = spmv_kernel<M, V>(sLanes, sUnroll, it > 0);
-        const double* partRR = learned && it > 0 ? partF : partU + nU;
-        const int nRR = learned && it > 0 ? nP : nU;
-        if (timed)
-            hipExtLaunchKernelGGL(kern, dim3(nS), dim3(kSpmvBlock), 0, c.s, c.evPool[2 * k], c.evPool[2 * k + 1], 0, itd, itArg, maxIter,
-                                  E.rowptr.p, E.col.p, valE, E.nnzb, K.rowptr.p, K.col.p, valK, K.nnzb, nV, rpxS, (const V*)z, pold, pnew,
-                                  q, partRZ, nRZ, partRR, nRR, partS, sc, flags);
-        else
-            hipLaunchKernelGGL(kern, dim3(nS), dim3(kSpmvBlock), 0, c.s, itd, itArg, maxIter, E.rowptr.p, E.col.p, valE, E.nnzb,
-                               K.rowptr.p, K.col.p, valK, K.nnzb, nV, rpxS, (const V*)z, pold, pnew, q, partRZ, nRZ, partRR, nRR, partS,
-                               sc, flags);
+        const bool sampled = timed;
+        auto go = [&](auto kern, auto... args) {
+            if (sampled)
+                hipExtLaunchKernelGGL(kern, dim3(nS), dim3(kSpmvBlock), 0, c.s, c.evPool[2 * k], c.evPool[2 * k + 1], 0, args...);
+            else
+                hipLaunchKernelGGL(kern, dim3(nS), dim3(kSpmvBlock), 0, c.s, args...);
+        };
         if (!learned) {
-            hipLaunchKernelGGL((k_pcg_update<V, kUpdBlock, true>), dim3(nU), dim3(kUpdBlock), 0, c.s, itd, itArg, nV, rpxU, xsol, r, z,
-                               (const V*)pnew, (const V*)q, dinv, (const double*)partS, nS, partU, sc, flags);
+            go(spmv_p_kernel<M, V>(sLanes, sUnroll), (const int*)E.rowptr.p, (const int*)E.col.p, valE, E.nnzb, (const int*)K.rowptr.p,
+               (const int*)K.col.p, valK, K.nnzb, nV, rpxS, (const V*)pbuf, dinv, q, partS, (const int*)flags);
+            // the first update reads the init kernel's partials, the others the previous update's
+            hipLaunchKernelGGL((updRows == kUpdRows ? k_pcg_update_p<V, kUpdRows> : k_pcg_update_p<V, kUpdRowsSmall>), dim3(nU),
+                               dim3(3 * updRows), 0, c.s, itd, itArg, maxIter, nV, rpxU, xsol, r,
+                               z, pbuf, (const V*)q, dinv, (const double*)partS, nS,
+                               (const double*)(it == 0 ? partI : partU + 2l * (it & 1) * nU), it == 0 ? nI : nU,
+                               partU + 2l * ((it + 1) & 1) * nU, sc, flags);
         } else {
+            const double* partRR = it > 0 ? partF : partI + nI;
+            const int nRR = it > 0 ? nP : nI;
+            go(spmv_kernel<M, V>(sLanes, sUnroll, it > 0), itd, itArg, maxIter, (const int*)E.rowptr.p, (const int*)E.col.p, valE, E.nnzb,
+               (const int*)K.rowptr.p, (const int*)K.col.p, valK, K.nnzb, nV, rpxS, (const V*)z, pold, pnew, q, partRZ, nRZ, partRR, nRR,
+               partS, sc, flags);
             LearnedPrecond& lp = *c.lp;
             V* rNew = rb[(it + 1) & 1];
             auto fused = c.lpLanes == 2    ? k_pcg_update_lower<2, kSpmvBlock, V>
@@ -908,8 +1078,7 @@ static int solve_form(Ctx& c, const double* b, double* xsol, double tol, int max
         hipLaunchKernelGGL(k_dinv<double>, dim3(nblocks(nV)), dim3(kBlock), 0, c.s, nV, E.rowptr.p, E.col.p, E.val.p, E.nnzb, K.rowptr.p,
                            K.col.p, K.val.p, K.nnzb, dinv);
         CIPC_LAUNCH_CHECK();
-        return pcg_run<double, double>(c, E.val.p, K.val.p, b, xsol, c.pr.ensure(n), c.pz.ensure(n), c.pp.ensure(2 * n), c.pq.ensure(n), dinv, tol,
-                                       maxIter, iters, relres, learned);
+        return pcg_run<double, double>(c, E.val.p, K.val.p, b, xsol, c.pr.ensure(n), c.pz.ensure(n), c.pp.ensure(2 * n), c.pq.ensure(n), dinv, tol, maxIter, iters, relres, learned);
     }
     // mixed forms: FP32 copies of the blocks; FP64 iterative refinement around the solve
     float* vE = c.valE32.ensure(9l * E.nnzb + 1);
