@@ -245,12 +245,21 @@ __global__ __launch_bounds__(256) void k_lp_wgrad(int nrows, int chunk, LpSeg s0
         if (pidx < P) part[(long)blockIdx.x * P + pidx] = acc[j];
     }
 }
-// grad[w] += sum_g part[g][w] (weights), grad[b] += sum_g part[g][K*NOUT + o] (bias)
-__global__ void k_lp_wgrad_sum(int ngroups, int P, int KN, const float* __restrict__ part, float* __restrict__ gw, float* __restrict__ gb) {
-    int pidx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (pidx >= P) return;
+// grad[w] += sum_g part[g][w] (weights), grad[b] += sum_g part[g][K*NOUT + o] (bias): 64
+// parameters per workgroup, the groups in four slices (each in index order) added in order
+__global__ __launch_bounds__(256) void k_lp_wgrad_sum(int ngroups, int P, int KN, const float* __restrict__ part, float* __restrict__ gw,
+                                                      float* __restrict__ gb) {
+    __shared__ float sl[4][64];
+    const int q = threadIdx.x >> 6, pidx = blockIdx.x * 64 + (threadIdx.x & 63);
+    const int per = (ngroups + 3) / 4, g1 = min(ngroups, (q + 1) * per);
     float s = 0.f;
-    for (int g = 0; g < ngroups; ++g) s += part[(long)g * P + pidx];
+    if (pidx < P)
+#pragma unroll 8
+        for (int g = q * per; g < g1; ++g) s += part[(long)g * P + pidx];
+    sl[q][threadIdx.x & 63] = s;
+    __syncthreads();
+    if (q != 0 || pidx >= P) return;
+    s = ((sl[0][threadIdx.x] + sl[1][threadIdx.x]) + sl[2][threadIdx.x]) + sl[3][threadIdx.x];
     if (pidx < KN) gw[pidx] += s;
     else gb[pidx - KN] += s;
 }
@@ -306,6 +315,200 @@ __global__ void k_lp_scatter_lower(int nL, const int* __restrict__ lEdge, const 
     de[(long)lEdge[l] * kLpHidden + f] = dE[t];
 }
 
+
+// ------------------------------------------------------------------ FP32 matrix-core layers
+// The training form of the 64-wide layers on v_mfma_f32_16x16x4_f32: FP32 inputs, weights,
+// products and accumulation, so nothing is rounded that the vector form kept.  Lane l feeds
+// A row l % 16 and B column l % 16 at one k per instruction and holds D rows 4 (l / 16) + t,
+// column l % 16.  Which k a lane feeds in which step is free as long as A and B agree: over
+// 16 k's, lane group l / 16 takes k = 4 (l / 16) + step, so that both operands of four
+// steps are one 16-byte load.  The operand held in LDS has rows of 64 n + 4 floats: the 16
+// lanes of a group then read 16 different groups of four banks.
+typedef float lp_f4 __attribute__((ext_vector_type(4)));
+constexpr int kLpF32Pad = 4;
+
+// out = act(b + [x0 x1 x2] W) (W [64 NSEG][nout], nout <= 16 NT), and sumOut = sumIn + out
+// when asked for.  A wave takes tiles of 16 rows.  Bound: the gathered rows (192 inputs per
+// edge) and the matrix cores alike; the vector form was bound by one LDS read per multiply.
+// Measured (two 61x61 sheets, 120,000 edges): 95 us per message layer; all dense layers of a
+// forward pass 1.17 -> 0.47 ms.
+template <int NSEG, int NT>
+__global__ __launch_bounds__(256, 3) void k_lp_dense_f32(int nrows, LpSeg s0, LpSeg s1, LpSeg s2, const float* __restrict__ W,
+                                                      const float* __restrict__ bias, int nout, int relu, float* __restrict__ out,
+                                                      const float* __restrict__ sumIn, float* __restrict__ sumOut) {
+    constexpr int K = 64 * NSEG, LD = K + kLpF32Pad;
+    __shared__ float Wt[16 * NT * LD];
+    // all loads of a batch in flight: one at a time, they took longer than the products.
+    // (The 64-wide layers' weights start at multiples of four floats in the flat vector.)
+    if (NT == 4) {   // nout = 64: four outputs of one k per load
+#pragma unroll 6
+        for (int t = threadIdx.x; t < K * 16; t += 256) {
+            const lp_f4 w = *reinterpret_cast<const lp_f4*>(W + 4 * t);
+            const int k = t / 16, o = 4 * (t % 16);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Wt[(o + i) * LD + k] = w[i];
+        }
+    } else {
+#pragma unroll 6
+        for (int t = threadIdx.x; t < K * 16 * NT; t += 256) {
+            const int k = t / (16 * NT), o = t % (16 * NT);
+            const float w = W[o < nout ? k * nout + o : 0];
+            Wt[o * LD + k] = o < nout ? w : 0.f;
+        }
+    }
+    __syncthreads();
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int nTiles = (nrows + 15) / 16;
+    for (int tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile < nTiles; tile += gridDim.x * 4) {
+        const int r = min(16 * tile + c, nrows - 1);
+        const float* row[3] = {s0.x + 64l * (s0.idx ? s0.idx[r] : r), NSEG > 1 ? s1.x + 64l * (s1.idx ? s1.idx[r] : r) : nullptr,
+                               NSEG > 2 ? s2.x + 64l * (s2.idx ? s2.idx[r] : r) : nullptr};
+        lp_f4 a[4 * NSEG];
+#pragma unroll
+        for (int s = 0; s < NSEG; ++s)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) a[4 * s + u] = *reinterpret_cast<const lp_f4*>(row[s] + 16 * u + 4 * g);
+        lp_f4 acc[NT];
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const float b = 16 * j + c < nout ? bias[16 * j + c] : 0.f;
+            acc[j] = lp_f4{b, b, b, b};
+        }
+#pragma unroll
+        for (int u = 0; u < 4 * NSEG; ++u)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const lp_f4 w = *reinterpret_cast<const lp_f4*>(&Wt[(16 * j + c) * LD + 16 * u + 4 * g]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][t], w[t], acc[j], 0, 0, 0);
+            }
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int rr = 16 * tile + 4 * g + t, o = 16 * j + c;
+                if (rr >= nrows || o >= nout) continue;
+                const float y = relu && !(acc[j][t] > 0.f) ? 0.f : acc[j][t];
+                out[(long)rr * nout + o] = y;
+                if (sumOut) sumOut[(long)rr * nout + o] = sumIn[(long)rr * nout + o] + y;
+            }
+    }
+}
+
+// input gradients of all segments from one pass over dY: dX_s[r][k] = sum_o dY[r][o]
+// W[64 s + k][o] (+ add_s[r][k], which may be dX_s itself: one lane reads and writes each
+// element).  W's rows are the columns of the product, so LDS holds them as they are.
+// Measured (as above): 86 us per message layer; all input gradients of a pass 2.86 -> 0.41 ms.
+struct LpGradOut {
+    const float* add;
+    float* dX;
+};
+template <int NSEG>
+__global__ __launch_bounds__(256, 3) void k_lp_dense_t_f32(int nrows, const float* __restrict__ dY, const float* __restrict__ W, LpGradOut o0,
+                                                        LpGradOut o1, LpGradOut o2) {
+    constexpr int LD = 64 + kLpF32Pad;
+    __shared__ float Wl[64 * NSEG * LD];
+#pragma unroll 6
+    for (int t = threadIdx.x; t < 16 * 64 * NSEG; t += 256)
+        *reinterpret_cast<lp_f4*>(&Wl[(t / 16) * LD + 4 * (t % 16)]) = *reinterpret_cast<const lp_f4*>(W + 4 * t);
+    __syncthreads();
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    const int nTiles = (nrows + 15) / 16;
+    for (int tile = blockIdx.x * 4 + (threadIdx.x >> 6); tile < nTiles; tile += gridDim.x * 4) {
+        const int r = min(16 * tile + c, nrows - 1);
+        lp_f4 a[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[u] = *reinterpret_cast<const lp_f4*>(dY + 64l * r + 16 * u + 4 * g);
+#pragma unroll
+        for (int s = 0; s < NSEG; ++s) {
+            const LpGradOut os = s == 0 ? o0 : s == 1 ? o1 : o2;
+            lp_f4 acc[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j] = lp_f4{0, 0, 0, 0};
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const lp_f4 w = *reinterpret_cast<const lp_f4*>(&Wl[(64 * s + 16 * j + c) * LD + 16 * u + 4 * g]);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][t], w[t], acc[j], 0, 0, 0);
+                }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const int rr = 16 * tile + 4 * g + t;
+                    if (rr >= nrows) continue;
+                    const long e = 64l * rr + 16 * j + c;
+                    os.dX[e] = os.add ? acc[j][t] + os.add[e] : acc[j][t];
+                }
+        }
+    }
+}
+
+// weight gradient partials: workgroup g sums x_seg[idx(r)]^T dY[r] over rows [g chunk,
+// (g + 1) chunk) into part[g][64 NSEG nout + nout] (bias last).  The contraction runs over
+// rows: wave w holds the NSEG tiles of 16 inputs 16 (4 i + w) against all NT output tiles,
+// four rows per instruction, the loads of 16 rows in flight.
+// Measured (as above): 76 us per message layer; all weight gradients of a pass 3.5 -> 0.55 ms
+// with the sums over the row ranges.
+template <int NSEG, int NT>
+__global__ __launch_bounds__(256) void k_lp_wgrad_f32(int nrows, int chunk, LpSeg s0, LpSeg s1, LpSeg s2, const float* __restrict__ dY,
+                                                      int nout, float* __restrict__ part) {
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4, w = threadIdx.x >> 6;
+    const int P = 64 * NSEG * nout + nout;
+    lp_f4 acc[NSEG][NT];
+    float bsum[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        bsum[j] = 0.f;
+#pragma unroll
+        for (int s = 0; s < NSEG; ++s) acc[s][j] = lp_f4{0, 0, 0, 0};
+    }
+    const int rbeg = blockIdx.x * chunk, rend = min(nrows, rbeg + chunk);
+    for (int r0 = rbeg; r0 < rend; r0 += 16) {
+        float a[4][NSEG], b[4][NT];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int r = r0 + 4 * u + g;
+            const bool on = r < rend;
+            const int rc = on ? r : rbeg;
+#pragma unroll
+            for (int s = 0; s < NSEG; ++s) {
+                const LpSeg sg = s == 0 ? s0 : s == 1 ? s1 : s2;
+                a[u][s] = sg.x[64l * (sg.idx ? sg.idx[rc] : rc) + 16 * w + c];
+            }
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const bool in = on && 16 * j + c < nout;
+                const float v = dY[in ? (long)rc * nout + 16 * j + c : 0];
+                b[u][j] = in ? v : 0.f;   // rows beyond the range contribute zero products
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                bsum[j] += b[u][j];
+#pragma unroll
+                for (int s = 0; s < NSEG; ++s) acc[s][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][s], b[u][j], acc[s][j], 0, 0, 0);
+            }
+    }
+    float* dst = part + (long)blockIdx.x * P;
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        const int o = 16 * j + c;
+        float bs = bsum[j];
+        bs += __shfl_xor(bs, 16, 64);
+        bs += __shfl_xor(bs, 32, 64);
+        if (o >= nout) continue;
+#pragma unroll
+        for (int s = 0; s < NSEG; ++s)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) dst[(64 * s + 16 * w + 4 * g + t) * nout + o] = acc[s][j][t];
+        if (w == 0 && g == 0) dst[64 * NSEG * nout + o] = bs;
+    }
+}
 
 // ------------------------------------------------------------------ MFMA inference layers
 // Inference form of the dense layers on the matrix cores: inputs and weights in BF16,
@@ -879,7 +1082,7 @@ void lp_build_graph(Ctx& c) {
     lp.Gl.ensure_exact(9 * (size_t)std::max(nL, 1));
     lp.raw.ensure_exact(6 * (size_t)nV);
     lp.Gblk.ensure_exact(9 * (size_t)nnzb);
-    lp.wpartial.ensure_exact((size_t)256 * (kLpMaxK * kLpHidden + kLpHidden));
+    lp.wpartial.ensure_exact((size_t)512 * (kLpMaxK * kLpHidden + kLpHidden));
     lp.graphReady = true;
     lp.forwardReady = false;
 }
@@ -986,16 +1189,45 @@ static void wgrad(Ctx& c, int nrows, LpSeg s0, LpSeg s1, LpSeg s2, const float* 
     chunk = (chunk + kLpRows - 1) / kLpRows * kLpRows;
     float* part = lp.wpartial.ensure((size_t)groups * P);
     hipLaunchKernelGGL(k_lp_wgrad<NOUT>, dim3(groups), dim3(256), 0, c.s, nrows, chunk, s0, s1, s2, dY, part);
-    hipLaunchKernelGGL(k_lp_wgrad_sum, dim3(nblocks(P)), dim3(kBlock), 0, c.s, groups, P, K * NOUT, (const float*)part, gw, gb);
+    hipLaunchKernelGGL(k_lp_wgrad_sum, dim3((P + 63) / 64), dim3(256), 0, c.s, groups, P, K * NOUT, (const float*)part, gw, gb);
     CIPC_LAUNCH_CHECK();
 }
-__global__ void k_lp_add(long n, const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ out) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) out[i] = a[i] + b[i];
+// the 64-wide layers (every segment 64 features) on the FP32 matrix cores
+static int f32_segments(LpSeg s0, LpSeg s1, LpSeg s2) {
+    if (s0.k != 64 || (s1.k != 0 && s1.k != 64) || (s2.k != 0 && s2.k != 64) || (s2.k && !s1.k))
+        throw HipError("learned preconditioner: segment widths", -1);
+    return 1 + (s1.k != 0) + (s2.k != 0);
 }
-static void add(Ctx& c, long n, const float* a, const float* b, float* out) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_lp_add, dim3((unsigned)((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.s, n, a, b, out);
+// workgroups: four tiles of 16 rows each at a time, the weights in LDS loaded once
+constexpr int kLpF32Grid = 768;   // three resident workgroups per CU
+static void dense_f32(Ctx& c, int nrows, LpSeg s0, LpSeg s1, LpSeg s2, const float* W, const float* b, int nout, int relu, float* out,
+                      const float* sumIn = nullptr, float* sumOut = nullptr) {
+    if (nrows <= 0) return;
+    const int ns = f32_segments(s0, s1, s2);
+    const int grid = std::min(kLpF32Grid, (nrows + 63) / 64);
+    auto kern = nout == 64 ? (ns == 3 ? k_lp_dense_f32<3, 4> : ns == 2 ? k_lp_dense_f32<2, 4> : k_lp_dense_f32<1, 4>)
+                          : (ns == 3 ? k_lp_dense_f32<3, 1> : ns == 2 ? k_lp_dense_f32<2, 1> : k_lp_dense_f32<1, 1>);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), 0, c.s, nrows, s0, s1, s2, W, b, nout, relu, out, sumIn, sumOut);
+    CIPC_LAUNCH_CHECK();
+}
+static void dense_t_f32(Ctx& c, int nrows, const float* dY, const float* W, int ns, LpGradOut o0, LpGradOut o1, LpGradOut o2 = {nullptr, nullptr}) {
+    if (nrows <= 0) return;
+    const int grid = std::min(kLpF32Grid, (nrows + 63) / 64);
+    hipLaunchKernelGGL((ns == 3 ? k_lp_dense_t_f32<3> : k_lp_dense_t_f32<2>), dim3(grid), dim3(256), 0, c.s, nrows, dY, W, o0, o1, o2);
+    CIPC_LAUNCH_CHECK();
+}
+static void wgrad_f32(Ctx& c, int nrows, LpSeg s0, LpSeg s1, LpSeg s2, const float* dY, int nout, float* gw, float* gb) {
+    if (nrows <= 0) return;
+    LearnedPrecond& lp = LP(c);
+    const int ns = f32_segments(s0, s1, s2), P = 64 * ns * nout + nout;
+    const int groups = std::min(512, (nrows + 63) / 64);
+    const int chunk = ((nrows + groups - 1) / groups + 15) / 16 * 16;
+    const int used = (nrows + chunk - 1) / chunk;
+    float* part = lp.wpartial.ensure((size_t)used * P);
+    auto kern = nout > 16 ? (ns == 3 ? k_lp_wgrad_f32<3, 4> : ns == 2 ? k_lp_wgrad_f32<2, 4> : k_lp_wgrad_f32<1, 4>)
+                          : (ns == 3 ? k_lp_wgrad_f32<3, 1> : ns == 2 ? k_lp_wgrad_f32<2, 1> : k_lp_wgrad_f32<1, 1>);
+    hipLaunchKernelGGL(kern, dim3(used), dim3(256), 0, c.s, nrows, chunk, s0, s1, s2, dY, nout, part);
+    hipLaunchKernelGGL(k_lp_wgrad_sum, dim3((P + 63) / 64), dim3(256), 0, c.s, used, P, 64 * ns * nout, (const float*)part, gw, gb);
     CIPC_LAUNCH_CHECK();
 }
 
@@ -1073,8 +1305,8 @@ static void lp_forward_mfma(Ctx& c) {
                    1, lp.h[l].p, lp.h[l + 1].p);
     }
     const float* hL = lp.h[kLpLayers].p;
-    dense<9>(c, nL, {hL, lp.lowSrc.p, kLpHidden}, {hL, lp.lowDst.p, kLpHidden}, {lp.e[kLpLayers].p, lp.lEdge.p, kLpHidden}, Wq + L.wo,
-             Wq + L.bo, 0, nullptr, lp.Gl.p);
+    dense_f32(c, nL, {hL, lp.lowSrc.p, kLpHidden}, {hL, lp.lowDst.p, kLpHidden}, {lp.e[kLpLayers].p, lp.lEdge.p, kLpHidden}, Wq + L.wo,
+              Wq + L.bo, 9, 0, lp.Gl.p);
     mfma_dense(c, nV, {hL, nullptr, kLpHidden}, kNoSeg, kNoSeg, Wq + L.wd, Wq + L.bd, 6, 0, nullptr, lp.raw.p);
 }
 
@@ -1083,7 +1315,6 @@ void lp_forward(Ctx& c) {
     const LpLayout& L = lp.L;
     const float* Wq = lp.Wq.p;
     const int nV = lp.nV, nE = lp.nE, nL = lp.nL;
-    const long H = kLpHidden;
     if (lp.mfma) {
         lp_forward_mfma(c);
         lp_assemble(c);
@@ -1093,18 +1324,16 @@ void lp_forward(Ctx& c) {
     dense<kLpHidden>(c, nE, {lp.edgeF.p, nullptr, kLpEdgeIn}, kNoSeg, kNoSeg, Wq + L.wx, Wq + L.bx, 1, nullptr, lp.e[0].p);
     for (int l = 0; l < kLpLayers; ++l) {
         const LpSeg ms0 = {lp.h[l].p, lp.eSrc.p, kLpHidden}, ms1 = {lp.h[l].p, lp.eDst.p, kLpHidden}, ms2 = {lp.e[l].p, nullptr, kLpHidden};
-        dense<kLpHidden>(c, nE, ms0, ms1, ms2, Wq + L.wm[l], Wq + L.bm[l], 1, nullptr, lp.m[l].p);
-        add(c, H * nE, lp.e[l].p, lp.m[l].p, lp.e[l + 1].p);
+        dense_f32(c, nE, ms0, ms1, ms2, Wq + L.wm[l], Wq + L.bm[l], kLpHidden, 1, lp.m[l].p, lp.e[l].p, lp.e[l + 1].p);
         hipLaunchKernelGGL(k_lp_agg, dim3((nV + 3) / 4), dim3(256), 0, c.s, nV, (const int*)lp.erp.p, (const float*)lp.m[l].p, lp.agg[l].p);
         CIPC_LAUNCH_CHECK();
-        dense<kLpHidden>(c, nV, {lp.h[l].p, nullptr, kLpHidden}, {lp.agg[l].p, nullptr, kLpHidden}, kNoSeg, Wq + L.wu[l], Wq + L.bu[l], 1,
-                         nullptr, lp.u[l].p);
-        add(c, H * nV, lp.h[l].p, lp.u[l].p, lp.h[l + 1].p);
+        dense_f32(c, nV, {lp.h[l].p, nullptr, kLpHidden}, {lp.agg[l].p, nullptr, kLpHidden}, kNoSeg, Wq + L.wu[l], Wq + L.bu[l], kLpHidden, 1,
+                  lp.u[l].p, lp.h[l].p, lp.h[l + 1].p);
     }
     const float* hL = lp.h[kLpLayers].p;
-    dense<9>(c, nL, {hL, lp.lowSrc.p, kLpHidden}, {hL, lp.lowDst.p, kLpHidden}, {lp.e[kLpLayers].p, lp.lEdge.p, kLpHidden}, Wq + L.wo,
-             Wq + L.bo, 0, nullptr, lp.Gl.p);
-    dense<6>(c, nV, {hL, nullptr, kLpHidden}, kNoSeg, kNoSeg, Wq + L.wd, Wq + L.bd, 0, nullptr, lp.raw.p);
+    dense_f32(c, nL, {hL, lp.lowSrc.p, kLpHidden}, {hL, lp.lowDst.p, kLpHidden}, {lp.e[kLpLayers].p, lp.lEdge.p, kLpHidden}, Wq + L.wo,
+              Wq + L.bo, 9, 0, lp.Gl.p);
+    dense_f32(c, nV, {hL, nullptr, kLpHidden}, kNoSeg, kNoSeg, Wq + L.wd, Wq + L.bd, 6, 0, lp.raw.p);
     lp_assemble(c);
 }
 
@@ -1250,8 +1479,8 @@ double lp_loss_grad(Ctx& c, int nProbes, uint64_t seed, float* gradOut) {
     const float* Wq = lp.Wq.p;
     const float* hL = lp.h[kLpLayers].p;
     // decoder, lower blocks
-    wgrad<9>(c, nL, {hL, lp.lowSrc.p, kLpHidden}, {hL, lp.lowDst.p, kLpHidden}, {lp.e[kLpLayers].p, lp.lEdge.p, kLpHidden}, dGl, gW + L.wo,
-             gW + L.bo);
+    wgrad_f32(c, nL, {hL, lp.lowSrc.p, kLpHidden}, {hL, lp.lowDst.p, kLpHidden}, {lp.e[kLpLayers].p, lp.lEdge.p, kLpHidden}, dGl, 9,
+              gW + L.wo, gW + L.bo);
     dense_t<9>(c, nL, dGl, Wq + L.wo, 0, nullptr, t1);
     dense_t<9>(c, nL, dGl, Wq + L.wo, kLpHidden, nullptr, t2);
     dense_t<9>(c, nL, dGl, Wq + L.wo, 2 * kLpHidden, nullptr, t3);
@@ -1265,26 +1494,24 @@ double lp_loss_grad(Ctx& c, int nProbes, uint64_t seed, float* gradOut) {
     }
     CIPC_LAUNCH_CHECK();
     // decoder, diagonal blocks
-    wgrad<6>(c, nV, {hL, nullptr, kLpHidden}, kNoSeg, kNoSeg, draw, gW + L.wd, gW + L.bd);
+    wgrad_f32(c, nV, {hL, nullptr, kLpHidden}, kNoSeg, kNoSeg, draw, 6, gW + L.wd, gW + L.bd);
     dense_t<6>(c, nV, draw, Wq + L.wd, 0, dh, dh);
     // message-passing layers in reverse
     for (int l = kLpLayers - 1; l >= 0; --l) {
         // h[l+1] = h[l] + u[l],  u[l] = relu(Wu [h[l], agg[l]] + bu)
         hipLaunchKernelGGL(k_lp_relu_mask, dim3(nblocks(H * nV)), dim3(kBlock), 0, c.s, H * nV, (const float*)lp.u[l].p, (const float*)dh, t1);
         CIPC_LAUNCH_CHECK();
-        wgrad<kLpHidden>(c, nV, {lp.h[l].p, nullptr, kLpHidden}, {lp.agg[l].p, nullptr, kLpHidden}, kNoSeg, t1, gW + L.wu[l], gW + L.bu[l]);
-        dense_t<kLpHidden>(c, nV, t1, Wq + L.wu[l], kLpHidden, nullptr, dagg);
-        dense_t<kLpHidden>(c, nV, t1, Wq + L.wu[l], 0, dh, dh);
+        wgrad_f32(c, nV, {lp.h[l].p, nullptr, kLpHidden}, {lp.agg[l].p, nullptr, kLpHidden}, kNoSeg, t1, kLpHidden, gW + L.wu[l],
+                  gW + L.bu[l]);
+        dense_t_f32(c, nV, t1, Wq + L.wu[l], 2, {dh, dh}, {nullptr, dagg});
         if (nE == 0) continue;
         // e[l+1] = e[l] + m[l],  m[l] = relu(Wm [h[l]_src, h[l]_dst, e[l]] + bm),  agg[l] = row sums of m[l]
         hipLaunchKernelGGL(k_lp_msg_grad, dim3((unsigned)((H * nE + kBlock - 1) / kBlock)), dim3(kBlock), 0, c.s, H * nE, (const int*)lp.eSrc.p,
                            (const float*)de, (const float*)dagg, (const float*)lp.m[l].p, t2);
         CIPC_LAUNCH_CHECK();
-        wgrad<kLpHidden>(c, nE, {lp.h[l].p, lp.eSrc.p, kLpHidden}, {lp.h[l].p, lp.eDst.p, kLpHidden}, {lp.e[l].p, nullptr, kLpHidden}, t2,
-                         gW + L.wm[l], gW + L.bm[l]);
-        dense_t<kLpHidden>(c, nE, t2, Wq + L.wm[l], 0, nullptr, t3);
-        dense_t<kLpHidden>(c, nE, t2, Wq + L.wm[l], kLpHidden, nullptr, de2);
-        dense_t<kLpHidden>(c, nE, t2, Wq + L.wm[l], 2 * kLpHidden, de, de);
+        wgrad_f32(c, nE, {lp.h[l].p, lp.eSrc.p, kLpHidden}, {lp.h[l].p, lp.eDst.p, kLpHidden}, {lp.e[l].p, nullptr, kLpHidden}, t2, kLpHidden,
+                  gW + L.wm[l], gW + L.bm[l]);
+        dense_t_f32(c, nE, t2, Wq + L.wm[l], 3, {nullptr, t3}, {nullptr, de2}, {de, de});
         hipLaunchKernelGGL(k_lp_gather_node, dim3((nV + 3) / 4), dim3(256), 0, c.s, nV, (const int*)lp.erp.p, (const int*)lp.eT.p,
                            (const float*)t3, (const float*)de2, dh);
         CIPC_LAUNCH_CHECK();
