@@ -8,15 +8,17 @@
 // (alpha /= alpha * mean|p| / voxel when > 1) and the overlap test are reproduced
 // exactly, so the candidate set, and with it the step size, matches the reference
 // rule.  Candidates are enumerated through cells of f x f x f voxels (f grown until the
-// cell table fits), then filtered by the exact voxel-range overlap.
+// cell table fits; walk.hpp), filtered by the exact voxel-range overlap.
 //
-// Each candidate runs the additive CCD in FP64 with the running per-primitive step as
-// its cut-off, as the reference does; every loop stops after at most ACCD_MAX_ITERS
+// Each candidate runs the additive CCD in FP64 with the smallest step found so far as its
+// cut-off (the reference: the primitive's running step; the minimum over all pairs is the
+// same); every loop stops after at most ACCD_MAX_ITERS
 // advances (touching stencils would otherwise never end) with the conservative time
 // accumulated so far.  The global step is a min-reduction over positive doubles
 // through their bit patterns (atomicMin on uint64).
 #include "ctx.hpp"
 #include "dev_math.hpp"
+#include "walk.hpp"
 #include <algorithm>
 #include <cmath>
 
@@ -301,7 +303,7 @@ __global__ void k_prim_vox_emit(int n, const int* __restrict__ plo, const int* _
         for (int iy = a[1]; iy <= b[1]; ++iy)
             for (int ix = a[0]; ix <= b[0]; ++ix) {
                 keys[o] = (uint64_t)ix + (uint64_t)G.edim[0] * ((uint64_t)iy + (uint64_t)G.edim[1] * (uint64_t)iz);
-                vals[o] = (uint32_t)i;
+                vals[o] = walk_entry(i, ix == a[0], iy == a[1], iz == a[2]);
                 ++o;
             }
 }
@@ -317,135 +319,110 @@ __device__ __forceinline__ void atomic_min_pos(unsigned long long* a, double v) 
     atomicMin(a, (unsigned long long)__double_as_longlong(v));
 }
 
-// voxel box of primitive i from its 32-byte record: lo = (a.x, a.y, a.z), hi = (a.w, b.x, b.y)
-struct VBox {
-    int4 a, b;
+// The step so far: the smallest of the workgroup's and the other workgroups' results, which
+// cuts the additive CCD off.  The minimum over all pairs does not depend on the cut-offs: a
+// pair is only given up once its time exceeds one that is already found.
+struct StepMin {
+    unsigned long long* __restrict__ gmin;
+    uint32_t* __restrict__ zero;
+    unsigned long long* best;   // LDS
+    __device__ __forceinline__ double cut() const {
+        const unsigned long long g = __hip_atomic_load(gmin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return __longlong_as_double((long long)min(g, *best));   // positive doubles order as their bits
+    }
+    __device__ __forceinline__ void found(double la) const {
+        const unsigned long long v = (unsigned long long)__double_as_longlong(la);
+        if (v < atomicMin(best, v)) atomicMin(gmin, v);
+        if (la == 0) atomicOr(zero, 1u);
+    }
 };
-__device__ __forceinline__ VBox ld_box(const int4* __restrict__ box, int i) { return {box[2l * i], box[2l * i + 1]}; }
-__device__ __forceinline__ bool box_overlap(const VBox& A, const VBox& B) {
-    return !(A.a.x > B.a.w || B.a.x > A.a.w || A.a.y > B.b.x || B.a.y > A.b.x || A.a.z > B.b.y || B.a.z > A.b.y);
+// two voxel boxes (lo xyz, hi x | hi yz)
+__device__ __forceinline__ bool box_overlap(const int4& Aa, const int4& Ab, const int4& Ba, const int4& Bb) {
+    return !(Aa.x > Ba.w || Ba.x > Aa.w || Aa.y > Bb.x || Ba.y > Ab.x || Aa.z > Bb.y || Ba.z > Ab.y);
 }
-
-// point vI against triangle t (IPC.h:2120-2164): exact voxel-range overlap (the
-// triangle's box record), shared vertex and Dirichlet filters, swept-box broad phase,
-// additive CCD with the running step `largest` as cut-off
-__device__ __forceinline__ void pt_ccd_candidate_box(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ tri,
-                                                     int nT, const uint8_t* __restrict__ dbc, const VBox& T, int vI, const int* nlo,
-                                                     const int* nhi, d3 P, d3 dP, int t, double xi, double& largest,
-                                                     uint32_t* __restrict__ zero) {
-    if (nlo[0] > T.a.w || T.a.x > nhi[0] || nlo[1] > T.b.x || T.a.y > nhi[1] || nlo[2] > T.b.y || T.a.z > nhi[2]) return;
-    int a = tri[t], b = tri[nT + t], c = tri[2 * nT + t];
-    if (vI == a || vI == b || vI == c) return;
-    if (dbc[vI] && dbc[a] && dbc[b] && dbc[c]) return;
-    d3 t0 = ld3(x, a), t1 = ld3(x, b), t2 = ld3(x, c);
-    d3 d0 = ld3(p, a), d1 = ld3(p, b), d2 = ld3(p, c);
-    if (!pt_ccd_broadphase(P, t0, t1, t2, dP, d0, d1, d2, xi)) return;
-    double la = largest;
-    if (pt_accd(P, t0, t1, t2, dP, d0, d1, d2, 0.1, xi, la)) {
-        if (largest > la) largest = la;
-        if (la == 0) atomicOr(zero, 1u);
-    }
+__device__ __forceinline__ void box_cells(const int4& a, const int4& b, const VoxGrid& G, int* qlo, int* qhi) {
+    qlo[0] = ecell(a.x, G.f, G.edim[0]); qlo[1] = ecell(a.y, G.f, G.edim[1]); qlo[2] = ecell(a.z, G.f, G.edim[2]);
+    qhi[0] = ecell(a.w, G.f, G.edim[0]); qhi[1] = ecell(b.x, G.f, G.edim[1]); qhi[2] = ecell(b.y, G.f, G.edim[2]);
 }
-// edge pair eA < eB (IPC.h:2166-2242) with both box records loaded; edge A first in
-// the additive CCD
-__device__ __forceinline__ void ee_ccd_candidate_box(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ bEdge,
-                                                     int nBE, const uint8_t* __restrict__ dbc, const VBox& A, const VBox& B, int eA, int eB,
-                                                     double xi, double& largest, uint32_t* __restrict__ zero) {
-    if (!box_overlap(A, B)) return;
-    int a0 = bEdge[eA], a1 = bEdge[nBE + eA], b0 = bEdge[eB], b1 = bEdge[nBE + eB];
-    if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) return;
-    if (dbc[a0] && dbc[a1] && dbc[b0] && dbc[b1]) return;
-    d3 A0 = ld3(x, a0), A1 = ld3(x, a1), dA0 = ld3(p, a0), dA1 = ld3(p, a1);
-    d3 B0 = ld3(x, b0), B1 = ld3(x, b1), dB0 = ld3(p, b0), dB1 = ld3(p, b1);
-    if (!ee_ccd_broadphase(A0, A1, B0, B1, dA0, dA1, dB0, dB1, xi)) return;
-    double la = largest;
-    if (ee_accd(A0, A1, B0, B1, dA0, dA1, dB0, dB1, 0.1, xi, la)) {
-        if (largest > la) largest = la;
-        if (la == 0) atomicOr(zero, 1u);
+// point against triangle (IPC.h:2120-2164): exact voxel-range overlap, shared vertex and
+// Dirichlet filters, swept-box broad phase, additive CCD
+struct CcdPT {
+    const double* __restrict__ x;
+    const double* __restrict__ p;
+    const int* __restrict__ bNode;
+    const int* __restrict__ tri;
+    int nT;
+    const uint8_t* __restrict__ dbc;
+    const int* __restrict__ vlo;
+    const int* __restrict__ vhi;
+    int nV;
+    VoxGrid G;
+    double xi;
+    StepMin m;
+    int4 qa, qb;
+    __device__ __forceinline__ bool begin(int slot, int* qlo, int* qhi) {
+        const int v = bNode[slot];
+        qa = make_int4(vlo[v], vlo[nV + v], vlo[2 * nV + v], vhi[v]);
+        qb = make_int4(vhi[nV + v], vhi[2 * nV + v], 0, 0);
+        box_cells(qa, qb, G, qlo, qhi);
+        return true;
     }
-}
-__global__ void k_ccd_pt(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ bNode, int nBN,
-                         const int* __restrict__ tri, int nT, const uint8_t* __restrict__ dbc, const int* __restrict__ vlo,
-                         const int* __restrict__ vhi, int nV, const int4* __restrict__ tbox, VoxGrid G,
-                         const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, const int4* __restrict__ crec,
-                         const int* __restrict__ lgList, const uint32_t* __restrict__ lgCount, double alpha0, double xi,
-                         unsigned long long* __restrict__ gmin, uint32_t* __restrict__ zero) {
-    int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nBN) return;
-    int vI = bNode[s];
-    int nlo[3], nhi[3], qlo[3], qhi[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        nlo[d] = vlo[d * nV + vI]; nhi[d] = vhi[d * nV + vI];
-        qlo[d] = ecell(nlo[d], G.f, G.edim[d]); qhi[d] = ecell(nhi[d], G.f, G.edim[d]);
+    __device__ __forceinline__ bool accept(int, int, const int4& a, const int4& b, bool) const { return box_overlap(qa, qb, a, b); }
+    __device__ __forceinline__ void flush(bool) const {}
+    __device__ __forceinline__ void exact(int slot, int t) const {
+        const int vI = bNode[slot], a = tri[t], b = tri[nT + t], c = tri[2 * nT + t];
+        if (vI == a || vI == b || vI == c) return;
+        if (dbc[vI] && dbc[a] && dbc[b] && dbc[c]) return;
+        d3 P = ld3(x, vI), dP = ld3(p, vI), t0 = ld3(x, a), t1 = ld3(x, b), t2 = ld3(x, c);
+        d3 d0 = ld3(p, a), d1 = ld3(p, b), d2 = ld3(p, c);
+        if (!pt_ccd_broadphase(P, t0, t1, t2, dP, d0, d1, d2, xi)) return;
+        double la = m.cut();
+        if (pt_accd(P, t0, t1, t2, dP, d0, d1, d2, 0.1, xi, la)) m.found(la);
     }
-    d3 P = ld3(x, vI), dP = ld3(p, vI);
-    double largest = alpha0;
-    for (int iz = qlo[2]; iz <= qhi[2]; ++iz)
-        for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
-            for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
-                uint64_t cell = (uint64_t)ix + (uint64_t)G.edim[0] * ((uint64_t)iy + (uint64_t)G.edim[1] * (uint64_t)iz);
-                uint32_t st = start[cell], en = end[cell];
-                for (uint32_t k = st; k < en; ++k) {
-                    const VBox T = ld_box(crec, (int)k);   // the cell's records are contiguous
-                    const int t = T.b.z;
-                    if (ix != max(qlo[0], ecell(T.a.x, G.f, G.edim[0])) || iy != max(qlo[1], ecell(T.a.y, G.f, G.edim[1])) ||
-                        iz != max(qlo[2], ecell(T.a.z, G.f, G.edim[2])))
-                        continue;
-                    pt_ccd_candidate_box(x, p, tri, nT, dbc, T, vI, nlo, nhi, P, dP, t, xi, largest, zero);
-                }
-            }
-    const uint32_t nl = *lgCount;
-    for (uint32_t k = 0; k < nl; ++k) {
-        const int t = lgList[k];
-        pt_ccd_candidate_box(x, p, tri, nT, dbc, ld_box(tbox, t), vI, nlo, nhi, P, dP, t, xi, largest, zero);
+};
+// edge pair (IPC.h:2166-2242), the edge of smaller index first; pair coverage as in
+// k_query_ee: grid-listed edges take grid-listed partners of larger index plus every large
+// edge; large edges take large partners of larger index
+struct CcdEE {
+    const double* __restrict__ x;
+    const double* __restrict__ p;
+    const int* __restrict__ bEdge;
+    int nBE;
+    const uint8_t* __restrict__ dbc;
+    const int4* __restrict__ box;
+    const uint8_t* __restrict__ lgFlag;
+    VoxGrid G;
+    double xi;
+    StepMin m;
+    int4 qa, qb;
+    __device__ __forceinline__ bool begin(int e, int* qlo, int* qhi) {
+        qa = box[2l * e];
+        qb = box[2l * e + 1];
+        box_cells(qa, qb, G, qlo, qhi);
+        return !lgFlag[e];
     }
-    if (largest < alpha0) atomic_min_pos(gmin, largest);
-}
-
-// pair coverage as in k_query_ee: grid-listed edges take grid-listed partners of
-// larger index plus every large edge; large edges take large partners of larger index
-__global__ void k_ccd_ee(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ bEdge, int nBE,
-                         const uint8_t* __restrict__ dbc, const int4* __restrict__ ebox, VoxGrid G,
-                         const uint32_t* __restrict__ start, const uint32_t* __restrict__ end, const int4* __restrict__ crec,
-                         const uint8_t* __restrict__ lgFlag, const int* __restrict__ lgList, const uint32_t* __restrict__ lgCount,
-                         double alpha0, double xi, unsigned long long* __restrict__ gmin, uint32_t* __restrict__ zero) {
-    int eI = blockIdx.x * blockDim.x + threadIdx.x;
-    if (eI >= nBE) return;
-    double largest = alpha0;
-    const uint32_t nl = *lgCount;
-    const VBox A = ld_box(ebox, eI);
-    if (lgFlag[eI]) {
-        for (uint32_t k = 0; k < nl; ++k) {
-            int eJ = lgList[k];
-            if (eJ > eI) ee_ccd_candidate_box(x, p, bEdge, nBE, dbc, A, ld_box(ebox, eJ), eI, eJ, xi, largest, zero);
-        }
-    } else {
-        const int qlo[3] = {ecell(A.a.x, G.f, G.edim[0]), ecell(A.a.y, G.f, G.edim[1]), ecell(A.a.z, G.f, G.edim[2])};
-        const int qhi[3] = {ecell(A.a.w, G.f, G.edim[0]), ecell(A.b.x, G.f, G.edim[1]), ecell(A.b.y, G.f, G.edim[2])};
-        for (int iz = qlo[2]; iz <= qhi[2]; ++iz)
-            for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
-                for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
-                    uint64_t cell = (uint64_t)ix + (uint64_t)G.edim[0] * ((uint64_t)iy + (uint64_t)G.edim[1] * (uint64_t)iz);
-                    uint32_t st = start[cell], en = end[cell];
-                    for (uint32_t k = st; k < en; ++k) {
-                        const VBox B = ld_box(crec, (int)k);   // the cell's records are contiguous
-                        const int eJ = B.b.z;
-                        if (eJ <= eI) continue;
-                        if (ix != max(qlo[0], ecell(B.a.x, G.f, G.edim[0])) || iy != max(qlo[1], ecell(B.a.y, G.f, G.edim[1])) ||
-                            iz != max(qlo[2], ecell(B.a.z, G.f, G.edim[2])))
-                            continue;
-                        ee_ccd_candidate_box(x, p, bEdge, nBE, dbc, A, B, eI, eJ, xi, largest, zero);
-                    }
-                }
-        for (uint32_t k = 0; k < nl; ++k) {
-            int eJ = lgList[k];
-            const VBox B = ld_box(ebox, eJ);
-            if (eJ > eI) ee_ccd_candidate_box(x, p, bEdge, nBE, dbc, A, B, eI, eJ, xi, largest, zero);
-            else ee_ccd_candidate_box(x, p, bEdge, nBE, dbc, B, A, eJ, eI, xi, largest, zero);
-        }
+    __device__ __forceinline__ bool accept(int e, int other, const int4& a, const int4& b, bool anyOrder) const {
+        return (anyOrder || other > e) && box_overlap(qa, qb, a, b);
     }
-    if (largest < alpha0) atomic_min_pos(gmin, largest);
+    __device__ __forceinline__ void flush(bool) const {}
+    __device__ __forceinline__ void exact(int e, int other) const {
+        const int eA = min(e, other), eB = max(e, other);
+        const int a0 = bEdge[eA], a1 = bEdge[nBE + eA], b0 = bEdge[eB], b1 = bEdge[nBE + eB];
+        if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) return;
+        if (dbc[a0] && dbc[a1] && dbc[b0] && dbc[b1]) return;
+        d3 A0 = ld3(x, a0), A1 = ld3(x, a1), dA0 = ld3(p, a0), dA1 = ld3(p, a1);
+        d3 B0 = ld3(x, b0), B1 = ld3(x, b1), dB0 = ld3(p, b0), dB1 = ld3(p, b1);
+        if (!ee_ccd_broadphase(A0, A1, B0, B1, dA0, dA1, dB0, dB1, xi)) return;
+        double la = m.cut();
+        if (ee_accd(A0, A1, B0, B1, dA0, dA1, dB0, dB1, 0.1, xi, la)) m.found(la);
+    }
+};
+template <class P>
+__global__ __launch_bounds__(kBlock) void k_ccd_walk(P T, int n, double alpha0, CellGrid G) {
+    __shared__ unsigned long long best;
+    T.m.best = &best;
+    if (threadIdx.x == 0) best = (unsigned long long)__double_as_longlong(alpha0);   // the walk's first barrier orders it
+    walk_pairs(T, n, G);
 }
 
 // particle (boundary-node slot s >= codimBN1) against rod segments, IPC.h:2095-2133,
@@ -487,13 +464,13 @@ __global__ void k_ccd_codim(const double* __restrict__ x, const double* __restri
                             const int* __restrict__ vlo, const int* __restrict__ vhi, int nV, const int* __restrict__ elo,
                             const int* __restrict__ ehi, VoxGrid G, const uint32_t* __restrict__ estart, const uint32_t* __restrict__ eend,
                             const uint32_t* __restrict__ evals, const int* __restrict__ lgListE, const uint32_t* __restrict__ lgCountE,
-                            const int* __restrict__ plo, const uint32_t* __restrict__ pstart, const uint32_t* __restrict__ pend,
+                            const uint32_t* __restrict__ pstart, const uint32_t* __restrict__ pend,
                             const uint32_t* __restrict__ pvals, const uint8_t* __restrict__ lgFlagP, const int* __restrict__ lgListP,
                             const uint32_t* __restrict__ lgCountP, double alpha0, double xi, unsigned long long* __restrict__ gmin) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     int s = codimBN1 + j;
     if (s >= nBN) return;
-    const int nPart = nBN - codimBN1, firstRod = nBE - nRod;
+    const int firstRod = nBE - nRod;
     int vI = bNode[s];
     int nlo[3], nhi[3], qlo[3], qhi[3];
 #pragma unroll
@@ -509,20 +486,17 @@ __global__ void k_ccd_codim(const double* __restrict__ x, const double* __restri
             for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
                 for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
                     uint64_t cell = (uint64_t)ix + (uint64_t)G.edim[0] * ((uint64_t)iy + (uint64_t)G.edim[1] * (uint64_t)iz);
+                    const int own = (ix == qlo[0] ? 1 : 0) | (iy == qlo[1] ? 2 : 0) | (iz == qlo[2] ? 4 : 0);
                     for (uint32_t k = estart[cell], en = eend[cell]; k < en; ++k) {
-                        int e = (int)evals[k];
+                        const int e = (int)(evals[k] & kWalkId), first = (int)(evals[k] >> kWalkIdBits);
                         if (e < firstRod) continue;
-                        if (ix != max(qlo[0], ecell(elo[e], G.f, G.edim[0])) || iy != max(qlo[1], ecell(elo[nBE + e], G.f, G.edim[1])) ||
-                            iz != max(qlo[2], ecell(elo[2l * nBE + e], G.f, G.edim[2])))
-                            continue;
+                        if ((first | own) != 7) continue;
                         pe_ccd_candidate(x, p, bEdge, nBE, dbc, elo, ehi, vI, nlo, nhi, P, dP, e, xi, largest);
                     }
                     for (uint32_t k = pstart[cell], en = pend[cell]; k < en; ++k) {
-                        int jJ = (int)pvals[k];
+                        const int jJ = (int)(pvals[k] & kWalkId), first = (int)(pvals[k] >> kWalkIdBits);
                         if (jJ <= j) continue;
-                        if (ix != max(qlo[0], ecell(plo[jJ], G.f, G.edim[0])) || iy != max(qlo[1], ecell(plo[nPart + jJ], G.f, G.edim[1])) ||
-                            iz != max(qlo[2], ecell(plo[2 * nPart + jJ], G.f, G.edim[2])))
-                            continue;
+                        if ((first | own) != 7) continue;
                         pp_ccd_candidate(x, p, dbc, vlo, vhi, nV, vI, bNode[codimBN1 + jJ], xi, largest);
                     }
                 }
@@ -551,19 +525,6 @@ static int bits_for2(uint64_t n) {
     int b = 1;
     while (b < 64 && (1ull << b) < n) ++b;
     return b;
-}
-
-// primitive boxes in cell order: record k = box of the k-th (cell, primitive) entry, its
-// spare third word of the second half holding the primitive, so a query walks a cell's
-// candidates through contiguous memory instead of gathering one box per candidate
-__global__ void k_cell_records(const uint32_t* __restrict__ vals, long total, const int4* __restrict__ box, int4* __restrict__ rec) {
-    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= total) return;
-    const int v = (int)vals[k];
-    int4 hi = box[2l * v + 1];
-    hi.z = v;
-    rec[2 * k] = box[2l * v];
-    rec[2 * k + 1] = hi;
 }
 
 static long build_vox_cells(Ctx& c, const int* verts, int n, int nv, const int* vlo, const int* vhi, const VoxGrid& G, DevBuf<int>& plo,
@@ -672,31 +633,34 @@ double ccd_stepsize(Ctx& c, const double* x, const double* p, double alpha, doub
     // point-triangle
     uint32_t* lgCountT = c.counters.p + 18;
     uint32_t* lgCountE = c.counters.p + 19;
+    auto records = [&](long total, const DevBuf<uint32_t>& vals, const DevBuf<int>& box, DevBuf<int>& rec) {
+        rec.ensure(8 * (size_t)std::max(total, 1L));
+        if (total > 0) {
+            hipLaunchKernelGGL(k_walk_records, dim3(nblocks(total)), dim3(kBlock), 0, c.s, (const uint32_t*)vals.p, total, (const int4*)box.p,
+                               (int4*)rec.p);
+            CIPC_LAUNCH_CHECK();
+        }
+    };
+    const StepMin sm = {gmin, c.counters.p + 13, nullptr};
     const long totT = build_vox_cells(c, c.btri.p, c.nBT, 3, vlo, vhi, G, c.ccdTlo, c.ccdThi, c.ccdTbox, c.k64a, c.u32c, c.cellStart, c.cellEnd,
                                       c.lgFlagT, c.lgListT, lgCountT);
-    int4* recT = (int4*)c.ccdTrec.ensure(8 * (size_t)std::max(totT, 1L));
-    if (totT > 0) {
-        hipLaunchKernelGGL(k_cell_records, dim3(nblocks(totT)), dim3(kBlock), 0, c.s, c.u32c.p, totT, (const int4*)c.ccdTbox.p, recT);
-        CIPC_LAUNCH_CHECK();
-    }
+    records(totT, c.u32c, c.ccdTbox, c.ccdTrec);
     if (c.nBN && c.nBT) {
-        hipLaunchKernelGGL(k_ccd_pt, dim3(nblocks(c.nBN)), dim3(kBlock), 0, c.s, x, p, c.bNode.p, c.nBN, c.btri.p, c.nBT, c.dbc.p, vlo, vhi, c.nV,
-                           (const int4*)c.ccdTbox.p, G, c.cellStart.p, c.cellEnd.p, (const int4*)recT, c.lgListT.p, lgCountT, alpha, xi, gmin,
-                           c.counters.p + 13);
+        const CcdPT pt = {x, p, c.bNode.p, c.btri.p, c.nBT, c.dbc.p, vlo, vhi, c.nV, G, xi, sm, {}, {}};
+        const CellGrid cg = {{G.edim[0], G.edim[1], G.edim[2]}, c.cellStart.p, c.cellEnd.p, (const int4*)c.ccdTrec.p, (const int4*)c.ccdTbox.p,
+                             c.lgListT.p, lgCountT};
+        hipLaunchKernelGGL(k_ccd_walk<CcdPT>, dim3(walk_grid(c.nBN)), dim3(kBlock), 0, c.s, pt, c.nBN, alpha, cg);
         CIPC_LAUNCH_CHECK();
     }
     // edge-edge
     const long totE = build_vox_cells(c, c.bEdge.p, c.nBE, 2, vlo, vhi, G, c.ccdElo, c.ccdEhi, c.ccdEbox, c.k64b, c.u32d, c.ecellStart,
                                       c.ecellEnd, c.lgFlagE, c.lgListE, lgCountE);
-    int4* recE = (int4*)c.ccdErec.ensure(8 * (size_t)std::max(totE, 1L));
-    if (totE > 0) {
-        hipLaunchKernelGGL(k_cell_records, dim3(nblocks(totE)), dim3(kBlock), 0, c.s, c.u32d.p, totE, (const int4*)c.ccdEbox.p, recE);
-        CIPC_LAUNCH_CHECK();
-    }
+    records(totE, c.u32d, c.ccdEbox, c.ccdErec);
     if (c.nBE) {
-        hipLaunchKernelGGL(k_ccd_ee, dim3(nblocks(c.nBE)), dim3(kBlock), 0, c.s, x, p, c.bEdge.p, c.nBE, c.dbc.p, (const int4*)c.ccdEbox.p, G,
-                           c.ecellStart.p, c.ecellEnd.p, (const int4*)recE, c.lgFlagE.p, c.lgListE.p, lgCountE, alpha, xi, gmin,
-                           c.counters.p + 13);
+        const CcdEE ee = {x, p, c.bEdge.p, c.nBE, c.dbc.p, (const int4*)c.ccdEbox.p, c.lgFlagE.p, G, xi, sm, {}, {}};
+        const CellGrid cg = {{G.edim[0], G.edim[1], G.edim[2]}, c.ecellStart.p, c.ecellEnd.p, (const int4*)c.ccdErec.p,
+                             (const int4*)c.ccdEbox.p, c.lgListE.p, lgCountE};
+        hipLaunchKernelGGL(k_ccd_walk<CcdEE>, dim3(walk_grid(c.nBE)), dim3(kBlock), 0, c.s, ee, c.nBE, alpha, cg);
         CIPC_LAUNCH_CHECK();
     }
     // particles against rod segments and particle pairs
@@ -706,7 +670,7 @@ double ccd_stepsize(Ctx& c, const double* x, const double* p, double alpha, doub
                         c.lgFlagP, c.lgListP, lgCountP);
         hipLaunchKernelGGL(k_ccd_codim, dim3(nblocks(c.nPart)), dim3(kBlock), 0, c.s, x, p, c.bNode.p, c.nBN, c.codimBN1, c.bEdge.p, c.nBE,
                            c.nRod, c.dbc.p, vlo, vhi, c.nV, c.ccdElo.p, c.ccdEhi.p, G, c.ecellStart.p, c.ecellEnd.p, c.u32d.p,
-                           c.lgListE.p, lgCountE, c.ccdPlo.p, c.pcellStart.p, c.pcellEnd.p, c.pVals.p, c.lgFlagP.p, c.lgListP.p,
+                           c.lgListE.p, lgCountE, c.pcellStart.p, c.pcellEnd.p, c.pVals.p, c.lgFlagP.p, c.lgListP.p,
                            lgCountP, alpha, xi, gmin);
         CIPC_LAUNCH_CHECK();
     }

@@ -8,7 +8,7 @@
 // Broad phase: a uniform grid (cell = mean rest boundary-edge length, grown so the
 // grid has at most 2^23 cells) holds each triangle / edge in every cell its AABB
 // touches; entries are sorted by cell (stable radix sort) and each cell's run is
-// found through dense start/end tables.  A query visits the cells of its box and
+// found through dense start/end tables.  A query visits the cells of its box (walk.hpp) and
 // accepts a candidate only in the first cell common to both boxes, so every pair is
 // tested once; indices are clamped into the grid, which keeps the search complete
 // for points outside it.  The active set is defined by the reference's predicates
@@ -20,6 +20,7 @@
 // lexicographic int4 order of the reference's std::map.
 #include "ctx.hpp"
 #include "dev_math.hpp"
+#include "walk.hpp"
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -34,26 +35,44 @@ __device__ __forceinline__ int cell_of(double v, double lb, double inv, int dim)
 }
 
 // ------------------------------------------------------------------ grid build
-// kind 0: triangles (tri SoA), kind 1: boundary edges (bEdge SoA).  Primitives whose
-// box covers more than kLargeCells cells get count 0 and go to the large list.
-__global__ void k_prim_range(const double* __restrict__ x, const int* __restrict__ verts, int n, int nv, GridParams G,
-                             int* __restrict__ lo, uint32_t* __restrict__ count, uint8_t* __restrict__ lgFlag,
-                             int* __restrict__ lgList, uint32_t* __restrict__ lgCount) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
+// Primitives are triangles (3 vertices, SoA), boundary edges (2) or particles (1).  Each gets
+// a box record of outward-rounded floats: a test on it can only accept too much, the exact
+// predicates decide on what it accepts.  Primitives whose box covers more than kLargeCells
+// cells get count 0 and go to the large list.
+__device__ __forceinline__ float float_below(double v) {
+    const float f = (float)v;
+    return f - fabsf(f) * 2.4e-7f - 1e-30f;
+}
+__device__ __forceinline__ float float_above(double v) {
+    const float f = (float)v;
+    return f + fabsf(f) * 2.4e-7f + 1e-30f;
+}
+__device__ __forceinline__ void prim_minmax(const double* __restrict__ x, const int* __restrict__ verts, int n, int nv, int i, double* mn,
+                                            double* mx) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) { mn[d] = 1e300; mx[d] = -1e300; }
     for (int k = 0; k < nv; ++k) {
         int v = verts[(long)k * n + i];
 #pragma unroll
         for (int d = 0; d < 3; ++d) { double c = x[3 * v + d]; mn[d] = c < mn[d] ? c : mn[d]; mx[d] = c > mx[d] ? c : mx[d]; }
     }
+}
+__global__ void k_prim_range(const double* __restrict__ x, const int* __restrict__ verts, int n, int nv, GridParams G,
+                             int4* __restrict__ box, uint32_t* __restrict__ count, uint8_t* __restrict__ lgFlag,
+                             int* __restrict__ lgList, uint32_t* __restrict__ lgCount) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    double mn[3], mx[3];
+    prim_minmax(x, verts, n, nv, i, mn, mx);
     uint64_t cnt = 1;
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         int a = cell_of(mn[d], G.lb[d], G.inv, G.dim[d]), b = cell_of(mx[d], G.lb[d], G.inv, G.dim[d]);
-        lo[(long)d * n + i] = a;
         cnt *= (uint64_t)(b - a + 1);
     }
+    box[2l * i] = make_int4(__float_as_int(float_below(mn[0])), __float_as_int(float_below(mn[1])), __float_as_int(float_below(mn[2])),
+                            __float_as_int(float_above(mx[0])));
+    box[2l * i + 1] = make_int4(__float_as_int(float_above(mx[1])), __float_as_int(float_above(mx[2])), 0, 0);
     const bool large = cnt > kLargeCells;
     lgFlag[i] = large ? 1 : 0;
     count[i] = large ? 0u : (uint32_t)cnt;
@@ -64,12 +83,8 @@ __global__ void k_prim_emit(const double* __restrict__ x, const int* __restrict_
                             uint32_t* __restrict__ vals) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n || lgFlag[i]) return;
-    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-    for (int k = 0; k < nv; ++k) {
-        int v = verts[(long)k * n + i];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) { double c = x[3 * v + d]; mn[d] = c < mn[d] ? c : mn[d]; mx[d] = c > mx[d] ? c : mx[d]; }
-    }
+    double mn[3], mx[3];
+    prim_minmax(x, verts, n, nv, i, mn, mx);
     int a[3], b[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) { a[d] = cell_of(mn[d], G.lb[d], G.inv, G.dim[d]); b[d] = cell_of(mx[d], G.lb[d], G.inv, G.dim[d]); }
@@ -78,7 +93,7 @@ __global__ void k_prim_emit(const double* __restrict__ x, const int* __restrict_
         for (int iy = a[1]; iy <= b[1]; ++iy)
             for (int ix = a[0]; ix <= b[0]; ++ix) {
                 keys[o] = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
-                vals[o] = (uint32_t)i;
+                vals[o] = walk_entry(i, ix == a[0], iy == a[1], iz == a[2]);
                 ++o;
             }
 }
@@ -98,7 +113,7 @@ static int bits_for(uint64_t n) {
 
 // builds the sorted cell lists of one primitive kind (large primitives listed apart,
 // their count left in device memory at lgCount); returns number of cell entries
-static long build_cells(Ctx& c, const double* x, const int* verts, int n, int nv, const GridParams& G, DevBuf<int>& lo,
+static long build_cells(Ctx& c, const double* x, const int* verts, int n, int nv, const GridParams& G, DevBuf<int>& box, DevBuf<int>& rec,
                         DevBuf<uint64_t>& keys, DevBuf<uint32_t>& vals, DevBuf<uint32_t>& start, DevBuf<uint32_t>& end,
                         DevBuf<uint8_t>& lgFlag, DevBuf<int>& lgList, uint32_t* lgCount) {
     long nCells = (long)G.dim[0] * G.dim[1] * G.dim[2];
@@ -110,10 +125,10 @@ static long build_cells(Ctx& c, const double* x, const int* verts, int n, int nv
     lgFlag.ensure((size_t)n + 1);
     lgList.ensure((size_t)n + 1);
     if (n == 0) return 0;
-    lo.ensure((size_t)3 * n);
+    box.ensure((size_t)8 * n);
     uint32_t* cnt = c.u32a.ensure(n + 1);
     uint32_t* off = c.u32b.ensure(n + 1);
-    hipLaunchKernelGGL(k_prim_range, dim3(nblocks(n)), dim3(kBlock), 0, c.s, x, verts, n, nv, G, lo.p, cnt, lgFlag.p, lgList.p, lgCount);
+    hipLaunchKernelGGL(k_prim_range, dim3(nblocks(n)), dim3(kBlock), 0, c.s, x, verts, n, nv, G, (int4*)box.p, cnt, lgFlag.p, lgList.p, lgCount);
     CIPC_LAUNCH_CHECK();
     scan_exclusive(cnt, off, n, c.counters.p + 8, c.pw, c.s);
     CIPC_HIP(hipMemcpyAsync(c.hCnt + 8, c.counters.p + 8, sizeof(uint32_t), hipMemcpyDeviceToHost, c.s));
@@ -126,6 +141,9 @@ static long build_cells(Ctx& c, const double* x, const int* verts, int n, int nv
     CIPC_LAUNCH_CHECK();
     radix_sort_pairs(keys.p, vals.p, total, bits_for((uint64_t)nCells), c.pw, c.s);
     hipLaunchKernelGGL(k_cell_bounds, dim3(nblocks(total)), dim3(kBlock), 0, c.s, keys.p, total, start.p, end.p);
+    rec.ensure((size_t)8 * total);
+    hipLaunchKernelGGL(k_walk_records, dim3(nblocks(total)), dim3(kBlock), 0, c.s, (const uint32_t*)vals.p, total, (const int4*)box.p,
+                       (int4*)rec.p);
     CIPC_LAUNCH_CHECK();
     return total;
 }
@@ -141,21 +159,68 @@ __device__ __forceinline__ uint64_t dup_key(int c0, int c1, int c2, int nV) {
     uint64_t a = (uint64_t)(nV - 1 - (-c0 - 1)), b = (uint64_t)c1, d = (uint64_t)(c2 + 1);
     return (a * (uint64_t)nV + b) * (uint64_t)(nV + 1) + d;
 }
-// Output slots are reserved once per wavefront: the lanes emitting at this point (whatever
-// the divergence) are found by a ballot, the lowest of them adds their count to the
-// counter, and each lane takes base + its rank among them (mbcnt).  The slot order is
-// arbitrary; the set is sorted by key afterwards, so the result is deterministic.
-__device__ __forceinline__ void emit_kept(const CSOut& o, uint64_t key, int c0, int c1, int c2, int c3) {
-    const uint32_t i = wave_reserve(o.cnt);
-    if (i < o.cap) {
-        o.key[i] = key;
-        o.c4[4 * (long)i] = c0; o.c4[4 * (long)i + 1] = c1; o.c4[4 * (long)i + 2] = c2; o.c4[4 * (long)i + 3] = c3;
+// Output slots reserved once per wavefront (wave_reserve).  The slot order is arbitrary; the
+// set is sorted by key afterwards, so the result is deterministic.
+struct WaveOut {
+    CSOut o;
+    __device__ __forceinline__ void dup(uint64_t key) const {
+        const uint32_t i = wave_reserve(o.dcnt);
+        if (i < o.dcap) o.dkey[i] = key;
     }
-}
-__device__ __forceinline__ void emit_dup(const CSOut& o, uint64_t key) {
-    const uint32_t i = wave_reserve(o.dcnt);
-    if (i < o.dcap) o.dkey[i] = key;
-}
+};
+// Output gathered in LDS and written out a few hundred entries at a time: one atomic on the
+// counter per flush.  (One per wavefront and emission was most of the queries' time on a
+// state with 10^6 constraints: atomics on one address take about 15 ns each.)
+constexpr int kOutCap = 2 * kBlock;   // a batch adds up to kBlock entries to at most kBlock
+struct OutBuf {
+    uint64_t key[kOutCap], dkey[kOutCap];
+    int4 c4[kOutCap];
+    int n, nd;
+    uint32_t base, dbase;
+};
+struct BlockOut {
+    CSOut o;
+    OutBuf* b;
+    __device__ __forceinline__ void init() const {
+        if (threadIdx.x == 0) b->n = b->nd = 0;   // the walk's first barrier orders it
+    }
+    __device__ __forceinline__ void kept(uint64_t key, int c0, int c1, int c2, int c3) const {
+        const int i = atomicAdd(&b->n, 1);
+        b->key[i] = key;
+        b->c4[i] = make_int4(c0, c1, c2, c3);
+    }
+    __device__ __forceinline__ void dup(uint64_t key) const { b->dkey[atomicAdd(&b->nd, 1)] = key; }
+    // whole workgroup, after a barrier
+    __device__ __forceinline__ void flush(bool all) const {
+        const int n = b->n, nd = b->nd, lim = all ? 0 : kOutCap - kBlock;
+        const bool fk = n > lim, fd = nd > lim;
+        if (fk || fd) {
+            if (threadIdx.x == 0) {
+                if (fk) b->base = atomicAdd(o.cnt, (uint32_t)n);
+                if (fd) b->dbase = atomicAdd(o.dcnt, (uint32_t)nd);
+            }
+            __syncthreads();
+            if (fk)
+                for (int i = threadIdx.x; i < n; i += kBlock) {
+                    const uint32_t k = b->base + i;
+                    if (k >= o.cap) break;
+                    o.key[k] = b->key[i];
+                    reinterpret_cast<int4*>(o.c4)[k] = b->c4[i];
+                }
+            if (fd)
+                for (int i = threadIdx.x; i < nd; i += kBlock) {
+                    const uint32_t k = b->dbase + i;
+                    if (k < o.dcap) o.dkey[k] = b->dkey[i];
+                }
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                if (fk) b->n = 0;
+                if (fd) b->nd = 0;
+            }
+        }
+        __syncthreads();   // the counts are read by all before the next batch adds to them
+    }
+};
 
 #pragma clang fp contract(off)
 __device__ __forceinline__ bool pt_cd_broadphase(d3 p, d3 t0, d3 t1, d3 t2, double dist) {
@@ -176,7 +241,8 @@ __device__ __forceinline__ bool ee_cd_broadphase(d3 a0, d3 a1, d3 b0, d3 b1, dou
 }
 
 // point vI (boundary-node slot svI) against triangle t: IPC.h:57-140
-__device__ __forceinline__ void pt_candidate(const CSOut& o, const double* __restrict__ x, const int* __restrict__ tri, int nT,
+template <class O>
+__device__ __forceinline__ void pt_candidate(const O& o, const double* __restrict__ x, const int* __restrict__ tri, int nT,
                                              const uint8_t* __restrict__ dbc, int svI, int vI, d3 p, int t, double dHat,
                                              double dHat2, int nV) {
     int a = tri[t], b = tri[nT + t], cc = tri[2 * nT + t];
@@ -197,21 +263,22 @@ __device__ __forceinline__ void pt_candidate(const CSOut& o, const double* __res
         default: d = dist2_pt(p, t0, t1, t2); break;
     }
     if (!(d < dHat2)) return;
-    if (ty == 6) emit_kept(o, (uint64_t)svI * (uint64_t)nT + (uint64_t)t, -vI - 1, a, b, cc);
-    else emit_dup(o, dup_key(-vI - 1, c1, c2, nV));
+    if (ty == 6) o.kept((uint64_t)svI * (uint64_t)nT + (uint64_t)t, -vI - 1, a, b, cc);
+    else o.dup(dup_key(-vI - 1, c1, c2, nV));
 }
 
 // edge pair eA < eB: IPC.h:142-330 (edge A supplies a0/a1 of the encoding)
-__device__ __forceinline__ void ee_candidate(const CSOut& o, const double* __restrict__ x, const double* __restrict__ X0,
+template <class O>
+__device__ __forceinline__ void ee_candidate(const O& o, const double* __restrict__ x, const double* __restrict__ X0,
                                              const int* __restrict__ bEdge, int nBE, const uint8_t* __restrict__ dbc, int eA, int a0,
-                                             int a1, d3 ea0, d3 ea1, d3 ra0, d3 ra1, int eB, double dHat, double dHat2, int nV) {
+                                             int a1, d3 ea0, d3 ea1, int eB, double dHat, double dHat2, int nV) {
     int b0 = bEdge[eB], b1 = bEdge[nBE + eB];
     if (a0 == b0 || a0 == b1 || a1 == b0 || a1 == b1) return;
     if (dbc[a0] && dbc[a1] && dbc[b0] && dbc[b1]) return;
     d3 eb0 = ld3(x, b0), eb1 = ld3(x, b1);
     if (!ee_cd_broadphase(ea0, ea1, eb0, eb1, dHat)) return;
     double crossN = ee_cross_norm2(ea0, ea1, eb0, eb1);
-    double eps = ee_mollifier_threshold(ra0, ra1, ld3(X0, b0), ld3(X0, b1));
+    double eps = ee_mollifier_threshold(ld3(X0, a0), ld3(X0, a1), ld3(X0, b0), ld3(X0, b1));
     bool moll = crossN < eps;
     double d;
     int c[4];
@@ -236,87 +303,101 @@ __device__ __forceinline__ void ee_candidate(const CSOut& o, const double* __res
             if (moll) { c[0] = a0; c[1] = a1; c[2] = -b0 - 1; c[3] = b1; } else { c[0] = a0; c[1] = a1; c[2] = b0; c[3] = b1; } break;
     }
     if (!(d < dHat2)) return;
-    if (c[0] >= 0) emit_kept(o, (uint64_t)eA * (uint64_t)nBE + (uint64_t)eB, c[0], c[1], c[2], c[3]);
-    else emit_dup(o, dup_key(c[0], c[1], c[2], nV));
+    if (c[0] >= 0) o.kept((uint64_t)eA * (uint64_t)nBE + (uint64_t)eB, c[0], c[1], c[2], c[3]);
+    else o.dup(dup_key(c[0], c[1], c[2], nV));
 }
 
-__global__ void k_query_pt(const double* __restrict__ x, const int* __restrict__ bNode, int nBN, const int* __restrict__ tri,
-                           int nT, const uint8_t* __restrict__ dbc, GridParams G, const uint32_t* __restrict__ start,
-                           const uint32_t* __restrict__ end, const uint32_t* __restrict__ vals, const int* __restrict__ triLo,
-                           const int* __restrict__ lgList, const uint32_t* __restrict__ lgCount, double dHat, double dHat2,
-                           int nV, CSOut o) {
-    int svI = xcd_item();
-    if (svI >= nBN) return;
-    int vI = bNode[svI];
-    d3 p = ld3(x, vI);
-    int qlo[3], qhi[3];
-    double pc[3] = {p.x, p.y, p.z};
+// float box of the item grown by dHat against a record's box
+struct QueryBox {
+    float lo[3], hi[3];
+    __device__ __forceinline__ void set(const double* mn, const double* mx, double dHat) {
 #pragma unroll
-    for (int d = 0; d < 3; ++d) { qlo[d] = cell_of(pc[d] - dHat, G.lb[d], G.inv, G.dim[d]); qhi[d] = cell_of(pc[d] + dHat, G.lb[d], G.inv, G.dim[d]); }
-    for (int iz = qlo[2]; iz <= qhi[2]; ++iz)
-        for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
-            for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
-                uint64_t cell = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
-                uint32_t s = start[cell], e = end[cell];
-                for (uint32_t k = s; k < e; ++k) {
-                    int t = (int)vals[k];
-                    int l0 = triLo[t], l1 = triLo[nT + t], l2 = triLo[2 * nT + t];
-                    if (ix != max(qlo[0], l0) || iy != max(qlo[1], l1) || iz != max(qlo[2], l2)) continue;
-                    pt_candidate(o, x, tri, nT, dbc, svI, vI, p, t, dHat, dHat2, nV);
-                }
-            }
-    const uint32_t nl = *lgCount;
-    for (uint32_t k = 0; k < nl; ++k) pt_candidate(o, x, tri, nT, dbc, svI, vI, p, lgList[k], dHat, dHat2, nV);
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = float_below(mn[d] - dHat);
+            hi[d] = float_above(mx[d] + dHat);
+        }
+    }
+    __device__ __forceinline__ bool meets(const int4& a, const int4& b) const {
+        return !(__int_as_float(a.x) > hi[0] || __int_as_float(a.w) < lo[0] || __int_as_float(a.y) > hi[1] || __int_as_float(b.x) < lo[1] ||
+                 __int_as_float(a.z) > hi[2] || __int_as_float(b.y) < lo[2]);
+    }
+};
+struct QueryPT {
+    const double* __restrict__ x;
+    const int* __restrict__ bNode;
+    const int* __restrict__ tri;
+    int nT;
+    const uint8_t* __restrict__ dbc;
+    GridParams G;
+    double dHat, dHat2;
+    int nV;
+    BlockOut o;
+    QueryBox q;
+    __device__ __forceinline__ void flush(bool all) const { o.flush(all); }
+    __device__ __forceinline__ bool begin(int slot, int* qlo, int* qhi) {
+        const d3 p = ld3(x, bNode[slot]);
+        const double pc[3] = {p.x, p.y, p.z};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            qlo[d] = cell_of(pc[d] - dHat, G.lb[d], G.inv, G.dim[d]);
+            qhi[d] = cell_of(pc[d] + dHat, G.lb[d], G.inv, G.dim[d]);
+        }
+        q.set(pc, pc, dHat);
+        return true;
+    }
+    __device__ __forceinline__ bool accept(int, int, const int4& a, const int4& b, bool) const { return q.meets(a, b); }
+    __device__ __forceinline__ void exact(int slot, int t) const {
+        const int vI = bNode[slot];
+        pt_candidate(o, x, tri, nT, dbc, slot, vI, ld3(x, vI), t, dHat, dHat2, nV);
+    }
+};
+__global__ __launch_bounds__(kBlock) void k_query_pt(QueryPT T, int nBN, CellGrid G) {
+    __shared__ OutBuf buf;
+    T.o.b = &buf;
+    T.o.init();
+    walk_pairs(T, nBN, G);
 }
 
 // Every unordered edge pair is tested once: a grid-listed edge finds grid-listed
 // edges of larger index in the first common cell and every large edge from the
 // list; a large edge only tests large edges of larger index.
-__global__ void k_query_ee(const double* __restrict__ x, const double* __restrict__ X0, const int* __restrict__ bEdge, int nBE,
-                           const uint8_t* __restrict__ dbc, GridParams G, const uint32_t* __restrict__ start,
-                           const uint32_t* __restrict__ end, const uint32_t* __restrict__ vals, const int* __restrict__ edgeLo,
-                           const uint8_t* __restrict__ lgFlag, const int* __restrict__ lgList, const uint32_t* __restrict__ lgCount,
-                           double dHat, double dHat2, int nV, CSOut o) {
-    int eI = blockIdx.x * blockDim.x + threadIdx.x;
-    if (eI >= nBE) return;
-    int a0 = bEdge[eI], a1 = bEdge[nBE + eI];
-    d3 ea0 = ld3(x, a0), ea1 = ld3(x, a1);
-    d3 ra0 = ld3(X0, a0), ra1 = ld3(X0, a1);
-    const uint32_t nl = *lgCount;
-    if (lgFlag[eI]) {
-        for (uint32_t k = 0; k < nl; ++k) {
-            int eJ = lgList[k];
-            if (eJ > eI) ee_candidate(o, x, X0, bEdge, nBE, dbc, eI, a0, a1, ea0, ea1, ra0, ra1, eJ, dHat, dHat2, nV);
-        }
-        return;
-    }
-    int qlo[3], qhi[3];
-    double mn[3] = {dmin(ea0.x, ea1.x), dmin(ea0.y, ea1.y), dmin(ea0.z, ea1.z)};
-    double mx[3] = {dmax(ea0.x, ea1.x), dmax(ea0.y, ea1.y), dmax(ea0.z, ea1.z)};
+struct QueryEE {
+    const double* __restrict__ x;
+    const double* __restrict__ X0;
+    const int* __restrict__ bEdge;
+    int nBE;
+    const uint8_t* __restrict__ dbc;
+    const uint8_t* __restrict__ lgFlag;
+    GridParams G;
+    double dHat, dHat2;
+    int nV;
+    BlockOut o;
+    QueryBox q;
+    __device__ __forceinline__ void flush(bool all) const { o.flush(all); }
+    __device__ __forceinline__ bool begin(int e, int* qlo, int* qhi) {
+        const d3 a = ld3(x, bEdge[e]), b = ld3(x, bEdge[nBE + e]);
+        const double mn[3] = {dmin(a.x, b.x), dmin(a.y, b.y), dmin(a.z, b.z)}, mx[3] = {dmax(a.x, b.x), dmax(a.y, b.y), dmax(a.z, b.z)};
 #pragma unroll
-    for (int d = 0; d < 3; ++d) { qlo[d] = cell_of(mn[d] - dHat, G.lb[d], G.inv, G.dim[d]); qhi[d] = cell_of(mx[d] + dHat, G.lb[d], G.inv, G.dim[d]); }
-    for (int iz = qlo[2]; iz <= qhi[2]; ++iz)
-        for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
-            for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
-                uint64_t cell = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
-                uint32_t s = start[cell], e = end[cell];
-                for (uint32_t k = s; k < e; ++k) {
-                    int eJ = (int)vals[k];
-                    if (eJ <= eI) continue;
-                    int l0 = edgeLo[eJ], l1 = edgeLo[nBE + eJ], l2 = edgeLo[2 * nBE + eJ];
-                    if (ix != max(qlo[0], l0) || iy != max(qlo[1], l1) || iz != max(qlo[2], l2)) continue;
-                    ee_candidate(o, x, X0, bEdge, nBE, dbc, eI, a0, a1, ea0, ea1, ra0, ra1, eJ, dHat, dHat2, nV);
-                }
-            }
-    for (uint32_t k = 0; k < nl; ++k) {
-        int eJ = lgList[k];
-        if (eJ > eI) {
-            ee_candidate(o, x, X0, bEdge, nBE, dbc, eI, a0, a1, ea0, ea1, ra0, ra1, eJ, dHat, dHat2, nV);
-        } else {
-            int b0 = bEdge[eJ], b1 = bEdge[nBE + eJ];
-            ee_candidate(o, x, X0, bEdge, nBE, dbc, eJ, b0, b1, ld3(x, b0), ld3(x, b1), ld3(X0, b0), ld3(X0, b1), eI, dHat, dHat2, nV);
+        for (int d = 0; d < 3; ++d) {
+            qlo[d] = cell_of(mn[d] - dHat, G.lb[d], G.inv, G.dim[d]);
+            qhi[d] = cell_of(mx[d] + dHat, G.lb[d], G.inv, G.dim[d]);
         }
+        q.set(mn, mx, dHat);
+        return !lgFlag[e];
     }
+    __device__ __forceinline__ bool accept(int e, int other, const int4& a, const int4& b, bool anyOrder) const {
+        return (anyOrder || other > e) && q.meets(a, b);
+    }
+    __device__ __forceinline__ void exact(int e, int other) const {
+        const int eA = min(e, other), eB = max(e, other), a0 = bEdge[eA], a1 = bEdge[nBE + eA];
+        ee_candidate(o, x, X0, bEdge, nBE, dbc, eA, a0, a1, ld3(x, a0), ld3(x, a1), eB, dHat, dHat2, nV);
+    }
+};
+__global__ __launch_bounds__(kBlock) void k_query_ee(QueryEE T, CellGrid G) {
+    __shared__ OutBuf buf;
+    T.o.b = &buf;
+    T.o.init();
+    walk_pairs(T, T.nBE, G);
 }
 // rod nodes and particles (boundary-node slots >= codimBN0) against rod segments (the
 // last nRod boundary edges), IPC.h:271-317; particles (slots >= codimBN1) against the
@@ -328,7 +409,8 @@ __device__ __forceinline__ bool pe_cd_broadphase(d3 p, d3 e0, d3 e1, double dist
     if (p.z - dmax(e0.z, e1.z) > dist || dmin(e0.z, e1.z) - p.z > dist) return false;
     return true;
 }
-__device__ __forceinline__ void pe_codim_candidate(const CSOut& o, const double* __restrict__ x, const int* __restrict__ bEdge, int nBE,
+template <class O>
+__device__ __forceinline__ void pe_codim_candidate(const O& o, const double* __restrict__ x, const int* __restrict__ bEdge, int nBE,
                                                    const uint8_t* __restrict__ dbc, int vI, d3 p, int eJ, double dHat, double dHat2,
                                                    int nV) {
     int a = bEdge[eJ], b = bEdge[nBE + eJ];
@@ -343,14 +425,15 @@ __device__ __forceinline__ void pe_codim_candidate(const CSOut& o, const double*
         case 1: d = dist2_pp(p, e1); c1 = b; break;
         default: d = dist2_pe(p, e0, e1); c1 = a; c2 = b; break;
     }
-    if (d < dHat2) emit_dup(o, dup_key(-vI - 1, c1, c2, nV));
+    if (d < dHat2) o.dup(dup_key(-vI - 1, c1, c2, nV));
 }
 __global__ void k_query_codim(const double* __restrict__ x, const int* __restrict__ bNode, int nBN, int codimBN0, int codimBN1,
                               const int* __restrict__ bEdge, int nBE, int nRod, const uint8_t* __restrict__ dbc, GridParams G,
                               const uint32_t* __restrict__ estart, const uint32_t* __restrict__ eend, const uint32_t* __restrict__ evals,
-                              const int* __restrict__ edgeLo, const int* __restrict__ lgListE, const uint32_t* __restrict__ lgCountE,
+                              const int* __restrict__ lgListE, const uint32_t* __restrict__ lgCountE,
                               const uint32_t* __restrict__ pstart, const uint32_t* __restrict__ pend, const uint32_t* __restrict__ pvals,
-                              double dHat, double dHat2, int nV, CSOut o) {
+                              double dHat, double dHat2, int nV, CSOut out) {
+    const WaveOut o{out};
     int s = codimBN0 + blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= nBN) return;
     int vI = bNode[s];
@@ -365,9 +448,9 @@ __global__ void k_query_codim(const double* __restrict__ x, const int* __restric
             for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
                 uint64_t cell = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
                 for (uint32_t k = estart[cell], e = eend[cell]; k < e; ++k) {
-                    int eJ = (int)evals[k];
+                    const int eJ = (int)(evals[k] & kWalkId), first = (int)(evals[k] >> kWalkIdBits);
                     if (eJ < firstRod) continue;
-                    if (ix != max(qlo[0], edgeLo[eJ]) || iy != max(qlo[1], edgeLo[nBE + eJ]) || iz != max(qlo[2], edgeLo[2 * nBE + eJ])) continue;
+                    if ((first | (ix == qlo[0] ? 1 : 0) | (iy == qlo[1] ? 2 : 0) | (iz == qlo[2] ? 4 : 0)) != 7) continue;
                     pe_codim_candidate(o, x, bEdge, nBE, dbc, vI, p, eJ, dHat, dHat2, nV);
                 }
             }
@@ -383,12 +466,12 @@ __global__ void k_query_codim(const double* __restrict__ x, const int* __restric
             for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
                 uint64_t cell = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
                 for (uint32_t k = pstart[cell], e = pend[cell]; k < e; ++k) {
-                    int sJ = codimBN1 + (int)pvals[k];
+                    int sJ = codimBN1 + (int)(pvals[k] & kWalkId);
                     if (sJ <= s) continue;
                     int vJ = bNode[sJ];
                     if (dbc[vI] && dbc[vJ]) continue;
                     double d = dist2_pp(p, ld3(x, vJ));
-                    if (d < dHat2) emit_dup(o, dup_key(-vI - 1, vJ, -1, nV));
+                    if (d < dHat2) o.dup(dup_key(-vI - 1, vJ, -1, nV));
                 }
             }
 }
@@ -451,10 +534,10 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
 
     uint32_t* lgCountT = c.counters.p + 16;
     uint32_t* lgCountE = c.counters.p + 17;
-    build_cells(c, x, c.btri.p, c.nBT, 3, G, c.triLo, c.k64a, c.u32c, c.cellStart, c.cellEnd, c.lgFlagT, c.lgListT, lgCountT);
-    build_cells(c, x, c.bEdge.p, c.nBE, 2, G, c.edgeLo, c.k64b, c.u32d, c.ecellStart, c.ecellEnd, c.lgFlagE, c.lgListE, lgCountE);
+    build_cells(c, x, c.btri.p, c.nBT, 3, G, c.csBoxT, c.csRecT, c.k64a, c.u32c, c.cellStart, c.cellEnd, c.lgFlagT, c.lgListT, lgCountT);
+    build_cells(c, x, c.bEdge.p, c.nBE, 2, G, c.csBoxE, c.csRecE, c.k64b, c.u32d, c.ecellStart, c.ecellEnd, c.lgFlagE, c.lgListE, lgCountE);
     if (c.nPart)
-        build_cells(c, x, c.partSlot.p, c.nPart, 1, G, c.pLo, c.pKeys, c.pVals, c.pcellStart, c.pcellEnd, c.lgFlagP, c.lgListP,
+        build_cells(c, x, c.partSlot.p, c.nPart, 1, G, c.csBoxP, c.csRecP, c.pKeys, c.pVals, c.pcellStart, c.pcellEnd, c.lgFlagP, c.lgListP,
                     c.counters.p + 20);
 
     // narrow phase with capacity retry
@@ -469,18 +552,21 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
         o.dcnt = c.counters.p + 1;
         CIPC_HIP(hipMemsetAsync(c.counters.p, 0, 4 * sizeof(uint32_t), c.s));
         // point-triangle kept entries fill [0, cap), edge-edge kept entries [cap, 2 cap)
-        hipLaunchKernelGGL(k_query_pt, dim3(xcd_grid(c.nBN)), dim3(kBlock), 0, c.s, x, c.bNode.p, c.nBN, c.btri.p, c.nBT, c.dbc.p, G,
-                           c.cellStart.p, c.cellEnd.p, c.u32c.p, c.triLo.p, c.lgListT.p, lgCountT, dHat, dHat2, c.nV, o);
+        const CellGrid GT = {{G.dim[0], G.dim[1], G.dim[2]}, c.cellStart.p, c.cellEnd.p, (const int4*)c.csRecT.p, (const int4*)c.csBoxT.p,
+                             c.lgListT.p, lgCountT};
+        const CellGrid GE = {{G.dim[0], G.dim[1], G.dim[2]}, c.ecellStart.p, c.ecellEnd.p, (const int4*)c.csRecE.p, (const int4*)c.csBoxE.p,
+                             c.lgListE.p, lgCountE};
+        const QueryPT pt = {x, c.bNode.p, c.btri.p, c.nBT, c.dbc.p, G, dHat, dHat2, c.nV, {o, nullptr}, {}};
+        hipLaunchKernelGGL(k_query_pt, dim3(walk_grid(c.nBN)), dim3(kBlock), 0, c.s, pt, c.nBN, GT);
         CIPC_LAUNCH_CHECK();
         CSOut oEE = o;
         oEE.key = o.key + cap; oEE.c4 = o.c4 + 4 * (size_t)cap; oEE.cnt = c.counters.p + 2;
-        hipLaunchKernelGGL(k_query_ee, dim3(nblocks(c.nBE)), dim3(kBlock), 0, c.s, x, c.X0.p, c.bEdge.p, c.nBE, c.dbc.p, G,
-                           c.ecellStart.p, c.ecellEnd.p, c.u32d.p, c.edgeLo.p, c.lgFlagE.p, c.lgListE.p, lgCountE, dHat, dHat2, c.nV,
-                           oEE);
+        const QueryEE ee = {x, c.X0.p, c.bEdge.p, c.nBE, c.dbc.p, c.lgFlagE.p, G, dHat, dHat2, c.nV, {oEE, nullptr}, {}};
+        hipLaunchKernelGGL(k_query_ee, dim3(walk_grid(c.nBE)), dim3(kBlock), 0, c.s, ee, GE);
         CIPC_LAUNCH_CHECK();
         if (c.nBN > c.codimBN0) {
             hipLaunchKernelGGL(k_query_codim, dim3(nblocks(c.nBN - c.codimBN0)), dim3(kBlock), 0, c.s, x, c.bNode.p, c.nBN, c.codimBN0,
-                               c.codimBN1, c.bEdge.p, c.nBE, c.nRod, c.dbc.p, G, c.ecellStart.p, c.ecellEnd.p, c.u32d.p, c.edgeLo.p,
+                               c.codimBN1, c.bEdge.p, c.nBE, c.nRod, c.dbc.p, G, c.ecellStart.p, c.ecellEnd.p, c.u32d.p,
                                c.lgListE.p, lgCountE, c.nPart ? c.pcellStart.p : c.ecellStart.p, c.nPart ? c.pcellEnd.p : c.ecellEnd.p,
                                c.nPart ? c.pVals.p : c.u32d.p, dHat, dHat2, c.nV, o);
             CIPC_LAUNCH_CHECK();

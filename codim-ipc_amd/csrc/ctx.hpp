@@ -152,7 +152,6 @@ struct Ctx {
     std::vector<int> hTet, hBTri;
     DevBuf<int> tetIdx, btri;
     DevBuf<double> tetIB, tetVol;
-    DevBuf<int> pLo;
     DevBuf<uint64_t> pKeys;
     DevBuf<uint32_t> pVals, pcellStart, pcellEnd;
     DevBuf<uint8_t> lgFlagP;
@@ -188,7 +187,8 @@ struct Ctx {
     DevBuf<uint64_t> csKey, csDKey;
     DevBuf<int> csC4;
     DevBuf<uint32_t> csPos, csIdx, csHead;
-    DevBuf<int> triLo, edgeLo;
+    DevBuf<int> csBoxT, csBoxE, csBoxP;   // constraint-set grid: float boxes per primitive (32-byte records)
+    DevBuf<int> csRecT, csRecE, csRecP;   // and in cell order
     DevBuf<int> ccdTlo, ccdThi, ccdElo, ccdEhi;
     // primitives spanning more than kLargeCells grid cells are kept out of the cell
     // lists and tested by every query directly (flag per primitive + compact list)
