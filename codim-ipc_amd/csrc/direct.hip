@@ -9,6 +9,7 @@
 // substitution.  Dense, so limited to kDirectMaxDof unknowns (4.5 GiB of FP64 matrix); it
 // is the fallback of the PCG solves for such scenes and a selectable solver.
 #include "ctx.hpp"
+#include <algorithm>
 #include <cmath>
 
 namespace cipc {
@@ -40,14 +41,74 @@ __global__ void k_dense_scatter(const int* __restrict__ rowOf, const int* __rest
         }
 }
 
+__device__ __forceinline__ double lane_read(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane), __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// s / d from the correctly rounded reciprocal r of d: one residual step
+__device__ __forceinline__ double div_by(double s, double d, double r) {
+    const double q = s * r;
+    return fma(fma(-q, d, s), r, q);
+}
+
+// sqrt(d) and 1 / sqrt(d) together by Goldschmidt's iteration from the hardware's reciprocal
+// square root, with a residual step on the root: a third of the dependent operations of a
+// square root followed by a division, which is the tile factor's serial chain.  Pivots near
+// the ends of the exponent range take the library functions.
+__device__ __forceinline__ void sqrt_and_inverse(double d, double& root, double& inv) {
+    if (d > 1e-280 && d < 1e280) {
+        const double y = __builtin_amdgcn_rsq(d);
+        double g = d * y, h = 0.5 * y;
+        double e = fma(-g, h, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        e = fma(-g, h, 0.5);
+        g = fma(g, e, g);
+        h = fma(h, e, h);
+        root = fma(fma(-g, g, d), h, g);
+        inv = 2 * h;
+    } else {
+        root = sqrt(d);
+        inv = 1.0 / root;
+    }
+}
+
+// A 64 x 64 tile (row-major, leading dimension ld) by 256 threads: 16 entries each as eight
+// 16-byte loads, all in flight before the first is stored (a load-store loop waits for each
+// in turn, which took longer than the products)
+typedef double dt_v2 __attribute__((ext_vector_type(2)));
+struct TileRegs {
+    dt_v2 v[8];
+    __device__ __forceinline__ void load(const double* __restrict__ a, long ld) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = *reinterpret_cast<const dt_v2*>(a + row(q) * ld + col());
+    }
+    __device__ __forceinline__ static int row(int q) { return 8 * q + (int)(threadIdx.x >> 5); }
+    __device__ __forceinline__ static int col() { return 2 * (int)(threadIdx.x & 31); }
+    template <int LD>
+    __device__ __forceinline__ void put(double (*T)[LD]) const {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            T[row(q)][col()] = v[q].x;
+            T[row(q)][col() + 1] = v[q].y;
+        }
+    }
+    template <int LD>
+    __device__ __forceinline__ void put_transposed(double (*T)[LD]) const {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            T[col()][row(q)] = v[q].x;
+            T[col() + 1][row(q)] = v[q].y;
+        }
+    }
+};
+
 // Cholesky of diagonal tile k (lower, in place) by four waves: wave h keeps columns
-// [16h, 16h+16) of every row in registers, so the trailing update of a column is 16
-// register FMAs per lane against a broadcast copy of the column in LDS.  Per column two
-// barriers: after the column's entries are published, and after its multipliers are
-// (both LDS buffers alternate between columns, so no third is needed).  The entry (i, j)
-// of the column being eliminated is published by the wave that holds it (picked from
-// registers by a select tree on the bits of j); every lane derives the pivot and its
-// row's multiplier from it with the same operations, so all lanes hold the same bits.
+// [16h, 16h+16) of every row (lane = row) in registers.  Panel by panel: wave p eliminates
+// its own 16 columns without a barrier (pivot and multipliers cross lanes by readlane),
+// publishes them in LDS, and after one barrier the later waves apply all 16 columns to
+// theirs.  The serial chain is the 64 square roots and divisions; two barriers per column
+// (as with the columns published one by one) had cost more than the arithmetic.
+// Measured (us per tile without / with the inverse): 40 / 58 -> 26 / 41.
 // A non-positive pivot sets *bad and continues with pivot 1 so that the factorisation
 // stays finite.  With diag0, a pivot at or below tau x diag0 (the unknown's diagonal
 // before elimination: a mode the matrix does not see) is dropped instead: a pivot at the
@@ -59,69 +120,69 @@ __global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict_
                                                              const double* __restrict__ diag0, int* __restrict__ dropped, double tau,
                                                              double* __restrict__ inv) {
     __shared__ double T[kDT][kDT + 1];
-    __shared__ double colj[2][kDT];
-    __shared__ double cur[2][kDT];
-    __shared__ double dg0[kDT];
     const int tid = threadIdx.x, i = tid & 63, h = tid >> 6;
     const long o = (long)k * kDT;
-    if (h == 0) dg0[i] = diag0 ? diag0[o + i] : 0.0;
-    for (int r = h; r < kDT; r += 4) T[r][i] = a[(o + r) * ld + o + i];
+    const double dg0 = diag0 ? diag0[o + i] : 0.0;
+    TileRegs tr;
+    tr.load(a + o * ld + o, ld);
+    tr.put(T);
     __syncthreads();
     double row[16];
 #pragma unroll
     for (int q = 0; q < 16; ++q) row[q] = T[i][16 * h + q];
-    for (int j = 0; j < kDT; ++j) {
-        const int b = j & 1;
-        if (h == (j >> 4)) {
-            double t4[4];
-            const bool s8 = j & 8, s4 = j & 4;
+    for (int p = 0; p < 4; ++p) {
+        if (h == p) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) t4[q] = s8 ? (s4 ? row[q + 12] : row[q + 8]) : (s4 ? row[q + 4] : row[q]);
-            const bool s2 = j & 2, s1 = j & 1;
-            cur[b][i] = s2 ? (s1 ? t4[3] : t4[2]) : (s1 ? t4[1] : t4[0]);
-        }
-        __syncthreads();
-        double d = cur[b][j];
-        const double rij = cur[b][i];
-        int dr = 0;
-        bool neg = false;
-        if (diag0) {
-            const double d0 = dg0[j];
-            if (!(d > tau * d0)) {
-                dr = 1;
-                d = d0 > 0 ? d0 : 1.0;
+            for (int j = 0; j < 16; ++j) {
+                const int J = 16 * p + j;
+                double d = lane_read(row[j], J);
+                int dr = 0;
+                bool neg = false;
+                if (diag0) {
+                    const double d0 = lane_read(dg0, J);
+                    if (!(d > tau * d0)) {
+                        dr = 1;
+                        d = d0 > 0 ? d0 : 1.0;
+                    }
+                } else if (!(d > 0)) {
+                    neg = true;
+                    d = 1.0;
+                }
+                if (i == J) {
+                    if (diag0) dropped[o + J] = dr;
+                    else if (neg) atomicOr(bad, 1);
+                }
+                double pv, ri;
+                sqrt_and_inverse(d, pv, ri);
+                const double lm = i > J && !dr ? div_by(row[j], pv, ri) : 0.0;   // multiplier of this row
+                row[j] = i == J ? pv : lm;
+#pragma unroll
+                for (int q = j + 1; q < 16; ++q) row[q] = fma(-lm, lane_read(lm, 16 * p + q), row[q]);
             }
-        } else if (!(d > 0)) {
-            neg = true;
-            d = 1.0;
-        }
-        if (tid == j) {
-            if (diag0) dropped[o + j] = dr;
-            else if (neg) atomicOr(bad, 1);
-        }
-        const double pv = sqrt(d);
-        double lij;
-        if (i == j) lij = pv;
-        else if (i > j) lij = dr ? 0.0 : rij / pv;
-        else lij = 0.0;
-        if (h == 0) {
-            T[i][j] = lij;
-            colj[b][i] = i > j ? lij : 0.0;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) T[i][16 * p + j] = row[j];
         }
         __syncthreads();
-        if (i > j) {
+        // (entries above the diagonal pick up values that nothing reads)
+        if (h > p)
+#pragma unroll 4
+            for (int j = 0; j < 16; ++j) {
+                const double lij = T[i][16 * p + j];
 #pragma unroll
-            for (int q = 0; q < 16; ++q) row[q] = fma(-lij, colj[b][16 * h + q], row[q]);
-        }
+                for (int q = 0; q < 16; ++q) row[q] = fma(-lij, T[16 * h + q][16 * p + j], row[q]);
+            }
     }
-    __syncthreads();
-    for (int r = h; r < kDT; r += 4) a[(o + r) * ld + o + i] = T[r][i];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) a[(o + 4 * q + h) * ld + o + i] = T[4 * q + h][i];
     if (inv) {
         // column i of the inverse, rows [16h, 16h+16) in wave h: X[r] = (delta_ri -
         // sum_{m<r} L[r][m] X[m]) / L[r][r] with the sum taken in m order, quarter by
         // quarter: wave s finishes its rows, then the later waves add their terms
         // from them
         __shared__ double X[kDT][kDT + 1];
+        __shared__ double rd[kDT];
+        if (h == 0) rd[i] = 1.0 / T[i][i];
+        __syncthreads();
         double sacc[16];
 #pragma unroll
         for (int q = 0; q < 16; ++q) sacc[q] = 16 * h + q == i ? 1.0 : 0.0;
@@ -133,7 +194,7 @@ __global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict_
                     const int r = 16 * st + q;
 #pragma unroll
                     for (int m = 0; m < q; ++m) sacc[q] = fma(-T[r][16 * st + m], xq[m], sacc[q]);
-                    xq[q] = r < i ? 0.0 : sacc[q] / T[r][r];
+                    xq[q] = r < i ? 0.0 : div_by(sacc[q], T[r][r], rd[r]);
                     X[r][i] = xq[q];
                 }
             }
@@ -148,89 +209,132 @@ __global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict_
             }
         }
         double* dst = inv + (long)k * kDT * kDT;
-        for (int r = h; r < kDT; r += 4) dst[r * kDT + i] = X[r][i];
+#pragma unroll
+        for (int q = 0; q < 16; ++q) dst[(4 * q + h) * kDT + i] = X[4 * q + h][i];
     }
 }
 
 // panel: tiles (i, k), i > k, become A_ik L_kk^-T (each row solved forward against L_kk);
-// columns of dropped pivots are zero
+// columns of dropped pivots are zero.  Four lanes per row hold every fourth column in
+// registers; a finished entry crosses to its row's lanes by a quad permutation, and the
+// sums run in column order as in one thread per row, whose 2,016 dependent products took
+// 46 us per launch (11 now, at 3,198 unknowns).
+template <int SUB>
+__device__ __forceinline__ double quad_get(double v) {
+    return dpp_move<SUB * 0x55>(v);
+}
 __global__ __launch_bounds__(kDirectBlock) void k_trsm_tiles(double* __restrict__ a, long ld, int k, const int* __restrict__ dropped) {
     __shared__ double L[kDT][kDT + 1];
     __shared__ double X[kDT][kDT + 1];
-    const int i = k + 1 + blockIdx.x;
+    __shared__ double rd[kDT];
+    const int i = k + 1 + blockIdx.x, tid = threadIdx.x;
     const long ok = (long)k * kDT, oi = (long)i * kDT;
-    for (int e = threadIdx.x; e < kDT * kDT; e += kDirectBlock) {
-        const int r = e / kDT, c = e % kDT;
-        L[r][c] = a[(ok + r) * ld + ok + c];
-        X[r][c] = a[(oi + r) * ld + ok + c];
+    {
+        TileRegs tl, tx;
+        tl.load(a + ok * ld + ok, ld);
+        tx.load(a + oi * ld + ok, ld);
+        tl.put(L);
+        tx.put(X);
     }
     __syncthreads();
-    // one thread per row (the running sums of a row are sequential)
-    if (threadIdx.x < kDT) {
-        const int r = threadIdx.x;
-        for (int c = 0; c < kDT; ++c) {
-            double s = X[r][c];
-            for (int m = 0; m < c; ++m) s -= X[r][m] * L[c][m];
-            X[r][c] = (dropped && dropped[ok + c]) ? 0.0 : s / L[c][c];
-        }
-    }
+    if (tid < kDT) rd[tid] = 1.0 / L[tid][tid];
     __syncthreads();
-    for (int e = threadIdx.x; e < kDT * kDT; e += kDirectBlock) {
-        const int r = e / kDT, c = e % kDT;
-        a[(oi + r) * ld + ok + c] = X[r][c];
+    const int r = tid >> 2, sub = tid & 3;
+    double xr[16];   // columns 4 q + sub
+#pragma unroll
+    for (int q = 0; q < 16; ++q) xr[q] = X[r][4 * q + sub];
+#pragma unroll
+    for (int c = 0; c < kDT; ++c) {
+        const double mine = xr[c >> 2];
+        const double sc = (c & 3) == 0 ? quad_get<0>(mine) : (c & 3) == 1 ? quad_get<1>(mine) : (c & 3) == 2 ? quad_get<2>(mine) : quad_get<3>(mine);
+        double x = div_by(sc, L[c][c], rd[c]);
+        if (dropped && dropped[ok + c]) x = 0.0;
+        if (sub == (c & 3)) xr[c >> 2] = x;
+#pragma unroll
+        for (int q = c >> 2; q < 16; ++q)
+            if (4 * q + sub > c) xr[q] = fma(-x, L[4 * q + sub][c], xr[q]);
+    }
+#pragma unroll
+    for (int q = 0; q < 16; ++q) X[r][4 * q + sub] = xr[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int rr = TileRegs::row(q), c = TileRegs::col();
+        *reinterpret_cast<dt_v2*>(a + (oi + rr) * ld + ok + c) = dt_v2{X[rr][c], X[rr][c + 1]};
     }
 }
 
 // C (64 x 64 tile, row-major, leading dimension ldc) -= P Q^T  (BT) or P Q  (!BT), P and Q
-// 64 x 64 tiles (ldp, ldq); overwrite: C = P Q instead.  Both operands are staged in LDS
-// (Pt[l][r] = P[r][l]; Qt[l][c] = Q[c][l] or Q[l][c]) so that a thread's four rows and four
-// columns are consecutive words; each thread owns a 4 x 4 block of C.  All reads of P and
-// Q precede the barrier, so C may be the tile Q.
+// 64 x 64 tiles (ldp, ldq); overwrite: C = P Q instead.  On the FP64 matrix cores
+// (v_mfma_f64_16x16x4_f64: lane l feeds A row l % 16 and B column l % 16 at k = l / 16 and
+// holds D rows 4 t + l / 16, column l % 16): each of the four waves owns a 32 x 32 quarter
+// of C.  Both operands are staged in LDS with k contiguous (rows of 66 doubles: 16 rows at
+// two neighbouring k's fall on 32 different bank pairs).  The 4 x 4 register blocks on the
+// vector units that this replaces read eight LDS words per sixteen products.  Measured (us
+// per launch at 3,520 unknowns, with the tiles' loads issued together): trailing update
+// 57 -> 35, update of the inverse 71 -> 36, panel 16 -> 6.6.  All reads of P, Q and C precede the
+// barrier, so C may be the tile Q.
+typedef double dt_v4 __attribute__((ext_vector_type(4)));
+constexpr int kDTLd = kDT + 2;
 template <bool BT>
 __device__ __forceinline__ void tile_update(double* __restrict__ C, long ldc, const double* P, long ldp, const double* Q, long ldq,
-                                            double (*Pt)[kDT + 2], double (*Qt)[kDT + 2], bool overwrite,
-                                            const int* colMask = nullptr) {
+                                            double (*Pl)[kDTLd], double (*Ql)[kDTLd], bool overwrite, const int* colMask = nullptr) {
     // colMask (BT only): output columns c with colMask[c] != 0 come out zero
-    for (int e = threadIdx.x; e < kDT * kDT; e += kDirectBlock) {
-        const int r = e / kDT, l = e % kDT;
-        Pt[l][r] = P[r * ldp + l];
-        if (BT) Qt[l][r] = (colMask && colMask[r]) ? 0.0 : Q[r * ldq + l];
-        else Qt[r][l] = Q[r * ldq + l];
-    }
+    const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, g = lane >> 4;
+    const int r0 = 32 * (tid >> 7), c0 = 32 * ((tid >> 6) & 1);
+    double cv[2][2][4];
+    if (!overwrite)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) cv[i][j][t] = C[(r0 + 16 * i + 4 * t + g) * ldc + c0 + 16 * j + c];
+    TileRegs tp, tq;
+    tp.load(P, ldp);
+    tq.load(Q, ldq);
+    if (BT && colMask)
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (colMask[TileRegs::row(q)]) tq.v[q] = dt_v2{0, 0};
+    tp.put(Pl);
+    if (BT) tq.put(Ql);
+    else tq.put_transposed(Ql);
     __syncthreads();
-    const int tr = threadIdx.x / 16, tc = threadIdx.x % 16;
-    double acc[4][4];
+    dt_v4 acc[2][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
+        for (int j = 0; j < 2; ++j) acc[i][j] = dt_v4{0, 0, 0, 0};
 #pragma unroll 4
-    for (int l = 0; l < kDT; ++l) {
-        double pv[4], qv[4];
+    for (int l = 0; l < kDT; l += 4) {
+        double pv[2], qv[2];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            pv[i] = Pt[l][4 * tr + i];
-            qv[i] = Qt[l][4 * tc + i];
+        for (int i = 0; i < 2; ++i) {
+            pv[i] = Pl[r0 + 16 * i + c][l + g];
+            qv[i] = Ql[c0 + 16 * i + c][l + g];
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = fma(pv[i], qv[j], acc[i][j]);
+            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(pv[i], qv[j], acc[i][j], 0, 0, 0);
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            double* dst = C + (4 * tr + i) * ldc + 4 * tc + j;
-            *dst = overwrite ? acc[i][j] : *dst - acc[i][j];
-        }
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                double* dst = C + (r0 + 16 * i + 4 * t + g) * ldc + c0 + 16 * j + c;
+                *dst = overwrite ? acc[i][j][t] : cv[i][j][t] - acc[i][j][t];
+            }
 }
 
 // trailing update of the lower tiles (i, j), k < j <= i: A_ij -= L_ik L_jk^T; block b
 // enumerates the lower triangle of the trailing tile matrix row by row
 __global__ __launch_bounds__(kDirectBlock) void k_syrk_tiles(double* __restrict__ a, long ld, int k, int nt) {
-    __shared__ double Pt[kDT][kDT + 2];
-    __shared__ double Qt[kDT][kDT + 2];
+    __shared__ double Pt[kDT][kDTLd];
+    __shared__ double Qt[kDT][kDTLd];
     const int m = nt - k - 1;
     int b = blockIdx.x, ii = 0;
     while (b >= ii + 1) { b -= ii + 1; ++ii; }   // row ii of the trailing triangle holds ii + 1 tiles
@@ -244,8 +348,8 @@ __global__ __launch_bounds__(kDirectBlock) void k_syrk_tiles(double* __restrict_
 // dropped pivots zero
 __global__ __launch_bounds__(kDirectBlock) void k_panel_tiles(double* __restrict__ a, long ld, int k, const double* __restrict__ inv,
                                                              const int* __restrict__ dropped) {
-    __shared__ double Pt[kDT][kDT + 2];
-    __shared__ double Qt[kDT][kDT + 2];
+    __shared__ double Pt[kDT][kDTLd];
+    __shared__ double Qt[kDT][kDTLd];
     const int i = k + 1 + blockIdx.x;
     const long ok = (long)k * kDT, oi = (long)i * kDT;
     double* Aik = a + oi * ld + ok;
@@ -274,15 +378,15 @@ void dense_cholesky(Ctx& c, double* A, int npad, int* bad, double* tileInv, cons
 // row k:  W_kj = inv(L_kk) W_kj  (j <= k; W_kj holds the updated right-hand side)
 // update: W_ij -= L_ik W_kj      (i > k, j <= k)
 __global__ __launch_bounds__(kDirectBlock) void k_inv_row(const double* __restrict__ inv, double* __restrict__ W, long ld, int k) {
-    __shared__ double Pt[kDT][kDT + 2];
-    __shared__ double Qt[kDT][kDT + 2];
+    __shared__ double Pt[kDT][kDTLd];
+    __shared__ double Qt[kDT][kDTLd];
     const long ok = (long)k * kDT, oj = (long)blockIdx.x * kDT;   // tile column j = blockIdx.x <= k
     double* Wkj = W + ok * ld + oj;
     tile_update<false>(Wkj, ld, inv + (long)k * kDT * kDT, kDT, Wkj, ld, Pt, Qt, true);
 }
 __global__ __launch_bounds__(kDirectBlock) void k_inv_update(const double* __restrict__ L, double* __restrict__ W, long ld, int k) {
-    __shared__ double Pt[kDT][kDT + 2];
-    __shared__ double Qt[kDT][kDT + 2];
+    __shared__ double Pt[kDT][kDTLd];
+    __shared__ double Qt[kDT][kDTLd];
     const int j = blockIdx.x % (k + 1), i = k + 1 + blockIdx.x / (k + 1);
     const long ok = (long)k * kDT, oi = (long)i * kDT, oj = (long)j * kDT;
     tile_update<false>(W + oi * ld + oj, ld, L + oi * ld + ok, ld, W + ok * ld + oj, ld, Pt, Qt, false);
@@ -306,52 +410,64 @@ void dense_lower_inverse(Ctx& c, const double* L, double* W, int npad, const dou
     }
 }
 
-// forward substitution, tile k: y_k = L_kk^-1 b_k (b_k already holds the updates of the
-// earlier tiles); backward: x_k = L_kk^-T y_k
-__global__ void k_trsv_tile(const double* __restrict__ a, long ld, int k, double* __restrict__ y, int transposed) {
+// Tile k of the substitutions, one launch: every workgroup solves the diagonal tile itself
+// (forward u_k = L_kk^-1 y_k; backward x_k = L_kk^-T u_k), the first writes the result, and
+// workgroup b subtracts its tile's product from the right-hand side of tile k + 1 + b
+// (forward) or b (backward).  The result goes to another vector than the right-hand side,
+// which the other workgroups still read.  The solve runs in one wave, lane = row: a finished
+// entry crosses by readlane and every row subtracts its term at once (one thread for the
+// whole triangle took 54 us); the tile for the product is loaded meanwhile.
+template <bool transposed>
+__global__ __launch_bounds__(kDirectBlock) void k_subst_tile(const double* __restrict__ a, long ld, int k, int nRest, double* __restrict__ y,
+                                                             double* __restrict__ out) {
     __shared__ double L[kDT][kDT + 1];
     __shared__ double v[kDT];
-    const long ok = (long)k * kDT;
-    for (int e = threadIdx.x; e < kDT * kDT; e += blockDim.x) {
-        const int r = e / kDT, c = e % kDT;
-        L[r][c] = a[(ok + r) * ld + ok + c];
+    __shared__ double part[4][kDT];
+    const int tid = threadIdx.x, b = blockIdx.x, ti = transposed ? b : k + 1 + b;
+    const long ok = (long)k * kDT, oi = (long)ti * kDT;
+    const bool work = b < nRest;
+    TileRegs tl;
+    tl.load(a + ok * ld + ok, ld);
+    double s = tid < kDT ? y[ok + tid] : 0.0;
+    // forward: rows 16 q + tid / 16, columns 4 (tid % 16) ..; backward: columns tid % 64,
+    // rows 16 (tid / 64) + q
+    double m[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) {
+        const long src = transposed ? (ok + 16 * (tid >> 6) + q) * ld + oi + (tid & 63)
+                                    : (oi + 16 * (q >> 2) + (tid >> 4)) * ld + ok + 4 * (tid & 15) + (q & 3);
+        m[q] = work ? a[src] : 0.0;
     }
-    for (int e = threadIdx.x; e < kDT; e += blockDim.x) v[e] = y[ok + e];
+    if (transposed) tl.put_transposed(L);
+    else tl.put(L);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        if (!transposed) {
-            for (int r = 0; r < kDT; ++r) {
-                double s = v[r];
-                for (int m = 0; m < r; ++m) s -= L[r][m] * v[m];
-                v[r] = s / L[r][r];
-            }
-        } else {
-            for (int r = kDT - 1; r >= 0; --r) {
-                double s = v[r];
-                for (int m = r + 1; m < kDT; ++m) s -= L[m][r] * v[m];
-                v[r] = s / L[r][r];
-            }
+    if (tid < kDT) {
+        const double d = L[tid][tid], rd = 1.0 / d;
+#pragma unroll
+        for (int n = 0; n < kDT; ++n) {
+            const int c = transposed ? kDT - 1 - n : n;
+            const double x = lane_read(div_by(s, d, rd), c);
+            s = tid == c ? x : (transposed ? tid < c : tid > c) ? fma(-L[tid][c], x, s) : s;
         }
+        v[tid] = s;
+        if (b == 0) out[ok + tid] = s;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < kDT; e += blockDim.x) y[ok + e] = v[e];
-}
-// forward: y_i -= L_ik y_k for tiles i > k (block per tile); backward: y_i -= L_ki^T y_k
-// for tiles i < k
-__global__ void k_gemv_tiles(const double* __restrict__ a, long ld, int k, double* __restrict__ y, int transposed) {
-    __shared__ double yk[kDT];
-    const int i = transposed ? blockIdx.x : k + 1 + blockIdx.x;
-    const long ok = (long)k * kDT, oi = (long)i * kDT;
-    for (int e = threadIdx.x; e < kDT; e += blockDim.x) yk[e] = y[ok + e];
-    __syncthreads();
-    if (threadIdx.x < kDT) {
-        const int r = threadIdx.x;
-        double s = 0;
-        if (!transposed)
-            for (int c = 0; c < kDT; ++c) s += a[(oi + r) * ld + ok + c] * yk[c];
-        else
-            for (int c = 0; c < kDT; ++c) s += a[(ok + c) * ld + oi + r] * yk[c];
-        y[oi + r] -= s;
+    if (!work) return;
+    if (!transposed) {
+        const int c4 = 4 * (tid & 15);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const double ps = lane_sum<16>(((m[4 * q] * v[c4] + m[4 * q + 1] * v[c4 + 1]) + m[4 * q + 2] * v[c4 + 2]) + m[4 * q + 3] * v[c4 + 3]);
+            if ((tid & 15) == 0) y[oi + 16 * q + (tid >> 4)] -= ps;
+        }
+    } else {
+        double ps = 0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) ps = fma(m[q], v[16 * (tid >> 6) + q], ps);
+        part[tid >> 6][tid & 63] = ps;
+        __syncthreads();
+        if (tid < kDT) y[oi + tid] -= ((part[0][tid] + part[1][tid]) + part[2][tid]) + part[3][tid];
     }
 }
 
@@ -374,19 +490,16 @@ int direct_solve(Ctx& c, const double* b, double* x) {
     int* bad = c.denseBad.ensure(1);
     CIPC_HIP(hipMemsetAsync(bad, 0, sizeof(int), c.s));
     dense_cholesky(c, A, npad, bad, nullptr);
-    double* y = c.denseY.ensure(npad);
+    double* y = c.denseY.ensure(3 * (size_t)npad);
+    double *u = y + npad, *xs = u + npad;   // forward and backward results
     CIPC_HIP(hipMemsetAsync(y, 0, npad * sizeof(double), c.s));
     CIPC_HIP(hipMemcpyAsync(y, b, n * sizeof(double), hipMemcpyDeviceToDevice, c.s));
-    for (int k = 0; k < nt; ++k) {
-        hipLaunchKernelGGL(k_trsv_tile, dim3(1), dim3(kDT), 0, c.s, A, ld, k, y, 0);
-        if (nt - k - 1 > 0) hipLaunchKernelGGL(k_gemv_tiles, dim3(nt - k - 1), dim3(kDT), 0, c.s, A, ld, k, y, 0);
-    }
-    for (int k = nt - 1; k >= 0; --k) {
-        hipLaunchKernelGGL(k_trsv_tile, dim3(1), dim3(kDT), 0, c.s, A, ld, k, y, 1);
-        if (k > 0) hipLaunchKernelGGL(k_gemv_tiles, dim3(k), dim3(kDT), 0, c.s, A, ld, k, y, 1);
-    }
+    for (int k = 0; k < nt; ++k)
+        hipLaunchKernelGGL(k_subst_tile<false>, dim3(std::max(1, nt - k - 1)), dim3(kDirectBlock), 0, c.s, (const double*)A, ld, k, nt - k - 1, y, u);
+    for (int k = nt - 1; k >= 0; --k)
+        hipLaunchKernelGGL(k_subst_tile<true>, dim3(std::max(1, k)), dim3(kDirectBlock), 0, c.s, (const double*)A, ld, k, k, u, xs);
     CIPC_LAUNCH_CHECK();
-    CIPC_HIP(hipMemcpyAsync(x, y, n * sizeof(double), hipMemcpyDeviceToDevice, c.s));
+    CIPC_HIP(hipMemcpyAsync(x, xs, n * sizeof(double), hipMemcpyDeviceToDevice, c.s));
     CIPC_HIP(hipMemcpyAsync(c.hCnt + 48, bad, sizeof(int), hipMemcpyDeviceToHost, c.s));
     CIPC_HIP(hipStreamSynchronize(c.s));
     c.directSolves++;
