@@ -263,10 +263,11 @@ __device__ __forceinline__ int ecell(int vox, int f, int dim) {
 // primitive voxel range = union of its nodes' ranges; count of enumeration cells
 // (0 for primitives covering more than kLargeCells cells, which go to the large list)
 __global__ void k_prim_vox(const int* __restrict__ verts, int n, int nv, const int* __restrict__ vlo, const int* __restrict__ vhi, int nV,
-                           VoxGrid G, int* __restrict__ plo, int* __restrict__ phi, int4* __restrict__ box, uint32_t* __restrict__ cnt,
+                           VoxGrid G, int* __restrict__ plo, int* __restrict__ phi, int4* __restrict__ box, uint32_t* __restrict__ count,
                            uint8_t* __restrict__ lgFlag, int* __restrict__ lgList, uint32_t* __restrict__ lgCount) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int i = cell_prim();
     if (i >= n) return;
+    const bool lead = threadIdx.x % kCellLanes == 0;
     uint64_t c = 1;
     int blo[3], bhi[3];
 #pragma unroll
@@ -277,42 +278,38 @@ __global__ void k_prim_vox(const int* __restrict__ verts, int n, int nv, const i
             lo = min(lo, vlo[d * nV + v]);
             hi = max(hi, vhi[d * nV + v]);
         }
-        plo[(long)d * n + i] = lo;
-        phi[(long)d * n + i] = hi;
+        if (lead) {
+            plo[(long)d * n + i] = lo;
+            phi[(long)d * n + i] = hi;
+        }
         blo[d] = lo;
         bhi[d] = hi;
         c *= (uint64_t)(ecell(hi, G.f, G.edim[d]) - ecell(lo, G.f, G.edim[d]) + 1);
     }
-    // the same box as one 32-byte record (lo xyz, hi x | hi yz) for the candidate loops
-    box[2l * i] = make_int4(blo[0], blo[1], blo[2], bhi[0]);
-    box[2l * i + 1] = make_int4(bhi[1], bhi[2], 0, 0);
     const bool large = c > kLargeCells;
-    lgFlag[i] = large ? 1 : 0;
-    cnt[i] = large ? 0u : (uint32_t)c;
-    if (large) lgList[atomicAdd(lgCount, 1u)] = i;
-}
-__global__ void k_prim_vox_emit(int n, const int* __restrict__ plo, const int* __restrict__ phi, VoxGrid G, const uint8_t* __restrict__ lgFlag,
-                                const uint32_t* __restrict__ off, uint64_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || lgFlag[i]) return;
+    if (lead) {
+        // the same box as one 32-byte record (lo xyz, hi x | hi yz) for the candidate loops
+        box[2l * i] = make_int4(blo[0], blo[1], blo[2], bhi[0]);
+        box[2l * i + 1] = make_int4(bhi[1], bhi[2], 0, 0);
+        lgFlag[i] = large ? 1 : 0;
+        if (large) lgList[atomicAdd(lgCount, 1u)] = i;
+    }
+    if (large) return;
     int a[3], b[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) { a[d] = ecell(plo[(long)d * n + i], G.f, G.edim[d]); b[d] = ecell(phi[(long)d * n + i], G.f, G.edim[d]); }
-    uint32_t o = off[i];
-    for (int iz = a[2]; iz <= b[2]; ++iz)
-        for (int iy = a[1]; iy <= b[1]; ++iy)
-            for (int ix = a[0]; ix <= b[0]; ++ix) {
-                keys[o] = (uint64_t)ix + (uint64_t)G.edim[0] * ((uint64_t)iy + (uint64_t)G.edim[1] * (uint64_t)iz);
-                vals[o] = walk_entry(i, ix == a[0], iy == a[1], iz == a[2]);
-                ++o;
-            }
+    for (int d = 0; d < 3; ++d) { a[d] = ecell(blo[d], G.f, G.edim[d]); b[d] = ecell(bhi[d], G.f, G.edim[d]); }
+    for_prim_cells(a, b, G.edim, [&](long cell, bool, bool, bool) { atomicAdd(&count[cell], 1u); });
 }
-__global__ void k_cell_bounds2(const uint64_t* __restrict__ keys, long n, uint32_t* __restrict__ start, uint32_t* __restrict__ end) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t k = keys[i];
-    if (i == 0 || keys[i - 1] != k) start[k] = (uint32_t)i;
-    if (i == n - 1 || keys[i + 1] != k) end[k] = (uint32_t)(i + 1);
+__global__ void k_prim_vox_emit(int n, const int4* __restrict__ box, VoxGrid G, const uint8_t* __restrict__ lgFlag,
+                                const uint32_t* __restrict__ start, uint32_t* __restrict__ count, int4* __restrict__ rec) {
+    const int i = cell_prim();
+    if (i >= n || lgFlag[i]) return;
+    const int4 ba = box[2l * i], bb = box[2l * i + 1];
+    const int lo[3] = {ba.x, ba.y, ba.z}, hi[3] = {ba.w, bb.x, bb.y};
+    int a[3], b[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) { a[d] = ecell(lo[d], G.f, G.edim[d]); b[d] = ecell(hi[d], G.f, G.edim[d]); }
+    for_prim_cells(a, b, G.edim, [&](long cell, bool fx, bool fy, bool fz) { walk_put(rec, start, count, cell, ba, bb, walk_entry(i, fx, fy, fz)); });
 }
 
 __device__ __forceinline__ void atomic_min_pos(unsigned long long* a, double v) {
@@ -462,10 +459,9 @@ __device__ __forceinline__ void pp_ccd_candidate(const double* __restrict__ x, c
 __global__ void k_ccd_codim(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ bNode, int nBN,
                             int codimBN1, const int* __restrict__ bEdge, int nBE, int nRod, const uint8_t* __restrict__ dbc,
                             const int* __restrict__ vlo, const int* __restrict__ vhi, int nV, const int* __restrict__ elo,
-                            const int* __restrict__ ehi, VoxGrid G, const uint32_t* __restrict__ estart, const uint32_t* __restrict__ eend,
-                            const uint32_t* __restrict__ evals, const int* __restrict__ lgListE, const uint32_t* __restrict__ lgCountE,
-                            const uint32_t* __restrict__ pstart, const uint32_t* __restrict__ pend,
-                            const uint32_t* __restrict__ pvals, const uint8_t* __restrict__ lgFlagP, const int* __restrict__ lgListP,
+                            const int* __restrict__ ehi, VoxGrid G, const uint32_t* __restrict__ estart,
+                            const int4* __restrict__ erec, const int* __restrict__ lgListE, const uint32_t* __restrict__ lgCountE,
+                            const uint32_t* __restrict__ pstart, const int4* __restrict__ prec, const uint8_t* __restrict__ lgFlagP, const int* __restrict__ lgListP,
                             const uint32_t* __restrict__ lgCountP, double alpha0, double xi, unsigned long long* __restrict__ gmin) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     int s = codimBN1 + j;
@@ -487,14 +483,16 @@ __global__ void k_ccd_codim(const double* __restrict__ x, const double* __restri
                 for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
                     uint64_t cell = (uint64_t)ix + (uint64_t)G.edim[0] * ((uint64_t)iy + (uint64_t)G.edim[1] * (uint64_t)iz);
                     const int own = (ix == qlo[0] ? 1 : 0) | (iy == qlo[1] ? 2 : 0) | (iz == qlo[2] ? 4 : 0);
-                    for (uint32_t k = estart[cell], en = eend[cell]; k < en; ++k) {
-                        const int e = (int)(evals[k] & kWalkId), first = (int)(evals[k] >> kWalkIdBits);
+                    for (uint32_t k = estart[cell], en = estart[cell + 1]; k < en; ++k) {
+                        const uint32_t entry = (uint32_t)erec[2l * k + 1].z;
+                        const int e = (int)(entry & kWalkId), first = (int)(entry >> kWalkIdBits);
                         if (e < firstRod) continue;
                         if ((first | own) != 7) continue;
                         pe_ccd_candidate(x, p, bEdge, nBE, dbc, elo, ehi, vI, nlo, nhi, P, dP, e, xi, largest);
                     }
-                    for (uint32_t k = pstart[cell], en = pend[cell]; k < en; ++k) {
-                        const int jJ = (int)(pvals[k] & kWalkId), first = (int)(pvals[k] >> kWalkIdBits);
+                    for (uint32_t k = pstart[cell], en = pstart[cell + 1]; k < en; ++k) {
+                        const uint32_t entry = (uint32_t)prec[2l * k + 1].z;
+                        const int jJ = (int)(entry & kWalkId), first = (int)(entry >> kWalkIdBits);
                         if (jJ <= j) continue;
                         if ((first | own) != 7) continue;
                         pp_ccd_candidate(x, p, dbc, vlo, vhi, nV, vI, bNode[codimBN1 + jJ], xi, largest);
@@ -521,45 +519,33 @@ __global__ void k_ccd_codim(const double* __restrict__ x, const double* __restri
     if (largest < alpha0) atomic_min_pos(gmin, largest);
 }
 
-static int bits_for2(uint64_t n) {
-    int b = 1;
-    while (b < 64 && (1ull << b) < n) ++b;
-    return b;
+struct VoxBuild {
+    const int* verts;
+    int n, nv;
+    DevBuf<int>&plo, &phi, &box, &rec;
+    DevBuf<uint32_t>&start, &count;
+    DevBuf<uint8_t>& lgFlag;
+    DevBuf<int>& lgList;
+    uint32_t *lgCount, *hTotal;
+};
+static void vox_count(Ctx& c, const int* vlo, const int* vhi, const VoxGrid& G, const VoxBuild& b) {
+    const long nCells = (long)G.edim[0] * G.edim[1] * G.edim[2];
+    walk_cells_begin(c, nCells, b.n, b.start, b.count, b.box, b.lgFlag, b.lgList);
+    b.plo.ensure(3l * std::max(b.n, 1));
+    b.phi.ensure(3l * std::max(b.n, 1));
+    if (b.n) {
+        hipLaunchKernelGGL(k_prim_vox, cell_blocks(b.n), dim3(kBlock), 0, c.s, b.verts, b.n, b.nv, vlo, vhi, c.nV, G, b.plo.p, b.phi.p,
+                           (int4*)b.box.p, b.count.p, b.lgFlag.p, b.lgList.p, b.lgCount);
+        CIPC_LAUNCH_CHECK();
+    }
+    walk_cells_scan(c, nCells, b.start, b.count, b.hTotal);
 }
-
-static long build_vox_cells(Ctx& c, const int* verts, int n, int nv, const int* vlo, const int* vhi, const VoxGrid& G, DevBuf<int>& plo,
-                            DevBuf<int>& phi, DevBuf<int>& box, DevBuf<uint64_t>& keys, DevBuf<uint32_t>& vals, DevBuf<uint32_t>& start,
-                            DevBuf<uint32_t>& end, DevBuf<uint8_t>& lgFlag, DevBuf<int>& lgList, uint32_t* lgCount) {
-    long nCells = (long)G.edim[0] * G.edim[1] * G.edim[2];
-    start.ensure(nCells);
-    end.ensure(nCells);
-    CIPC_HIP(hipMemsetAsync(start.p, 0, nCells * sizeof(uint32_t), c.s));
-    CIPC_HIP(hipMemsetAsync(end.p, 0, nCells * sizeof(uint32_t), c.s));
-    CIPC_HIP(hipMemsetAsync(lgCount, 0, sizeof(uint32_t), c.s));
-    lgFlag.ensure((size_t)n + 1);
-    lgList.ensure((size_t)n + 1);
-    if (n == 0) return 0;
-    plo.ensure(3l * n);
-    phi.ensure(3l * n);
-    box.ensure(8l * n);
-    uint32_t* cnt = c.u32a.ensure(n + 1);
-    uint32_t* off = c.u32b.ensure(n + 1);
-    hipLaunchKernelGGL(k_prim_vox, dim3(nblocks(n)), dim3(kBlock), 0, c.s, verts, n, nv, vlo, vhi, c.nV, G, plo.p, phi.p, (int4*)box.p, cnt, lgFlag.p,
-                       lgList.p, lgCount);
+static void vox_emit(Ctx& c, const VoxGrid& G, const VoxBuild& b) {
+    b.rec.ensure(8 * (size_t)std::max(*b.hTotal, 1u));
+    if (*b.hTotal == 0) return;
+    hipLaunchKernelGGL(k_prim_vox_emit, cell_blocks(b.n), dim3(kBlock), 0, c.s, b.n, (const int4*)b.box.p, G, (const uint8_t*)b.lgFlag.p,
+                       (const uint32_t*)b.start.p, b.count.p, (int4*)b.rec.p);
     CIPC_LAUNCH_CHECK();
-    scan_exclusive(cnt, off, n, c.counters.p + 9, c.pw, c.s);
-    CIPC_HIP(hipMemcpyAsync(c.hCnt + 9, c.counters.p + 9, sizeof(uint32_t), hipMemcpyDeviceToHost, c.s));
-    CIPC_HIP(hipStreamSynchronize(c.s));
-    long total = c.hCnt[9];
-    if (total == 0) return 0;
-    keys.ensure(total);
-    vals.ensure(total);
-    hipLaunchKernelGGL(k_prim_vox_emit, dim3(nblocks(n)), dim3(kBlock), 0, c.s, n, plo.p, phi.p, G, lgFlag.p, off, keys.p, vals.p);
-    CIPC_LAUNCH_CHECK();
-    radix_sort_pairs(keys.p, vals.p, total, bits_for2((uint64_t)nCells), c.pw, c.s);
-    hipLaunchKernelGGL(k_cell_bounds2, dim3(nblocks(total)), dim3(kBlock), 0, c.s, keys.p, total, start.p, end.p);
-    CIPC_LAUNCH_CHECK();
-    return total;
 }
 
 double ccd_stepsize(Ctx& c, const double* x, const double* p, double alpha, double* clamped, int* zeroToi) {
@@ -630,47 +616,40 @@ double ccd_stepsize(Ctx& c, const double* x, const double* p, double alpha, doub
     double a0 = alpha;
     CIPC_HIP(hipMemcpyAsync(gmin, &a0, sizeof(double), hipMemcpyHostToDevice, c.s));
     CIPC_HIP(hipMemsetAsync(c.counters.p + 13, 0, sizeof(uint32_t), c.s));
-    // point-triangle
-    uint32_t* lgCountT = c.counters.p + 18;
-    uint32_t* lgCountE = c.counters.p + 19;
-    auto records = [&](long total, const DevBuf<uint32_t>& vals, const DevBuf<int>& box, DevBuf<int>& rec) {
-        rec.ensure(8 * (size_t)std::max(total, 1L));
-        if (total > 0) {
-            hipLaunchKernelGGL(k_walk_records, dim3(nblocks(total)), dim3(kBlock), 0, c.s, (const uint32_t*)vals.p, total, (const int4*)box.p,
-                               (int4*)rec.p);
-            CIPC_LAUNCH_CHECK();
-        }
-    };
+    uint32_t* lgCountT = c.counters.p + 19;
+    uint32_t* lgCountE = c.counters.p + 20;
+    uint32_t* lgCountP = c.counters.p + 21;
+    CIPC_HIP(hipMemsetAsync(lgCountT, 0, 3 * sizeof(uint32_t), c.s));
+    const VoxBuild bt = {c.btri.p, c.nBT, 3, c.ccdTlo, c.ccdThi, c.ccdTbox, c.ccdTrec, c.cellStart, c.cellCount, c.lgFlagT, c.lgListT, lgCountT, c.hCnt + 9};
+    const VoxBuild be = {c.bEdge.p, c.nBE, 2, c.ccdElo, c.ccdEhi, c.ccdEbox, c.ccdErec, c.ecellStart, c.ecellCount, c.lgFlagE, c.lgListE, lgCountE, c.hCnt + 10};
+    const VoxBuild bp = {c.partSlot.p, c.nPart, 1, c.ccdPlo, c.ccdPhi, c.ccdPbox, c.ccdPrec, c.pcellStart, c.pcellCount, c.lgFlagP, c.lgListP, lgCountP, c.hCnt + 11};
+    vox_count(c, vlo, vhi, G, bt);
+    vox_count(c, vlo, vhi, G, be);
+    if (c.nPart) vox_count(c, vlo, vhi, G, bp);
+    CIPC_HIP(hipStreamSynchronize(c.s));   // the three totals
+    vox_emit(c, G, bt);
+    vox_emit(c, G, be);
+    if (c.nPart) vox_emit(c, G, bp);
     const StepMin sm = {gmin, c.counters.p + 13, nullptr};
-    const long totT = build_vox_cells(c, c.btri.p, c.nBT, 3, vlo, vhi, G, c.ccdTlo, c.ccdThi, c.ccdTbox, c.k64a, c.u32c, c.cellStart, c.cellEnd,
-                                      c.lgFlagT, c.lgListT, lgCountT);
-    records(totT, c.u32c, c.ccdTbox, c.ccdTrec);
     if (c.nBN && c.nBT) {
         const CcdPT pt = {x, p, c.bNode.p, c.btri.p, c.nBT, c.dbc.p, vlo, vhi, c.nV, G, xi, sm, {}, {}};
-        const CellGrid cg = {{G.edim[0], G.edim[1], G.edim[2]}, c.cellStart.p, c.cellEnd.p, (const int4*)c.ccdTrec.p, (const int4*)c.ccdTbox.p,
+        const CellGrid cg = {{G.edim[0], G.edim[1], G.edim[2]}, c.cellStart.p, (const int4*)c.ccdTrec.p, (const int4*)c.ccdTbox.p,
                              c.lgListT.p, lgCountT};
         hipLaunchKernelGGL(k_ccd_walk<CcdPT>, dim3(walk_grid(c.nBN)), dim3(kBlock), 0, c.s, pt, c.nBN, alpha, cg);
         CIPC_LAUNCH_CHECK();
     }
-    // edge-edge
-    const long totE = build_vox_cells(c, c.bEdge.p, c.nBE, 2, vlo, vhi, G, c.ccdElo, c.ccdEhi, c.ccdEbox, c.k64b, c.u32d, c.ecellStart,
-                                      c.ecellEnd, c.lgFlagE, c.lgListE, lgCountE);
-    records(totE, c.u32d, c.ccdEbox, c.ccdErec);
     if (c.nBE) {
         const CcdEE ee = {x, p, c.bEdge.p, c.nBE, c.dbc.p, (const int4*)c.ccdEbox.p, c.lgFlagE.p, G, xi, sm, {}, {}};
-        const CellGrid cg = {{G.edim[0], G.edim[1], G.edim[2]}, c.ecellStart.p, c.ecellEnd.p, (const int4*)c.ccdErec.p,
-                             (const int4*)c.ccdEbox.p, c.lgListE.p, lgCountE};
+        const CellGrid cg = {{G.edim[0], G.edim[1], G.edim[2]}, c.ecellStart.p, (const int4*)c.ccdErec.p, (const int4*)c.ccdEbox.p,
+                             c.lgListE.p, lgCountE};
         hipLaunchKernelGGL(k_ccd_walk<CcdEE>, dim3(walk_grid(c.nBE)), dim3(kBlock), 0, c.s, ee, c.nBE, alpha, cg);
         CIPC_LAUNCH_CHECK();
     }
     // particles against rod segments and particle pairs
     if (c.nPart) {
-        uint32_t* lgCountP = c.counters.p + 21;
-        build_vox_cells(c, c.partSlot.p, c.nPart, 1, vlo, vhi, G, c.ccdPlo, c.ccdPhi, c.ccdPbox, c.pKeys, c.pVals, c.pcellStart, c.pcellEnd,
-                        c.lgFlagP, c.lgListP, lgCountP);
         hipLaunchKernelGGL(k_ccd_codim, dim3(nblocks(c.nPart)), dim3(kBlock), 0, c.s, x, p, c.bNode.p, c.nBN, c.codimBN1, c.bEdge.p, c.nBE,
-                           c.nRod, c.dbc.p, vlo, vhi, c.nV, c.ccdElo.p, c.ccdEhi.p, G, c.ecellStart.p, c.ecellEnd.p, c.u32d.p,
-                           c.lgListE.p, lgCountE, c.pcellStart.p, c.pcellEnd.p, c.pVals.p, c.lgFlagP.p, c.lgListP.p,
+                           c.nRod, c.dbc.p, vlo, vhi, c.nV, c.ccdElo.p, c.ccdEhi.p, G, c.ecellStart.p, (const int4*)c.ccdErec.p,
+                           c.lgListE.p, lgCountE, c.pcellStart.p, (const int4*)c.ccdPrec.p, c.lgFlagP.p, c.lgListP.p,
                            lgCountP, alpha, xi, gmin);
         CIPC_LAUNCH_CHECK();
     }

@@ -7,8 +7,7 @@
 //
 // Broad phase: a uniform grid (cell = mean rest boundary-edge length, grown so the
 // grid has at most 2^23 cells) holds each triangle / edge in every cell its AABB
-// touches; entries are sorted by cell (stable radix sort) and each cell's run is
-// found through dense start/end tables.  A query visits the cells of its box (walk.hpp) and
+// touches, cell after cell (counted, prefix sum, placed).  A query visits the cells of its box (walk.hpp) and
 // accepts a candidate only in the first cell common to both boxes, so every pair is
 // tested once; indices are clamped into the grid, which keeps the search complete
 // for points outside it.  The active set is defined by the reference's predicates
@@ -59,93 +58,77 @@ __device__ __forceinline__ void prim_minmax(const double* __restrict__ x, const 
 }
 __global__ void k_prim_range(const double* __restrict__ x, const int* __restrict__ verts, int n, int nv, GridParams G,
                              int4* __restrict__ box, uint32_t* __restrict__ count, uint8_t* __restrict__ lgFlag,
-                             int* __restrict__ lgList, uint32_t* __restrict__ lgCount) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+                             int* __restrict__ lgList, uint32_t* __restrict__ lgCount) {   // count: per cell
+    const int i = cell_prim();
     if (i >= n) return;
     double mn[3], mx[3];
     prim_minmax(x, verts, n, nv, i, mn, mx);
     uint64_t cnt = 1;
+    int a[3], b[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-        int a = cell_of(mn[d], G.lb[d], G.inv, G.dim[d]), b = cell_of(mx[d], G.lb[d], G.inv, G.dim[d]);
-        cnt *= (uint64_t)(b - a + 1);
+        a[d] = cell_of(mn[d], G.lb[d], G.inv, G.dim[d]);
+        b[d] = cell_of(mx[d], G.lb[d], G.inv, G.dim[d]);
+        cnt *= (uint64_t)(b[d] - a[d] + 1);
     }
-    box[2l * i] = make_int4(__float_as_int(float_below(mn[0])), __float_as_int(float_below(mn[1])), __float_as_int(float_below(mn[2])),
-                            __float_as_int(float_above(mx[0])));
-    box[2l * i + 1] = make_int4(__float_as_int(float_above(mx[1])), __float_as_int(float_above(mx[2])), 0, 0);
     const bool large = cnt > kLargeCells;
-    lgFlag[i] = large ? 1 : 0;
-    count[i] = large ? 0u : (uint32_t)cnt;
-    if (large) lgList[atomicAdd(lgCount, 1u)] = i;
+    if (threadIdx.x % kCellLanes == 0) {
+        box[2l * i] = make_int4(__float_as_int(float_below(mn[0])), __float_as_int(float_below(mn[1])), __float_as_int(float_below(mn[2])),
+                                __float_as_int(float_above(mx[0])));
+        box[2l * i + 1] = make_int4(__float_as_int(float_above(mx[1])), __float_as_int(float_above(mx[2])), 0, 0);
+        lgFlag[i] = large ? 1 : 0;
+        if (large) lgList[atomicAdd(lgCount, 1u)] = i;
+    }
+    if (large) return;
+    for_prim_cells(a, b, G.dim, [&](long cell, bool, bool, bool) { atomicAdd(&count[cell], 1u); });
 }
 __global__ void k_prim_emit(const double* __restrict__ x, const int* __restrict__ verts, int n, int nv, GridParams G,
-                            const uint8_t* __restrict__ lgFlag, const uint32_t* __restrict__ off, uint64_t* __restrict__ keys,
-                            uint32_t* __restrict__ vals) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+                            const uint8_t* __restrict__ lgFlag, const int4* __restrict__ box, const uint32_t* __restrict__ start,
+                            uint32_t* __restrict__ count, int4* __restrict__ rec) {
+    const int i = cell_prim();
     if (i >= n || lgFlag[i]) return;
     double mn[3], mx[3];
     prim_minmax(x, verts, n, nv, i, mn, mx);
     int a[3], b[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) { a[d] = cell_of(mn[d], G.lb[d], G.inv, G.dim[d]); b[d] = cell_of(mx[d], G.lb[d], G.inv, G.dim[d]); }
-    uint32_t o = off[i];
-    for (int iz = a[2]; iz <= b[2]; ++iz)
-        for (int iy = a[1]; iy <= b[1]; ++iy)
-            for (int ix = a[0]; ix <= b[0]; ++ix) {
-                keys[o] = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
-                vals[o] = walk_entry(i, ix == a[0], iy == a[1], iz == a[2]);
-                ++o;
-            }
+    const int4 ba = box[2l * i], bb = box[2l * i + 1];
+    for_prim_cells(a, b, G.dim, [&](long cell, bool fx, bool fy, bool fz) { walk_put(rec, start, count, cell, ba, bb, walk_entry(i, fx, fy, fz)); });
 }
-__global__ void k_cell_bounds(const uint64_t* __restrict__ keys, long n, uint32_t* __restrict__ start, uint32_t* __restrict__ end) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    uint64_t k = keys[i];
-    if (i == 0 || keys[i - 1] != k) start[k] = (uint32_t)i;
-    if (i == n - 1 || keys[i + 1] != k) end[k] = (uint32_t)(i + 1);
-}
-
 static int bits_for(uint64_t n) {
     int b = 1;
     while (b < 64 && (1ull << b) < n) ++b;
     return b;
 }
 
-// builds the sorted cell lists of one primitive kind (large primitives listed apart,
-// their count left in device memory at lgCount); returns number of cell entries
-static long build_cells(Ctx& c, const double* x, const int* verts, int n, int nv, const GridParams& G, DevBuf<int>& box, DevBuf<int>& rec,
-                        DevBuf<uint64_t>& keys, DevBuf<uint32_t>& vals, DevBuf<uint32_t>& start, DevBuf<uint32_t>& end,
-                        DevBuf<uint8_t>& lgFlag, DevBuf<int>& lgList, uint32_t* lgCount) {
-    long nCells = (long)G.dim[0] * G.dim[1] * G.dim[2];
-    start.ensure(nCells);
-    end.ensure(nCells);
-    CIPC_HIP(hipMemsetAsync(start.p, 0, nCells * sizeof(uint32_t), c.s));
-    CIPC_HIP(hipMemsetAsync(end.p, 0, nCells * sizeof(uint32_t), c.s));
-    CIPC_HIP(hipMemsetAsync(lgCount, 0, sizeof(uint32_t), c.s));
-    lgFlag.ensure((size_t)n + 1);
-    lgList.ensure((size_t)n + 1);
-    if (n == 0) return 0;
-    box.ensure((size_t)8 * n);
-    uint32_t* cnt = c.u32a.ensure(n + 1);
-    uint32_t* off = c.u32b.ensure(n + 1);
-    hipLaunchKernelGGL(k_prim_range, dim3(nblocks(n)), dim3(kBlock), 0, c.s, x, verts, n, nv, G, (int4*)box.p, cnt, lgFlag.p, lgList.p, lgCount);
+// cell lists of one primitive kind (large primitives listed apart, their count left in
+// device memory at lgCount): counts and starts, then, once the host knows the number of
+// entries, the records
+struct CellBuild {
+    const int* verts;
+    int n, nv;
+    DevBuf<int>&box, &rec;
+    DevBuf<uint32_t>&start, &count;
+    DevBuf<uint8_t>& lgFlag;
+    DevBuf<int>& lgList;
+    uint32_t *lgCount, *hTotal;
+};
+static void cells_count(Ctx& c, const double* x, const GridParams& G, const CellBuild& b) {
+    const long nCells = (long)G.dim[0] * G.dim[1] * G.dim[2];
+    walk_cells_begin(c, nCells, b.n, b.start, b.count, b.box, b.lgFlag, b.lgList);
+    if (b.n) {
+        hipLaunchKernelGGL(k_prim_range, cell_blocks(b.n), dim3(kBlock), 0, c.s, x, b.verts, b.n, b.nv, G, (int4*)b.box.p, b.count.p,
+                           b.lgFlag.p, b.lgList.p, b.lgCount);
+        CIPC_LAUNCH_CHECK();
+    }
+    walk_cells_scan(c, nCells, b.start, b.count, b.hTotal);
+}
+static void cells_emit(Ctx& c, const double* x, const GridParams& G, const CellBuild& b) {
+    b.rec.ensure(8 * (size_t)std::max(*b.hTotal, 1u));
+    if (*b.hTotal == 0) return;
+    hipLaunchKernelGGL(k_prim_emit, cell_blocks(b.n), dim3(kBlock), 0, c.s, x, b.verts, b.n, b.nv, G, (const uint8_t*)b.lgFlag.p,
+                       (const int4*)b.box.p, (const uint32_t*)b.start.p, b.count.p, (int4*)b.rec.p);
     CIPC_LAUNCH_CHECK();
-    scan_exclusive(cnt, off, n, c.counters.p + 8, c.pw, c.s);
-    CIPC_HIP(hipMemcpyAsync(c.hCnt + 8, c.counters.p + 8, sizeof(uint32_t), hipMemcpyDeviceToHost, c.s));
-    CIPC_HIP(hipStreamSynchronize(c.s));
-    long total = c.hCnt[8];
-    if (total == 0) return 0;
-    keys.ensure(total);
-    vals.ensure(total);
-    hipLaunchKernelGGL(k_prim_emit, dim3(nblocks(n)), dim3(kBlock), 0, c.s, x, verts, n, nv, G, lgFlag.p, off, keys.p, vals.p);
-    CIPC_LAUNCH_CHECK();
-    radix_sort_pairs(keys.p, vals.p, total, bits_for((uint64_t)nCells), c.pw, c.s);
-    hipLaunchKernelGGL(k_cell_bounds, dim3(nblocks(total)), dim3(kBlock), 0, c.s, keys.p, total, start.p, end.p);
-    rec.ensure((size_t)8 * total);
-    hipLaunchKernelGGL(k_walk_records, dim3(nblocks(total)), dim3(kBlock), 0, c.s, (const uint32_t*)vals.p, total, (const int4*)box.p,
-                       (int4*)rec.p);
-    CIPC_LAUNCH_CHECK();
-    return total;
 }
 
 // ------------------------------------------------------------------ narrow phase
@@ -429,9 +412,9 @@ __device__ __forceinline__ void pe_codim_candidate(const O& o, const double* __r
 }
 __global__ void k_query_codim(const double* __restrict__ x, const int* __restrict__ bNode, int nBN, int codimBN0, int codimBN1,
                               const int* __restrict__ bEdge, int nBE, int nRod, const uint8_t* __restrict__ dbc, GridParams G,
-                              const uint32_t* __restrict__ estart, const uint32_t* __restrict__ eend, const uint32_t* __restrict__ evals,
+                              const uint32_t* __restrict__ estart, const int4* __restrict__ erec,
                               const int* __restrict__ lgListE, const uint32_t* __restrict__ lgCountE,
-                              const uint32_t* __restrict__ pstart, const uint32_t* __restrict__ pend, const uint32_t* __restrict__ pvals,
+                              const uint32_t* __restrict__ pstart, const int4* __restrict__ prec,
                               double dHat, double dHat2, int nV, CSOut out) {
     const WaveOut o{out};
     int s = codimBN0 + blockIdx.x * blockDim.x + threadIdx.x;
@@ -447,8 +430,9 @@ __global__ void k_query_codim(const double* __restrict__ x, const int* __restric
         for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
             for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
                 uint64_t cell = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
-                for (uint32_t k = estart[cell], e = eend[cell]; k < e; ++k) {
-                    const int eJ = (int)(evals[k] & kWalkId), first = (int)(evals[k] >> kWalkIdBits);
+                for (uint32_t k = estart[cell], e = estart[cell + 1]; k < e; ++k) {
+                    const uint32_t entry = (uint32_t)erec[2l * k + 1].z;
+                    const int eJ = (int)(entry & kWalkId), first = (int)(entry >> kWalkIdBits);
                     if (eJ < firstRod) continue;
                     if ((first | (ix == qlo[0] ? 1 : 0) | (iy == qlo[1] ? 2 : 0) | (iz == qlo[2] ? 4 : 0)) != 7) continue;
                     pe_codim_candidate(o, x, bEdge, nBE, dbc, vI, p, eJ, dHat, dHat2, nV);
@@ -465,8 +449,8 @@ __global__ void k_query_codim(const double* __restrict__ x, const int* __restric
         for (int iy = qlo[1]; iy <= qhi[1]; ++iy)
             for (int ix = qlo[0]; ix <= qhi[0]; ++ix) {
                 uint64_t cell = (uint64_t)ix + (uint64_t)G.dim[0] * ((uint64_t)iy + (uint64_t)G.dim[1] * (uint64_t)iz);
-                for (uint32_t k = pstart[cell], e = pend[cell]; k < e; ++k) {
-                    int sJ = codimBN1 + (int)(pvals[k] & kWalkId);
+                for (uint32_t k = pstart[cell], e = pstart[cell + 1]; k < e; ++k) {
+                    int sJ = codimBN1 + (int)((uint32_t)prec[2l * k + 1].z & kWalkId);
                     if (sJ <= s) continue;
                     int vJ = bNode[sJ];
                     if (dbc[vI] && dbc[vJ]) continue;
@@ -534,11 +518,18 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
 
     uint32_t* lgCountT = c.counters.p + 16;
     uint32_t* lgCountE = c.counters.p + 17;
-    build_cells(c, x, c.btri.p, c.nBT, 3, G, c.csBoxT, c.csRecT, c.k64a, c.u32c, c.cellStart, c.cellEnd, c.lgFlagT, c.lgListT, lgCountT);
-    build_cells(c, x, c.bEdge.p, c.nBE, 2, G, c.csBoxE, c.csRecE, c.k64b, c.u32d, c.ecellStart, c.ecellEnd, c.lgFlagE, c.lgListE, lgCountE);
-    if (c.nPart)
-        build_cells(c, x, c.partSlot.p, c.nPart, 1, G, c.csBoxP, c.csRecP, c.pKeys, c.pVals, c.pcellStart, c.pcellEnd, c.lgFlagP, c.lgListP,
-                    c.counters.p + 20);
+    uint32_t* lgCountP = c.counters.p + 18;
+    CIPC_HIP(hipMemsetAsync(lgCountT, 0, 3 * sizeof(uint32_t), c.s));
+    const CellBuild bt = {c.btri.p, c.nBT, 3, c.csBoxT, c.csRecT, c.cellStart, c.cellCount, c.lgFlagT, c.lgListT, lgCountT, c.hCnt + 8};
+    const CellBuild be = {c.bEdge.p, c.nBE, 2, c.csBoxE, c.csRecE, c.ecellStart, c.ecellCount, c.lgFlagE, c.lgListE, lgCountE, c.hCnt + 9};
+    const CellBuild bp = {c.partSlot.p, c.nPart, 1, c.csBoxP, c.csRecP, c.pcellStart, c.pcellCount, c.lgFlagP, c.lgListP, lgCountP, c.hCnt + 10};
+    cells_count(c, x, G, bt);
+    cells_count(c, x, G, be);
+    if (c.nPart) cells_count(c, x, G, bp);
+    CIPC_HIP(hipStreamSynchronize(c.s));   // the three totals
+    cells_emit(c, x, G, bt);
+    cells_emit(c, x, G, be);
+    if (c.nPart) cells_emit(c, x, G, bp);
 
     // narrow phase with capacity retry
     CSOut o;
@@ -552,9 +543,9 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
         o.dcnt = c.counters.p + 1;
         CIPC_HIP(hipMemsetAsync(c.counters.p, 0, 4 * sizeof(uint32_t), c.s));
         // point-triangle kept entries fill [0, cap), edge-edge kept entries [cap, 2 cap)
-        const CellGrid GT = {{G.dim[0], G.dim[1], G.dim[2]}, c.cellStart.p, c.cellEnd.p, (const int4*)c.csRecT.p, (const int4*)c.csBoxT.p,
+        const CellGrid GT = {{G.dim[0], G.dim[1], G.dim[2]}, c.cellStart.p, (const int4*)c.csRecT.p, (const int4*)c.csBoxT.p,
                              c.lgListT.p, lgCountT};
-        const CellGrid GE = {{G.dim[0], G.dim[1], G.dim[2]}, c.ecellStart.p, c.ecellEnd.p, (const int4*)c.csRecE.p, (const int4*)c.csBoxE.p,
+        const CellGrid GE = {{G.dim[0], G.dim[1], G.dim[2]}, c.ecellStart.p, (const int4*)c.csRecE.p, (const int4*)c.csBoxE.p,
                              c.lgListE.p, lgCountE};
         const QueryPT pt = {x, c.bNode.p, c.btri.p, c.nBT, c.dbc.p, G, dHat, dHat2, c.nV, {o, nullptr}, {}};
         hipLaunchKernelGGL(k_query_pt, dim3(walk_grid(c.nBN)), dim3(kBlock), 0, c.s, pt, c.nBN, GT);
@@ -566,9 +557,9 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
         CIPC_LAUNCH_CHECK();
         if (c.nBN > c.codimBN0) {
             hipLaunchKernelGGL(k_query_codim, dim3(nblocks(c.nBN - c.codimBN0)), dim3(kBlock), 0, c.s, x, c.bNode.p, c.nBN, c.codimBN0,
-                               c.codimBN1, c.bEdge.p, c.nBE, c.nRod, c.dbc.p, G, c.ecellStart.p, c.ecellEnd.p, c.u32d.p,
-                               c.lgListE.p, lgCountE, c.nPart ? c.pcellStart.p : c.ecellStart.p, c.nPart ? c.pcellEnd.p : c.ecellEnd.p,
-                               c.nPart ? c.pVals.p : c.u32d.p, dHat, dHat2, c.nV, o);
+                               c.codimBN1, c.bEdge.p, c.nBE, c.nRod, c.dbc.p, G, c.ecellStart.p, (const int4*)c.csRecE.p,
+                               c.lgListE.p, lgCountE, c.nPart ? c.pcellStart.p : c.ecellStart.p,
+                               (const int4*)(c.nPart ? c.csRecP.p : c.csRecE.p), dHat, dHat2, c.nV, o);
             CIPC_LAUNCH_CHECK();
         }
         CIPC_HIP(hipMemcpyAsync(c.hCnt, c.counters.p, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c.s));
@@ -584,11 +575,11 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
         uint32_t nUnique = 0;
         uint32_t* dpos = c.csPos.ensure((size_t)std::max<uint32_t>(nDup, 1) + 1);
         uint32_t* si = c.csIdx.ensure((size_t)std::max<uint32_t>(std::max(std::max(nPT, nEE), nDup), 1));
+        const uint64_t* dkey = nullptr;
         if (nDup) {
-            fill_iota(si, nDup, c.s);
-            radix_sort_pairs(o.dkey, si, nDup, bits_for((uint64_t)c.nV * c.nV * (c.nV + 1)), c.pw, c.s);
+            dkey = radix_sort_pairs(o.dkey, si, nDup, bits_for((uint64_t)c.nV * c.nV * (c.nV + 1)), c.pw, c.s, true).keys;
             uint32_t* h = c.csHead.ensure(nDup);
-            hipLaunchKernelGGL(k_run_flags, dim3(nblocks(nDup)), dim3(kBlock), 0, c.s, o.dkey, (int)nDup, h);
+            hipLaunchKernelGGL(k_run_flags, dim3(nblocks(nDup)), dim3(kBlock), 0, c.s, dkey, (int)nDup, h);
             CIPC_LAUNCH_CHECK();
             scan_exclusive(h, dpos, nDup, c.counters.p + 4, c.pw, c.s);
             CIPC_HIP(hipMemcpyAsync(c.hCnt + 4, c.counters.p + 4, sizeof(uint32_t), hipMemcpyDeviceToHost, c.s));
@@ -597,21 +588,19 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
         }
         int nC = (int)(nPT + nEE + nUnique);
         out.ensure((size_t)4 * std::max(nC, 1));
+        if (nDup) {   // before the next sort, which may reuse dkey's buffer
+            hipLaunchKernelGGL(k_run_emit, dim3(nblocks(nDup)), dim3(kBlock), 0, c.s, dkey, (int)nDup, dpos, out.p, nC,
+                               (int)(nPT + nEE), c.nV);
+            CIPC_LAUNCH_CHECK();
+        }
         if (nPT) {
-            fill_iota(si, nPT, c.s);
-            radix_sort_pairs(o.key, si, nPT, bits_for((uint64_t)c.nBN * c.nBT), c.pw, c.s);
-            hipLaunchKernelGGL(k_gather_c4, dim3(nblocks(nPT)), dim3(kBlock), 0, c.s, si, o.c4, (int)nPT, out.p, nC, 0);
+            const uint32_t* idx = radix_sort_pairs(o.key, si, nPT, bits_for((uint64_t)c.nBN * c.nBT), c.pw, c.s, true).vals;
+            hipLaunchKernelGGL(k_gather_c4, dim3(nblocks(nPT)), dim3(kBlock), 0, c.s, idx, o.c4, (int)nPT, out.p, nC, 0);
             CIPC_LAUNCH_CHECK();
         }
         if (nEE) {
-            fill_iota(si, nEE, c.s);
-            radix_sort_pairs(oEE.key, si, nEE, bits_for((uint64_t)c.nBE * c.nBE), c.pw, c.s);
-            hipLaunchKernelGGL(k_gather_c4, dim3(nblocks(nEE)), dim3(kBlock), 0, c.s, si, oEE.c4, (int)nEE, out.p, nC, (int)nPT);
-            CIPC_LAUNCH_CHECK();
-        }
-        if (nDup) {
-            hipLaunchKernelGGL(k_run_emit, dim3(nblocks(nDup)), dim3(kBlock), 0, c.s, o.dkey, (int)nDup, dpos, out.p, nC,
-                               (int)(nPT + nEE), c.nV);
+            const uint32_t* idx = radix_sort_pairs(oEE.key, si, nEE, bits_for((uint64_t)c.nBE * c.nBE), c.pw, c.s, true).vals;
+            hipLaunchKernelGGL(k_gather_c4, dim3(nblocks(nEE)), dim3(kBlock), 0, c.s, idx, oEE.c4, (int)nEE, out.p, nC, (int)nPT);
             CIPC_LAUNCH_CHECK();
         }
         nOut = nC;
@@ -1020,15 +1009,14 @@ void scatter_local_gradient(Ctx& c, const double* gl, const int* gv, long ns, do
     uint32_t* slot = c.u32c.ensure(ns);
     hipLaunchKernelGGL(k_grad_keys, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, gv, ns, c.nV, skip, key);
     CIPC_LAUNCH_CHECK();
-    fill_iota(slot, ns, c.s);
-    radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV + 1), c.pw, c.s);
+    const SortedPairs sorted = radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV + 1), c.pw, c.s, true);
     uint32_t* st = c.u32a.ensure(c.nV);
     uint32_t* en = c.u32b.ensure(c.nV);
     CIPC_HIP(hipMemsetAsync(st, 0, c.nV * sizeof(uint32_t), c.s));
     CIPC_HIP(hipMemsetAsync(en, 0, c.nV * sizeof(uint32_t), c.s));
-    hipLaunchKernelGGL(k_vert_bounds, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, key, ns, c.nV, st, en);
+    hipLaunchKernelGGL(k_vert_bounds, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, (const uint64_t*)sorted.keys, ns, c.nV, st, en);
     CIPC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_grad_gather, dim3(nblocks(c.nV)), dim3(kBlock), 0, c.s, gl, ns, slot, st, en, c.nV, g);
+    hipLaunchKernelGGL(k_grad_gather, dim3(nblocks(c.nV)), dim3(kBlock), 0, c.s, gl, ns, (const uint32_t*)sorted.vals, st, en, c.nV, g);
     CIPC_LAUNCH_CHECK();
 }
 
@@ -1118,11 +1106,11 @@ void barrier_hessian(Ctx& c, const double* x, const int* C, int nC, double kappa
         friction_hess_local(c, x, fricXn, hl, ns, 16l * nC);
         friction_hess_keys(c, key + 16l * nC);
     }
-    fill_iota(slot, ns, c.s);
-    radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV * c.nV + 1), c.pw, c.s);
+    const SortedPairs sorted = radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV * c.nV + 1), c.pw, c.s, true);
+    const uint64_t* skey = sorted.keys;
     uint32_t* head = c.u32a.ensure(ns);
     uint32_t* pos = c.u32b.ensure(ns);
-    hipLaunchKernelGGL(k_bsr_from_sorted, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, key, ns, c.nV, head);
+    hipLaunchKernelGGL(k_bsr_from_sorted, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, skey, ns, c.nV, head);
     CIPC_LAUNCH_CHECK();
     scan_exclusive(head, pos, ns, c.counters.p + 5, c.pw, c.s);
     CIPC_HIP(hipMemcpyAsync(c.hCnt + 5, c.counters.p + 5, sizeof(uint32_t), hipMemcpyDeviceToHost, c.s));
@@ -1133,7 +1121,7 @@ void barrier_hessian(Ctx& c, const double* x, const int* C, int nC, double kappa
     A.col.ensure(std::max(nnzb, 1));
     A.val.ensure(9l * std::max(nnzb, 1));
     A.rowptr.ensure(c.nV + 1);
-    hipLaunchKernelGGL(k_bsr_sum, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, key, ns, c.nV, pos, slot, hl, ns, proj_mask(c), nnzb,
+    hipLaunchKernelGGL(k_bsr_sum, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, skey, ns, c.nV, pos, (const uint32_t*)sorted.vals, hl, ns, proj_mask(c), nnzb,
                        A.rowOf.p, A.col.p, A.val.p);
     CIPC_LAUNCH_CHECK();
     hipLaunchKernelGGL(k_rowptr, dim3(nblocks(c.nV + 1)), dim3(kBlock), 0, c.s, A.rowOf.p, nnzb, c.nV, A.rowptr.p);

@@ -152,13 +152,12 @@ struct Ctx {
     std::vector<int> hTet, hBTri;
     DevBuf<int> tetIdx, btri;
     DevBuf<double> tetIB, tetVol;
-    DevBuf<uint64_t> pKeys;
-    DevBuf<uint32_t> pVals, pcellStart, pcellEnd;
+    DevBuf<uint32_t> pcellStart, pcellCount;
     DevBuf<uint8_t> lgFlagP;
     DevBuf<int> lgListP;
     DevBuf<int> ccdPlo, ccdPhi;
     DevBuf<int> ccdTbox, ccdEbox, ccdPbox;   // the same voxel boxes as 32-byte records (lo xyz, hi xyz, 2 pad)
-    DevBuf<int> ccdTrec, ccdErec;            // those records in cell order (third pad word = primitive)
+    DevBuf<int> ccdTrec, ccdErec, ccdPrec;            // those records in cell order (third pad word = primitive)
 
     // device state
     DevBuf<double> x, xn, xt, v, xprev, X0, mass, p, g, rhs;
@@ -182,7 +181,7 @@ struct Ctx {
     DevBuf<uint32_t> u32a, u32b, u32c, u32d, counters;
     DevBuf<uint64_t> k64a, k64b;
     DevBuf<int> i32a, i32b, i32c;
-    DevBuf<uint32_t> cellStart, cellEnd, ecellStart, ecellEnd;
+    DevBuf<uint32_t> cellStart, cellCount, ecellStart, ecellCount;   // cell lists: starts (one more than cells), counters
     uint32_t csCap = 1u << 16;
     DevBuf<uint64_t> csKey, csDKey;
     DevBuf<int> csC4;
@@ -330,7 +329,6 @@ struct Ctx {
 };
 
 // ---- utilities (util.hip)
-void fill_iota(uint32_t* a, long n, hipStream_t s);
 void bbox_minmax(Ctx& c, const double* x, double* out6);   // min xyz, max xyz into device memory
 void minmax6_final(const double* part, int nb, double* out6, hipStream_t s);   // reduce (lo, hi) records
 

@@ -86,9 +86,41 @@ __global__ void k_scan_apply(const uint32_t* __restrict__ in, uint32_t* __restri
     }
 }
 
+// up to kScanSmall values in one workgroup of 1024 threads, 16 consecutive values each: one
+// launch instead of three where the launches are the time
+constexpr int kScanSmall = 16384;
+__global__ __launch_bounds__(1024) void k_scan_small(const uint32_t* __restrict__ in, uint32_t* __restrict__ out, int n,
+                                                     uint32_t* __restrict__ total) {
+    __shared__ uint32_t lds[16];
+    const int base = 16 * threadIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t v[16], s = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = base + i < n ? in[base + i] : 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s += v[i];
+    const uint32_t inc = wave_incl_scan_u32(s);
+    if (lane == 63) lds[wid] = inc;
+    __syncthreads();
+    uint32_t run = inc - s;
+#pragma unroll
+    for (int w = 0; w < 16; ++w)
+        if (w < wid) run += lds[w];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        if (base + i < n) out[base + i] = run;
+        run += v[i];
+    }
+    if (total && threadIdx.x == 1023) *total = run;
+}
+
 void scan_exclusive(const uint32_t* in, uint32_t* out, long n, uint32_t* total, PrimWork& w, hipStream_t s) {
     if (n <= 0) {
         if (total) CIPC_HIP(hipMemsetAsync(total, 0, sizeof(uint32_t), s));
+        return;
+    }
+    if (n <= kScanSmall) {
+        hipLaunchKernelGGL(k_scan_small, dim3(1), dim3(1024), 0, s, in, out, (int)n, total);
+        CIPC_LAUNCH_CHECK();
         return;
     }
     int nb = (int)((n + SCAN_TILE - 1) / SCAN_TILE);
@@ -101,90 +133,144 @@ void scan_exclusive(const uint32_t* in, uint32_t* out, long n, uint32_t* total, 
     CIPC_LAUNCH_CHECK();
 }
 
-// ------------------------------------------------------------------ radix sort
+// ------------------------------------------------------------------ sort
+// Least-significant-digit radix sort, digits of up to kMaxDigit bits: the key's bits are
+// split evenly, so 18 bits take two passes and 35 bits four (three and five with 8-bit
+// digits); the passes' launches and their scans are the time on all but the largest inputs.
 constexpr int RS_ITEMS = 8;
 constexpr int RS_TILE = kBlock * RS_ITEMS;
+constexpr int kMaxDigit = 9, kBins = 1 << kMaxDigit, kBinsPer = kBins / kBlock;
 
-__global__ void k_rs_hist(const uint64_t* __restrict__ keys, long n, int shift, uint32_t* __restrict__ hist, int nb) {
-    __shared__ uint32_t h[256];
-    h[threadIdx.x] = 0;
+__global__ void k_rs_hist(const uint64_t* __restrict__ keys, long n, int shift, uint32_t mask, uint32_t* __restrict__ hist, int nb) {
+    __shared__ uint32_t h[kBins];
+#pragma unroll
+    for (int k = 0; k < kBinsPer; ++k) h[threadIdx.x + k * kBlock] = 0;
     __syncthreads();
     long base = (long)blockIdx.x * RS_TILE;
 #pragma unroll
     for (int i = 0; i < RS_ITEMS; ++i) {
         long idx = base + (long)i * kBlock + threadIdx.x;
-        if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
+        if (idx < n) atomicAdd(&h[(uint32_t)(keys[idx] >> shift) & mask], 1u);
     }
     __syncthreads();
-    hist[(long)threadIdx.x * nb + blockIdx.x] = h[threadIdx.x];
+#pragma unroll
+    for (int k = 0; k < kBinsPer; ++k) {
+        const uint32_t d = threadIdx.x + k * kBlock;
+        if (d <= mask) hist[(long)d * nb + blockIdx.x] = h[d];
+    }
 }
 
+// vin == nullptr: the values are the positions 0, 1, ...
 __global__ void k_rs_scatter(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                             uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, long n, int shift,
+                             uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, long n, int shift, int digitBits,
                              const uint32_t* __restrict__ histScan, int nb) {
-    __shared__ uint32_t gbase[256];
-    __shared__ uint32_t run[256];
-    __shared__ uint32_t wcnt[4][256];
+    __shared__ uint32_t next[kBins];         // output position of the digit's next key
+    __shared__ uint32_t wcnt[4][kBins];
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
-    gbase[tid] = histScan[(long)tid * nb + blockIdx.x];
-    run[tid] = 0;
+    const uint32_t mask = (1u << digitBits) - 1;
+#pragma unroll
+    for (int k = 0; k < kBinsPer; ++k) {
+        const uint32_t d = tid + k * kBlock;
+        next[d] = d <= mask ? histScan[(long)d * nb + blockIdx.x] : 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) wcnt[w][d] = 0;
+    }
     const uint64_t ltmask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     long base = (long)blockIdx.x * RS_TILE;
+    uint64_t key[RS_ITEMS];
+    uint32_t val[RS_ITEMS];
+#pragma unroll
     for (int r = 0; r < RS_ITEMS; ++r) {
-        long idx = base + (long)r * kBlock + tid;
-        bool valid = idx < n;
-        uint64_t key = valid ? kin[idx] : 0;
-        uint32_t val = valid ? vin[idx] : 0;
-        uint32_t dig = (uint32_t)((key >> shift) & 255u);
+        const long idx = base + (long)r * kBlock + tid;
+        key[r] = idx < n ? kin[idx] : 0;
+        val[r] = idx < n ? (vin ? vin[idx] : (uint32_t)idx) : 0;
+    }
+    __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 4; ++k) wcnt[k][tid] = 0;
-        __syncthreads();
+    for (int r = 0; r < RS_ITEMS; ++r) {
+        const bool valid = base + (long)r * kBlock + tid < n;
+        const uint32_t dig = (uint32_t)(key[r] >> shift) & mask;
         uint64_t peers = __ballot(valid);
-#pragma unroll
-        for (int b = 0; b < 8; ++b) {
+        for (int b = 0; b < digitBits; ++b) {
             uint64_t m = __ballot((dig >> b) & 1u);
             peers &= ((dig >> b) & 1u) ? m : ~m;
         }
-        uint32_t rankInWave = (uint32_t)__popcll(peers & ltmask);
+        const uint32_t rankInWave = (uint32_t)__popcll(peers & ltmask);
         if (valid && rankInWave == 0) wcnt[wid][dig] = (uint32_t)__popcll(peers);
         __syncthreads();
         if (valid) {
-            uint32_t off = run[dig];
-            for (int k = 0; k < wid; ++k) off += wcnt[k][dig];
-            uint32_t dst = gbase[dig] + off + rankInWave;
-            kout[dst] = key;
-            vout[dst] = val;
+            uint32_t dst = next[dig] + rankInWave;
+            for (int k = 0; k < wid; ++k) dst += wcnt[k][dig];
+            kout[dst] = key[r];
+            vout[dst] = val[r];
         }
         __syncthreads();
-        run[tid] += wcnt[0][tid] + wcnt[1][tid] + wcnt[2][tid] + wcnt[3][tid];
+#pragma unroll
+        for (int k = 0; k < kBinsPer; ++k) {
+            const uint32_t d = tid + k * kBlock;
+            next[d] += (wcnt[0][d] + wcnt[1][d]) + (wcnt[2][d] + wcnt[3][d]);
+#pragma unroll
+            for (int w = 0; w < 4; ++w) wcnt[w][d] = 0;
+        }
         __syncthreads();
     }
 }
 
-void radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, PrimWork& w, hipStream_t s) {
-    if (n <= 1) return;
-    int nb = (int)((n + RS_TILE - 1) / RS_TILE);
+// Short inputs by counting: an element's place is the number of smaller keys plus the equal
+// ones before it.  64 elements per workgroup, each of its four waves compares them with a
+// quarter of the keys (uniform addresses: scalar loads); one launch instead of five per
+// digit.  kRankSort: from there on the quadratic work is longer than the passes of 20-bit
+// keys, the shortest in use (us, counting / passes of 20 bits / of 40 bits: 2,000 keys 13.5 /
+// 36.8 / 63, 8,000 keys 41.4 / 42.0 / 74, 16,000 keys 79 / 43 / 80).
+constexpr int kRankSort = 8192;
+__global__ __launch_bounds__(kBlock) void k_rank_sort(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
+                                                      uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, int n) {
+    __shared__ uint32_t part[4][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int first = blockIdx.x * 64, i = first + lane;
+    const uint64_t mine = i < n ? kin[i] : 0;
+    const int per = (n + 3) / 4, j0 = w * per, j1 = min(n, j0 + per);
+    // keys before this workgroup's count when not larger, keys behind it when smaller
+    uint32_t r = 0;
+    const int a = min(max(first, j0), j1), b = min(max(first + 64, j0), j1);
+#pragma unroll 8
+    for (int j = j0; j < a; ++j) r += kin[j] <= mine;
+    for (int j = a; j < b; ++j) r += kin[j] < mine || (kin[j] == mine && j < i);
+#pragma unroll 8
+    for (int j = b; j < j1; ++j) r += kin[j] < mine;
+    part[w][lane] = r;
+    __syncthreads();
+    if (w != 0 || i >= n) return;
+    r = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    kout[r] = mine;
+    vout[r] = vin ? vin[i] : (uint32_t)i;
+}
+
+SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, PrimWork& w, hipStream_t s, bool iota) {
+    if (n <= 0) return {keys, vals};
     uint64_t* k2 = w.keyAlt.ensure(n);
     uint32_t* v2 = w.valAlt.ensure(n);
-    uint32_t* hist = w.hist.ensure((size_t)256 * nb);
-    uint32_t* hs = w.histScan.ensure((size_t)256 * nb);
+    if (n <= kRankSort) {
+        hipLaunchKernelGGL(k_rank_sort, dim3((unsigned)((n + 63) / 64)), dim3(kBlock), 0, s, keys, iota ? nullptr : vals, k2, v2, (int)n);
+        CIPC_LAUNCH_CHECK();
+        return {k2, v2};
+    }
+    int nb = (int)((n + RS_TILE - 1) / RS_TILE);
+    const int passes = (bits + kMaxDigit - 1) / kMaxDigit, rb = (bits + passes - 1) / passes;
+    uint32_t* hist = w.hist.ensure((size_t)nb << rb);
+    uint32_t* hs = w.histScan.ensure((size_t)nb << rb);
     uint64_t *ka = keys, *kb = k2;
     uint32_t *va = vals, *vb = v2;
-    int passes = (bits + 7) / 8;
     for (int p = 0; p < passes; ++p) {
-        int shift = 8 * p;
-        hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(kBlock), 0, s, ka, n, shift, hist, nb);
+        hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(kBlock), 0, s, ka, n, rb * p, (1u << rb) - 1, hist, nb);
         CIPC_LAUNCH_CHECK();
-        scan_exclusive(hist, hs, (long)256 * nb, nullptr, w, s);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(kBlock), 0, s, ka, va, kb, vb, n, shift, hs, nb);
+        scan_exclusive(hist, hs, (long)nb << rb, nullptr, w, s);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(kBlock), 0, s, ka, p == 0 && iota ? nullptr : va, kb, vb, n, rb * p, rb, hs, nb);
         CIPC_LAUNCH_CHECK();
         std::swap(ka, kb);
         std::swap(va, vb);
     }
-    if (ka != keys) {
-        CIPC_HIP(hipMemcpyAsync(keys, ka, n * sizeof(uint64_t), hipMemcpyDeviceToDevice, s));
-        CIPC_HIP(hipMemcpyAsync(vals, va, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, s));
-    }
+    return {ka, va};
 }
 
 // ------------------------------------------------------------------ reductions

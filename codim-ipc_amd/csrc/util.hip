@@ -1,17 +1,7 @@
-// Small device utilities: index fill, bounding box.
+// Small device utilities: bounding box.
 #include "ctx.hpp"
 
 namespace cipc {
-
-__global__ void k_iota(uint32_t* __restrict__ a, long n) {
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = (uint32_t)i;
-}
-void fill_iota(uint32_t* a, long n, hipStream_t s) {
-    if (n <= 0) return;
-    hipLaunchKernelGGL(k_iota, dim3(nblocks(n)), dim3(kBlock), 0, s, a, n);
-    CIPC_LAUNCH_CHECK();
-}
 
 __global__ void k_bbox_partial(const double* __restrict__ x, int nV, double* __restrict__ part) {
     __shared__ double lo[3][kBlock], hi[3][kBlock];

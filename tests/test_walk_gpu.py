@@ -40,6 +40,19 @@ def test_constraint_set_equals_oracle_for_every_cell_size(require_gpu, name, cel
     sim.close()
 
 
+# short sets are sorted by counting and long ones by digits, short runs of cells are summed
+# by one workgroup: 4,600 to 25,000 constraints lie on both sides of both lines
+@pytest.mark.parametrize("n", [14, 18, 20, 30])
+def test_constraint_set_order_below_and_above_the_short_sorts(require_gpu, n):
+    sd = scenes.cloth_on_sphere(sheets=3, n=n, y0=0.2008, dy=0.0008, sphere_level=1, seed=2, twists=[0.0, 5.0, 10.0])
+    sd.X[:sd.n_cloth, 0] *= 0.03 * n / 14
+    sd.X[:sd.n_cloth, 2] *= 0.03 * n / 14
+    sim = Simulator(sd)
+    got = sim.constraint_set(sd.X.ravel())
+    sim.close()
+    assert np.array_equal(got, O.OracleScene(sd, threads=2).constraint_set(sd.X.ravel()))
+
+
 @pytest.mark.parametrize("name", ["tiny", "dense", "ground", "codim"])
 def test_ccd_step_equals_oracle(require_gpu, name):
     sd = scene(name)
