@@ -198,7 +198,7 @@ struct Ctx {
     BSR Ael;
     DevBuf<int> planOff, planSlot;     // per BSR block: list of local block slots
     DevBuf<double> elLocal;            // local 3x3 blocks, [nSlots][9]
-    DevBuf<double> hingeH;             // hinge Hessians before projection, [nH][12][12]
+    DevBuf<double> hingeH;             // reduced hinge Hessians before projection, [45][nH]
     int nElSlots = 0, nTriSlots = 0;
     DevBuf<int> gplanOff, gplanSlot;   // per vertex: gradient slots (tri 3 per, hinge 4 per)
     DevBuf<double> gLocal;             // local gradient 3-vectors, [nGSlots][3]
@@ -206,9 +206,7 @@ struct Ctx {
 
     // contact Hessian (rebuilt per Newton iteration)
     BSR Acon;
-    DevBuf<double> conLocal;           // SoA [9][16 nC]
-    DevBuf<double> conH;               // local barrier Hessians before projection, [nC][12][12]
-    DevBuf<int> conNv;                 // vertices of each constraint's Hessian (0: not evaluated)
+    DevBuf<double> conLocal;           // local 3x3 blocks of contacts and friction, [slot][9]
     DevBuf<int> conPlanSlot;           // sorted slot order
     DevBuf<double> conGLocal;          // SoA [3][4 nC]
     DevBuf<int> conGVert;              // vertex of each gradient slot (4 nC; -1 unused)
@@ -347,7 +345,7 @@ void scatter_local_gradient(Ctx& c, const double* gl, const int* gv, long ns, do
 void friction_basis(Ctx& c, const double* x, const int* C, int nC, double kappa);
 double friction_energy(Ctx& c, const double* x, const double* xn);
 void friction_gradient(Ctx& c, const double* x, const double* xn, double* g, const uint8_t* skip = nullptr);   // g +=
-void friction_hess_local(Ctx& c, const double* x, const double* xn, double* hl, long ns, long off);
+void friction_hess_local(Ctx& c, const double* x, const double* xn, double* hl, long off);
 void friction_hess_keys(Ctx& c, uint64_t* key);
 // weight of the shell's membrane, bending, strain-limit and fibre terms: h^2, or 1 in a
 // static solve (staticSolve ? 1.0 : h in the reference; rods and tets keep h^2)

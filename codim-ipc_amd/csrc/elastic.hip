@@ -300,12 +300,17 @@ __global__ void __launch_bounds__(64) k_memb_hess_local(const double* __restrict
 }
 // Hinge Hessians in two kernels, so that the register-hungry row evaluation and the
 // eigensolver each run at their own occupancy (Math/UTILS.h:10-27 for the projection).
-// Stage 1: the symmetrised, scaled hinge Hessian, row r by lane r, into H[144 h + 12 r + c]
-// (zero for inactive hinges).
+// Stage 1: the symmetrised, scaled hinge Hessian (zero for inactive hinges), row r by lane
+// r of 16, and from it in LDS the reduced matrix: the dihedral energy is invariant under
+// translations, so H (x + t) = 0 for every rigid translation t = (u, u, u, u), and with the
+// orthonormal basis Q = Wq (x) I3 of the translation complement (tr_basis<4>: the three
+// +-1/2 patterns orthogonal to (1, 1, 1, 1)) the projection is H+ = Q proj(Q^T H Q) Q^T.
+// H9 = Q^T H Q goes out as its 45 upper entries, entry e of hinge h at H9[e nH + h].
 __global__ void __launch_bounds__(256) k_bend_hess_rows(const double* __restrict__ x, const int* __restrict__ hg, int nH,
                                                         const double* __restrict__ hi, double kb, double h2,
-                                                        const uint8_t* __restrict__ dbc, double* __restrict__ H) {
+                                                        const uint8_t* __restrict__ dbc, double* __restrict__ H9) {
     __shared__ double sh[16][144];
+    __shared__ double red[45][17];
     const int grp = threadIdx.x >> 4, r = threadIdx.x & 15;
     const int h = blockIdx.x * 16 + grp;
     const bool live = h < nH;
@@ -332,108 +337,42 @@ __global__ void __launch_bounds__(256) k_bend_hess_rows(const double* __restrict
     double gr = 0;
 #pragma unroll
     for (int c = 0; c < 12; ++c) gr = (c == r) ? g[c] : gr;
-    if (live && r < 12)
+    if (r < 12)
 #pragma unroll
-        for (int c = 0; c < 12; ++c) H[144l * h + 12 * r + c] = s1 * (0.5 * (M[r * 12 + c] + M[c * 12 + r])) + s2 * gr * g[c];
-}
-// Stage 2, one hinge per thread: the dihedral energy is invariant under translations, so
-// H (x + t) = 0 for every rigid translation t = (u, u, u, u), and with the orthonormal
-// basis Q = Wq (x) I3 of the translation complement (Wq: the three +-1/2 patterns
-// orthogonal to (1, 1, 1, 1)) the projection is H+ = Q proj(Q^T H Q) Q^T.  The 9x9
-// problem fits in registers (45 upper entries + 81 eigenvector entries): cyclic Jacobi,
-// fully unrolled over the 36 pairs of a sweep, stopping at off^2 <= 1e-24 ||H9||_F^2.
-__device__ __forceinline__ constexpr int u9(int i, int j) { return i <= j ? i * 9 - i * (i - 1) / 2 + (j - i) : j * 9 - j * (j - 1) / 2 + (i - j); }
-__device__ __forceinline__ constexpr int wsign(int k, int a) {
-    // Wq[k][a] = wsign / 2: columns (+,-,+,-), (+,+,-,-), (+,-,-,+)
-    return a == 0 ? ((k & 1) ? -1 : 1) : a == 1 ? ((k >> 1) ? -1 : 1) : (((k & 1) ^ (k >> 1)) ? -1 : 1);
-}
-__global__ void __launch_bounds__(64) k_bend_hess_proj9(const double* __restrict__ H, int nH, double* __restrict__ hl, long off) {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= nH) return;
-    const double* Hh = H + 144l * h;
-    // H9 = Q^T H Q, upper triangle: block (a, b), entry (i, j) = 1/4 sum_kl s_ka s_lb H[3k+i][3l+j]
-    double a9[45];
+        for (int c = 0; c < 12; ++c) A[c] = s1 * (0.5 * (M[r * 12 + c] + M[c * 12 + r])) + s2 * gr * g[c];
+    __syncthreads();
+    if (r < 12)
 #pragma unroll
-    for (int e = 0; e < 45; ++e) a9[e] = 0.0;
+        for (int c = 0; c < 12; ++c) M[r * 12 + c] = A[c];
+    __syncthreads();
+    for (int e = r; e < 45; e += 16) {
+        int R = 0, C = e;   // upper entry e in row order
+        while (C >= 9 - R) { C -= 9 - R; ++R; }
+        C += R;
+        const int a = R / 3, i = R - 3 * a, b = C / 3, j = C - 3 * b;
+        double sum = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < 4; ++k)
 #pragma unroll
-        for (int l = 0; l < 4; ++l)
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-#pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    const double v = 0.25 * Hh[(3 * k + i) * 12 + 3 * l + j];
-#pragma unroll
-                    for (int a = 0; a < 3; ++a)
-#pragma unroll
-                        for (int b = 0; b < 3; ++b) {
-                            const int R = 3 * a + i, C = 3 * b + j;
-                            if (R <= C) a9[u9(R, C)] += (wsign(k, a) * wsign(l, b) > 0) ? v : -v;
-                        }
-                }
-    double V[81];
-#pragma unroll
-    for (int e = 0; e < 81; ++e) V[e] = (e % 10 == 0) ? 1.0 : 0.0;
-    double fro = 0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-        for (int j = i; j < 9; ++j) fro += (i == j ? 1.0 : 2.0) * a9[u9(i, j)] * a9[u9(i, j)];
-    const double tol = 1e-24 * fro;
-    for (int sweep = 0; sweep < 16; ++sweep) {
-        double offd = 0;
-#pragma unroll
-        for (int i = 0; i < 9; ++i)
-#pragma unroll
-            for (int j = i + 1; j < 9; ++j) offd += a9[u9(i, j)] * a9[u9(i, j)];
-        if (offd <= 0.5 * tol) break;   // off^2 of the full matrix is twice the upper sum
-#pragma unroll
-        for (int p = 0; p < 8; ++p)
-#pragma unroll
-            for (int q = p + 1; q < 9; ++q) {
-                const double apq = a9[u9(p, q)];
-                if (apq == 0.0) continue;
-                const double app = a9[u9(p, p)], aqq = a9[u9(q, q)];
-                const double theta = (aqq - app) / (2 * apq);
-                const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1));
-                const double c = 1 / sqrt(t * t + 1), s = t * c;
-                a9[u9(p, p)] = app - t * apq;
-                a9[u9(q, q)] = aqq + t * apq;
-                a9[u9(p, q)] = 0.0;
-#pragma unroll
-                for (int k = 0; k < 9; ++k) {
-                    if (k == p || k == q) continue;
-                    const double akp = a9[u9(k, p)], akq = a9[u9(k, q)];
-                    a9[u9(k, p)] = c * akp - s * akq;
-                    a9[u9(k, q)] = s * akp + c * akq;
-                }
-#pragma unroll
-                for (int k = 0; k < 9; ++k) {
-                    const double vkp = V[9 * k + p], vkq = V[9 * k + q];
-                    V[9 * k + p] = c * vkp - s * vkq;
-                    V[9 * k + q] = s * vkp + c * vkq;
-                }
-            }
+            for (int l = 0; l < 4; ++l) sum += (tr_basis<4>(k, a) * tr_basis<4>(l, b)) * M[(3 * k + i) * 12 + 3 * l + j];
+        red[e][grp] = sum;
     }
-    // H9+ = V diag(max(lambda, 0)) V^T (upper), reusing a9
-    double lam[9];
+    __syncthreads();
+    for (int o = threadIdx.x; o < 45 * 16; o += 256) {
+        const int e = o >> 4, hh = blockIdx.x * 16 + (o & 15);
+        if (hh < nH) H9[(long)e * nH + hh] = red[e][o & 15];
+    }
+}
+// Stage 2, one hinge per thread: the positive part of the 9x9 reduced matrix in registers
+// and its expansion to the hinge's 16 local 3x3 blocks.
+__global__ void __launch_bounds__(64) k_bend_hess_proj9(const double* __restrict__ H9, int nH, double* __restrict__ hl, long off) {
+    __shared__ double lds[kEmitLds];
+    const int h0 = blockIdx.x * 64, h = h0 + threadIdx.x;
+    double a[45];
 #pragma unroll
-    for (int i = 0; i < 9; ++i) lam[i] = a9[u9(i, i)] > 0 ? a9[u9(i, i)] : 0.0;
-#pragma unroll
-    for (int i = 0; i < 9; ++i)
-#pragma unroll
-        for (int j = i; j < 9; ++j) {
-            double sum = 0;
-#pragma unroll
-            for (int m = 0; m < 9; ++m) sum += V[9 * i + m] * lam[m] * V[9 * j + m];
-            a9[u9(i, j)] = sum;
-        }
-    // H+ = Q H9+ Q^T: block (k, l), entry (i, j) = 1/4 sum_ab s_ka s_lb H9+[3a+i][3b+j],
-    // written as the hinge's 16 local 3x3 blocks
-    double* dst = hl + 9 * (off + 16l * h);
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
+    for (int e = 0; e < 45; ++e) a[e] = h < nH ? H9[(long)e * nH + h] : 0.0;
+    jacobi_psd<9, 9, false>(a);
+    emit_blocks(4, nH - h0, lds, hl + 9 * (off + 16l * h0), [&](int k, double* row) {
 #pragma unroll
         for (int l = 0; l < 4; ++l)
 #pragma unroll
@@ -442,14 +381,15 @@ __global__ void __launch_bounds__(64) k_bend_hess_proj9(const double* __restrict
                 for (int j = 0; j < 3; ++j) {
                     double sum = 0;
 #pragma unroll
-                    for (int a = 0; a < 3; ++a)
+                    for (int p = 0; p < 3; ++p)
 #pragma unroll
-                        for (int b = 0; b < 3; ++b) {
-                            const double v = a9[u9(3 * a + i, 3 * b + j)];
-                            sum += (wsign(k, a) * wsign(l, b) > 0) ? v : -v;
+                        for (int q = 0; q < 3; ++q) {
+                            const double v = a[upk(9, 3 * p + i, 3 * q + j)];
+                            sum += tr_basis<4>(k, p) * tr_basis<4>(l, q) > 0 ? v : -v;
                         }
-                    dst[9 * (4 * k + l) + 3 * i + j] = 0.25 * sum;
+                    row[9 * l + 3 * i + j] = 0.25 * sum;
                 }
+    });
 }
 
 // rod segment s block (a, b) at off + 4 s + 2 a + b; rod hinge h block (a, b) at
@@ -518,7 +458,7 @@ void elastic_hessian(Ctx& c, const double* x) {
     }
     if (c.nH) {
         double kb = c.P.bendMult != 0 ? c.kBend : 0.0;
-        double* Hh = c.hingeH.ensure(144 * (size_t)c.nH);
+        double* Hh = c.hingeH.ensure(45 * (size_t)c.nH);
         hipLaunchKernelGGL(k_bend_hess_rows, dim3((c.nH + 15) / 16), dim3(256), 0, c.s, x, c.hinge.p, c.nH, c.hInfo.p, kb, h2, c.dbc.p, Hh);
         hipLaunchKernelGGL(k_bend_hess_proj9, dim3(nblocks(c.nH, 64)), dim3(64), 0, c.s, (const double*)Hh, c.nH, hl, 9l * c.nT);
         CIPC_LAUNCH_CHECK();

@@ -208,7 +208,7 @@ __global__ void k_fric_grad_local(const double* __restrict__ x, const double* __
 
 // Hessian blocks of stencil i at slots off + 16 i + 4 a + b of the SoA [9][ns] array
 __global__ void k_fric_hess_local(const double* __restrict__ x, const double* __restrict__ xn, const int* __restrict__ fC,
-                                  const double* __restrict__ fI, int nF, double ev, double mu, double* __restrict__ hl, long ns,
+                                  const double* __restrict__ fI, int nF, double ev, double mu, double* __restrict__ hl,
                                   long off) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= nF) return;
@@ -255,7 +255,7 @@ __global__ void k_fric_hess_local(const double* __restrict__ x, const double* __
         for (int b = 0; b < 4; ++b) {
             const double cab = (a < E.s.nv && b < E.s.nv) ? E.s.coef[a] * E.s.coef[b] : 0.0;
 #pragma unroll
-            for (int e = 0; e < 9; ++e) hl[(long)e * ns + base + 4 * a + b] = cab * K[e];
+            for (int e = 0; e < 9; ++e) hl[9 * (base + 4 * a + b) + e] = cab * K[e];
         }
 }
 
@@ -323,10 +323,10 @@ void friction_gradient(Ctx& c, const double* x, const double* xn, double* g, con
     scatter_local_gradient(c, gl, gv, ns, g, skip);
 }
 
-void friction_hess_local(Ctx& c, const double* x, const double* xn, double* hl, long ns, long off) {
+void friction_hess_local(Ctx& c, const double* x, const double* xn, double* hl, long off) {
     if (c.nF == 0) return;
     hipLaunchKernelGGL(k_fric_hess_local, dim3(nblocks(c.nF)), dim3(kBlock), 0, c.s, x, xn, c.fC.p, c.fI.p, c.nF, fric_ev(c),
-                       fric_mu(c), hl, ns, off);
+                       fric_mu(c), hl, off);
     CIPC_LAUNCH_CHECK();
 }
 
