@@ -636,8 +636,7 @@ bool coarse_prepare(Ctx& c, const double* x) {
     CIPC_LAUNCH_CHECK();
     // a pivot below 1e-9 of its diagonal is a mode the matrix does not see (one vertex,
     // or collinear members: rotation about their line)
-    dense_cholesky(c, g.A.p, g.npad, g.flag.p, g.tileInv.p, g.diag0.p, g.dropped.p, 1e-9);
-    dense_lower_inverse(c, g.A.p, g.W.p, g.npad, g.tileInv.p);
+    dense_cholesky(c, g.A.p, g.npad, g.flag.p, g.tileInv.p, g.diag0.p, g.dropped.p, 1e-9, g.W.p);
     const int nt = g.npad / kCgTile;
     if (g.bf16) {
         g.W16.ensure_exact((size_t)g.npad * g.npad);

@@ -397,9 +397,7 @@ int direct_solve(Ctx& c, const double* b, double* x);
 // panels by substitution.  With diag0 / dropped: a pivot below tau x its original
 // diagonal is dropped (pivot at that scale, zero column) and flagged instead.
 void dense_cholesky(Ctx& c, double* A, int npad, int* bad, double* tileInv, const double* diag0 = nullptr, int* dropped = nullptr,
-                    double tau = 0);
-// W = L^-1 of a dense_cholesky factor whose diagonal-tile inverses are in tileInv
-void dense_lower_inverse(Ctx& c, const double* L, double* W, int npad, const double* tileInv);
+                    double tau = 0, double* W = nullptr);
 // two-level correction (coarse.hip)
 bool coarse_prepare(Ctx& c, const double* x);            // aggregates (once), Galerkin matrix, factor; false: unavailable
 template <class V>

@@ -116,10 +116,9 @@ struct TileRegs {
 // tile is written there too.  Every sum runs in a fixed order: trailing updates in
 // column order, substitution sums in index order.
 static_assert(kDirectBlock == 4 * kDT, "the tile factor runs four waves of one lane per row");
-__global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict__ a, long ld, int k, int* __restrict__ bad,
-                                                             const double* __restrict__ diag0, int* __restrict__ dropped, double tau,
-                                                             double* __restrict__ inv) {
-    __shared__ double T[kDT][kDT + 1];
+__device__ __forceinline__ void potrf_tile(double* a, long ld, int k, int* __restrict__ bad, const double* __restrict__ diag0,
+                                           int* __restrict__ dropped, double tau, double* __restrict__ inv, double (*T)[kDT + 1],
+                                           double (*X)[kDT + 1], double* rd) {
     const int tid = threadIdx.x, i = tid & 63, h = tid >> 6;
     const long o = (long)k * kDT;
     const double dg0 = diag0 ? diag0[o + i] : 0.0;
@@ -179,8 +178,6 @@ __global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict_
         // sum_{m<r} L[r][m] X[m]) / L[r][r] with the sum taken in m order, quarter by
         // quarter: wave s finishes its rows, then the later waves add their terms
         // from them
-        __shared__ double X[kDT][kDT + 1];
-        __shared__ double rd[kDT];
         if (h == 0) rd[i] = 1.0 / T[i][i];
         __syncthreads();
         double sacc[16];
@@ -212,6 +209,14 @@ __global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict_
 #pragma unroll
         for (int q = 0; q < 16; ++q) dst[(4 * q + h) * kDT + i] = X[4 * q + h][i];
     }
+}
+__global__ __launch_bounds__(kDirectBlock) void k_potrf_tile(double* __restrict__ a, long ld, int k, int* __restrict__ bad,
+                                                             const double* __restrict__ diag0, int* __restrict__ dropped, double tau,
+                                                             double* __restrict__ inv) {
+    __shared__ double T[kDT][kDT + 1];
+    __shared__ double X[kDT][kDT + 1];
+    __shared__ double rd[kDT];
+    potrf_tile(a, ld, k, bad, diag0, dropped, tau, inv, T, X, rd);
 }
 
 // panel: tiles (i, k), i > k, become A_ik L_kk^-T (each row solved forward against L_kk);
@@ -330,82 +335,83 @@ __device__ __forceinline__ void tile_update(double* __restrict__ C, long ldc, co
             }
 }
 
-// trailing update of the lower tiles (i, j), k < j <= i: A_ij -= L_ik L_jk^T; block b
-// enumerates the lower triangle of the trailing tile matrix row by row
-__global__ __launch_bounds__(kDirectBlock) void k_syrk_tiles(double* __restrict__ a, long ld, int k, int nt) {
+// One step k of the factorisation, after the diagonal tile, is two launches.
+// Panel: tiles (i, k), i > k, by product with the inverted diagonal tile, A_ik <- A_ik
+// inv(L_kk)^T, columns of dropped pivots zero.  When the inverse W = L^-1 is wanted (blocked
+// forward substitution on the identity, right-looking), the next blocks take its row k at
+// the same time: W_kj = inv(L_kk) W_kj, j <= k.
+__global__ __launch_bounds__(kDirectBlock) void k_panel_tiles(double* __restrict__ a, long ld, int k, int m, const double* __restrict__ inv,
+                                                             const int* __restrict__ dropped, double* __restrict__ W) {
     __shared__ double Pt[kDT][kDTLd];
     __shared__ double Qt[kDT][kDTLd];
-    const int m = nt - k - 1;
-    int b = blockIdx.x, ii = 0;
-    while (b >= ii + 1) { b -= ii + 1; ++ii; }   // row ii of the trailing triangle holds ii + 1 tiles
-    if (ii >= m) return;
-    const int i = k + 1 + ii, j = k + 1 + b;
-    const long ok = (long)k * kDT, oi = (long)i * kDT, oj = (long)j * kDT;
-    tile_update<true>(a + oi * ld + oj, ld, a + oi * ld + ok, ld, a + oj * ld + ok, ld, Pt, Qt, false);
+    const long ok = (long)k * kDT;
+    const double* Ikk = inv + (long)k * kDT * kDT;
+    if ((int)blockIdx.x < m) {
+        double* Aik = a + (long)(k + 1 + blockIdx.x) * kDT * ld + ok;
+        tile_update<true>(Aik, ld, Aik, ld, Ikk, kDT, Pt, Qt, true, dropped ? dropped + ok : nullptr);
+    } else {
+        double* Wkj = W + ok * ld + (long)((int)blockIdx.x - m) * kDT;
+        tile_update<false>(Wkj, ld, Ikk, kDT, Wkj, ld, Pt, Qt, true);
+    }
 }
-
-// panel by product with the inverted diagonal tile: A_ik <- A_ik inv(L_kk)^T, columns of
-// dropped pivots zero
-__global__ __launch_bounds__(kDirectBlock) void k_panel_tiles(double* __restrict__ a, long ld, int k, const double* __restrict__ inv,
-                                                             const int* __restrict__ dropped) {
+// Trailing update of the lower tiles (i, j), k < j <= i: A_ij -= L_ik L_jk^T; block b
+// enumerates the lower triangle of the trailing tile matrix row by row.  Block 0 has the next
+// diagonal tile and factors it at once: the tile factor is one workgroup's serial chain, and
+// as a launch of its own the chip waited for it in every step.  The blocks after the
+// triangle update W: W_ij -= L_ik W_kj (i > k, j <= k).  Measured (us per step): at 3,520
+// unknowns with the inverse, five launches one after the other 124 (tile factor 41, updates
+// 35 and 36), two 80; at 3,198 without, tile factor and update 59 -> 33.
+__global__ __launch_bounds__(kDirectBlock) void k_trailing_tiles(double* a, long ld, int k, int nt, int* __restrict__ bad,
+                                                                const double* __restrict__ diag0, int* __restrict__ dropped, double tau,
+                                                                double* __restrict__ inv, double* __restrict__ W) {
     __shared__ double Pt[kDT][kDTLd];
     __shared__ double Qt[kDT][kDTLd];
-    const int i = k + 1 + blockIdx.x;
-    const long ok = (long)k * kDT, oi = (long)i * kDT;
-    double* Aik = a + oi * ld + ok;
-    tile_update<true>(Aik, ld, Aik, ld, inv + (long)k * kDT * kDT, kDT, Pt, Qt, true, dropped ? dropped + ok : nullptr);
-}
-
-void dense_cholesky(Ctx& c, double* A, int npad, int* bad, double* tileInv, const double* diag0, int* dropped, double tau) {
-    const int nt = npad / kDT;
-    const long ld = npad;
-    for (int k = 0; k < nt; ++k) {
-        // the diagonal tile's inverse (tileInv) turns the panel into a product; without it
-        // the panel rows are solved by substitution (the direct solve's exact path)
-        hipLaunchKernelGGL(k_potrf_tile, dim3(1), dim3(kDirectBlock), 0, c.s, A, ld, k, bad, diag0, dropped, tau, tileInv);
-        const int m = nt - k - 1;
-        if (m > 0) {
-            if (tileInv) hipLaunchKernelGGL(k_panel_tiles, dim3(m), dim3(kDirectBlock), 0, c.s, A, ld, k, (const double*)tileInv,
-                                            (const int*)dropped);
-            else hipLaunchKernelGGL(k_trsm_tiles, dim3(m), dim3(kDirectBlock), 0, c.s, A, ld, k, (const int*)dropped);
-            hipLaunchKernelGGL(k_syrk_tiles, dim3(m * (m + 1) / 2), dim3(kDirectBlock), 0, c.s, A, ld, k, nt);
+    __shared__ double rd[kDT];
+    const int m = nt - k - 1, nSyrk = m * (m + 1) / 2;
+    const long ok = (long)k * kDT;
+    int b = blockIdx.x;
+    if (b < nSyrk) {
+        int ii = 0;
+        while (b >= ii + 1) { b -= ii + 1; ++ii; }   // row ii of the trailing triangle holds ii + 1 tiles
+        const long oi = (long)(k + 1 + ii) * kDT, oj = (long)(k + 1 + b) * kDT;
+        tile_update<true>(a + oi * ld + oj, ld, a + oi * ld + ok, ld, a + oj * ld + ok, ld, Pt, Qt, false);
+        if (blockIdx.x == 0) {
+            __syncthreads();   // the tile is in memory for the whole workgroup, the operands' LDS is free
+            potrf_tile(a, ld, k + 1, bad, diag0, dropped, tau, inv, reinterpret_cast<double (*)[kDT + 1]>(&Pt[0][0]),
+                       reinterpret_cast<double (*)[kDT + 1]>(&Qt[0][0]), rd);
         }
-        CIPC_LAUNCH_CHECK();
+    } else {
+        b -= nSyrk;
+        const int j = b % (k + 1), i = k + 1 + b / (k + 1);
+        const long oi = (long)i * kDT, oj = (long)j * kDT;
+        tile_update<false>(W + oi * ld + oj, ld, a + oi * ld + ok, ld, W + ok * ld + oj, ld, Pt, Qt, false);
     }
 }
 
-// L^-1 by blocked forward substitution on the identity, right-looking over tile rows k:
-// row k:  W_kj = inv(L_kk) W_kj  (j <= k; W_kj holds the updated right-hand side)
-// update: W_ij -= L_ik W_kj      (i > k, j <= k)
-__global__ __launch_bounds__(kDirectBlock) void k_inv_row(const double* __restrict__ inv, double* __restrict__ W, long ld, int k) {
-    __shared__ double Pt[kDT][kDTLd];
-    __shared__ double Qt[kDT][kDTLd];
-    const long ok = (long)k * kDT, oj = (long)blockIdx.x * kDT;   // tile column j = blockIdx.x <= k
-    double* Wkj = W + ok * ld + oj;
-    tile_update<false>(Wkj, ld, inv + (long)k * kDT * kDT, kDT, Wkj, ld, Pt, Qt, true);
-}
-__global__ __launch_bounds__(kDirectBlock) void k_inv_update(const double* __restrict__ L, double* __restrict__ W, long ld, int k) {
-    __shared__ double Pt[kDT][kDTLd];
-    __shared__ double Qt[kDT][kDTLd];
-    const int j = blockIdx.x % (k + 1), i = k + 1 + blockIdx.x / (k + 1);
-    const long ok = (long)k * kDT, oi = (long)i * kDT, oj = (long)j * kDT;
-    tile_update<false>(W + oi * ld + oj, ld, L + oi * ld + ok, ld, W + ok * ld + oj, ld, Pt, Qt, false);
-}
 __global__ void k_dense_identity(double* __restrict__ a, long ld, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) a[(long)i * ld + i] = 1.0;
 }
 
-// W = L^-1; tileInv holds the inverses of L's diagonal tiles (dense_cholesky with tileInv)
-void dense_lower_inverse(Ctx& c, const double* L, double* W, int npad, const double* tileInv) {
+// Factors A = L L^T in place (lower); with W, its inverse L^-1 is built in the same steps,
+// tileInv taking the diagonal tiles' inverses, which also turn the panel into a product.
+// Without, the panel rows are solved by substitution (the direct solve's exact path).
+void dense_cholesky(Ctx& c, double* A, int npad, int* bad, double* tileInv, const double* diag0, int* dropped, double tau, double* W) {
     const int nt = npad / kDT;
     const long ld = npad;
-    hipLaunchKernelGGL(k_dense_zero, dim3(2048), dim3(kBlock), 0, c.s, W, (long)npad * npad);
-    hipLaunchKernelGGL(k_dense_identity, dim3(nblocks(npad)), dim3(kBlock), 0, c.s, W, ld, npad);
+    if (W) {
+        hipLaunchKernelGGL(k_dense_zero, dim3(2048), dim3(kBlock), 0, c.s, W, (long)npad * npad);
+        hipLaunchKernelGGL(k_dense_identity, dim3(nblocks(npad)), dim3(kBlock), 0, c.s, W, ld, npad);
+    }
+    hipLaunchKernelGGL(k_potrf_tile, dim3(1), dim3(kDirectBlock), 0, c.s, A, ld, 0, bad, diag0, dropped, tau, tileInv);
     CIPC_LAUNCH_CHECK();
     for (int k = 0; k < nt; ++k) {
-        hipLaunchKernelGGL(k_inv_row, dim3(k + 1), dim3(kDirectBlock), 0, c.s, tileInv, W, ld, k);
-        if (k + 1 < nt) hipLaunchKernelGGL(k_inv_update, dim3((nt - k - 1) * (k + 1)), dim3(kDirectBlock), 0, c.s, L, W, ld, k);
+        const int m = nt - k - 1;
+        if (W) hipLaunchKernelGGL(k_panel_tiles, dim3(m + k + 1), dim3(kDirectBlock), 0, c.s, A, ld, k, m, (const double*)tileInv,
+                                  (const int*)dropped, W);
+        else if (m > 0) hipLaunchKernelGGL(k_trsm_tiles, dim3(m), dim3(kDirectBlock), 0, c.s, A, ld, k, (const int*)dropped);
+        if (m > 0) hipLaunchKernelGGL(k_trailing_tiles, dim3(m * (m + 1) / 2 + (W ? m * (k + 1) : 0)), dim3(kDirectBlock), 0, c.s, A, ld, k,
+                                      nt, bad, diag0, dropped, tau, tileInv, W);
         CIPC_LAUNCH_CHECK();
     }
 }
