@@ -344,9 +344,9 @@ class Simulator:
         """Compute_Constraint_Set (IPC.h:19-740)."""
         x = self._x(x)
         n = ctypes.c_int32(0)
-        cap = 1 << 16
+        cap = max(1 << 16, 16 * self.nV)   # rows nobody writes are never paged in
         while True:
-            out = np.zeros(4 * cap, dtype=np.int32)
+            out = np.empty(4 * cap, dtype=np.int32)
             rc = self.lib.cipc_constraint_set(self.h, _d(x), _i(out), cap, ctypes.byref(n))
             if rc == -7:
                 cap = n.value

@@ -20,6 +20,7 @@ using namespace cipc;
 struct cipc_ctx {
     Ctx c;
     DevBuf<double> qx, qp, qb, qsol, qout;
+    DevBuf<int> qRows;   // constraint sets as the caller holds them
     DevBuf<int> qC;
     unsigned char* scratch = nullptr;   // device address of this device's `scratch` array
 };
@@ -97,14 +98,18 @@ static void upload_x(cipc_ctx* ctx, DevBuf<double>& b, const double* h, size_t n
 // the device and is rejected here (CIPC_E_INVALID through guarded()).
 static void upload_cs(cipc_ctx* ctx, const int32_t* cs, int32_t n) {
     const int nV = ctx->c.nV;
-    for (size_t i = 0; i < 4 * (size_t)n; ++i)
-        if (cs[i] < -nV || cs[i] >= nV)
-            throw std::invalid_argument("constraint " + std::to_string(i / 4) + " has an entry outside [-n_vertices, n_vertices)");
-    std::vector<int> soa(4 * (size_t)std::max(n, 1));
-    for (int i = 0; i < n; ++i)
-        for (int k = 0; k < 4; ++k) soa[(size_t)k * n + i] = cs[4 * (size_t)i + k];
-    ctx->qC.ensure(soa.size());
-    CIPC_HIP(hipMemcpyAsync(ctx->qC.p, soa.data(), soa.size() * sizeof(int), hipMemcpyHostToDevice, ctx->c.s));
+    const size_t m = 4 * (size_t)n;
+    bool out = false;   // no branch in the loop: it is a pass of vector compares
+    for (size_t i = 0; i < m; ++i) out |= (uint32_t)cs[i] + (uint32_t)nV >= 2u * (uint32_t)nV;
+    if (out)
+        for (size_t i = 0; i < m; ++i)
+            if (cs[i] < -nV || cs[i] >= nV)
+                throw std::invalid_argument("constraint " + std::to_string(i / 4) + " has an entry outside [-n_vertices, n_vertices)");
+    ctx->qC.ensure(std::max<size_t>(m, 4));
+    if (n == 0) return;
+    int* rows = ctx->qRows.ensure(m);
+    CIPC_HIP(hipMemcpyAsync(rows, cs, m * sizeof(int), hipMemcpyHostToDevice, ctx->c.s));
+    constraint_rows(ctx->c, ctx->qC.p, rows, n, false);
     CIPC_HIP(hipStreamSynchronize(ctx->c.s));
 }
 
@@ -318,11 +323,11 @@ int cipc_constraint_set(cipc_ctx* ctx, const double* x, int32_t* out, int32_t ca
         constraint_set(c, ctx->qx.p, outD, nC);
         *n = nC;
         if (nC > cap || !out) return nC > cap ? CIPC_E_CAPACITY : CIPC_OK;
-        std::vector<int> soa(4 * (size_t)std::max(nC, 1));
-        CIPC_HIP(hipMemcpyAsync(soa.data(), outD.p, 4 * (size_t)nC * sizeof(int), hipMemcpyDeviceToHost, c.s));
+        if (nC == 0) return CIPC_OK;
+        int* rows = ctx->qRows.ensure(4 * (size_t)nC);
+        constraint_rows(c, outD.p, rows, nC, true);
+        CIPC_HIP(hipMemcpyAsync(out, rows, 4 * (size_t)nC * sizeof(int), hipMemcpyDeviceToHost, c.s));
         CIPC_HIP(hipStreamSynchronize(c.s));
-        for (int i = 0; i < nC; ++i)
-            for (int k = 0; k < 4; ++k) out[4 * (size_t)i + k] = soa[(size_t)k * nC + i];
         return CIPC_OK;
     });
 }

@@ -332,6 +332,7 @@ void minmax6_final(const double* part, int nb, double* out6, hipStream_t s);   /
 
 // ---- stages (implemented in the .hip files)
 void ctx_init_device(Ctx& c);                                      // upload + derived data
+void constraint_rows(Ctx& c, int* C, int* rows, int nC, bool toRows);   // SoA set <-> int4 rows, on the device
 void constraint_set(Ctx& c, const double* x, DevBuf<int>& out, int& nOut);
 double barrier_energy(Ctx& c, const double* x, const int* C, int nC, double kappa, int* bad);
 // int4-row constraints, caller-supplied device partials / sum / flags; allocates nothing
