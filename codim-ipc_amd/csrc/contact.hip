@@ -1067,17 +1067,36 @@ __global__ void k_grad_keys(const int* __restrict__ gv, long n, int nV, const ui
     int v = gv[i];
     key[i] = (v < 0 || (skip && skip[v])) ? (uint64_t)nV : (uint64_t)v;
 }
+// Eight lanes per vertex fetch eight slots at a time, the next eight while these are added in
+// slot order: a vertex that many stencils touch was one thread's chain of loads.
+// Measured: 171 -> 86 us on 4 sheets of 201 x 201 in contact, 46 -> 28 on 101 x 101 (one thread
+// with eight slots in flight: 52).
+constexpr int kGatherLanes = 8;
 __global__ void k_grad_gather(const double* __restrict__ gl, long ns, const uint32_t* __restrict__ slot, const uint32_t* __restrict__ start,
                               const uint32_t* __restrict__ end, int nV, double* __restrict__ g) {
-    int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= nV) return;
-    uint32_t s = start[v], e = end[v];
-    double a = 0, b = 0, d = 0;
-    for (uint32_t k = s; k < e; ++k) {
-        long q = slot[k];
-        a += gl[q]; b += gl[ns + q]; d += gl[2 * ns + q];
+    const int lane = threadIdx.x % kGatherLanes;
+    const int v = (int)(((long)blockIdx.x * blockDim.x + threadIdx.x) / kGatherLanes);
+    const uint32_t s = v < nV ? start[v] : 0, e = v < nV ? end[v] : 0;
+    double sum = 0;   // lanes 0, 1, 2: x, y, z
+    double na = 0, nb = 0, nd = 0;
+    auto fetch = [&](uint32_t k) {
+        const bool on = k + lane < e;
+        const long q = on ? slot[k + lane] : 0;
+        na = on ? gl[q] : 0.0;
+        nb = on ? gl[ns + q] : 0.0;
+        nd = on ? gl[2 * ns + q] : 0.0;
+    };
+    if (s < e) fetch(s);
+    for (uint32_t k = s; k < e; k += kGatherLanes) {
+        const double a = na, b = nb, d = nd;
+        if (k + kGatherLanes < e) fetch(k + kGatherLanes);
+#pragma unroll
+        for (int u = 0; u < kGatherLanes; ++u) {
+            const double x = __shfl(a, u, kGatherLanes), y = __shfl(b, u, kGatherLanes), z = __shfl(d, u, kGatherLanes);
+            sum += lane == 0 ? x : lane == 1 ? y : z;   // past the end: + 0
+        }
     }
-    g[3 * v] += a; g[3 * v + 1] += b; g[3 * v + 2] += d;
+    if (v < nV && lane < 3) g[3 * v + lane] += sum;
 }
 
 // g += barrier gradient (deterministic: slots sorted by vertex, summed in slot order)
@@ -1106,7 +1125,7 @@ void scatter_local_gradient(Ctx& c, const double* gl, const int* gv, long ns, do
     CIPC_HIP(hipMemsetAsync(en, 0, c.nV * sizeof(uint32_t), c.s));
     hipLaunchKernelGGL(k_vert_bounds, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, (const uint64_t*)sorted.keys, ns, c.nV, st, en);
     CIPC_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_grad_gather, dim3(nblocks(c.nV)), dim3(kBlock), 0, c.s, gl, ns, (const uint32_t*)sorted.vals, st, en, c.nV, g);
+    hipLaunchKernelGGL(k_grad_gather, dim3(nblocks((long)c.nV * kGatherLanes)), dim3(kBlock), 0, c.s, gl, ns, (const uint32_t*)sorted.vals, st, en, c.nV, g);
     CIPC_LAUNCH_CHECK();
 }
 
