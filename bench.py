@@ -56,9 +56,9 @@ sys.path.insert(0, os.path.join(ROOT, "codim-ipc_amd"))
 
 METRIC = "sim steps/s + ms/Newton iter, 320k-tri cloth; plain FP64 vs mixed+learned PCG"
 HBM_PEAK_GBS = 8000.0
-KERNEL = {"fp64": ("k_pcg_spmv_p<double,double,%d,256,%d>", "PCG SpMV, FP64 blocks, FP64 vectors"),
-          "mixed": ("k_pcg_spmv_p<float,double,%d,256,%d>", "PCG SpMV, FP32 blocks, FP64 vectors"),
-          "fp32": ("k_pcg_spmv_p<float,float,%d,256,%d>", "PCG SpMV, FP32 blocks, FP32 vectors"),
+KERNEL = {"fp64": ("k_pcg_spmv_p<double,double,%d,256,true,%d>", "PCG SpMV, FP64 blocks, FP64 vectors"),
+          "mixed": ("k_pcg_spmv_p<float,double,%d,256,true,%d>", "PCG SpMV, FP32 blocks, FP64 vectors"),
+          "fp32": ("k_pcg_spmv_p<float,float,%d,256,true,%d>", "PCG SpMV, FP32 blocks, FP32 vectors"),
           "mixed_learned": ("k_pcg_spmv<float,double,%d,256,true,%d>", "PCG SpMV, FP32 blocks, FP64 vectors"),
           "fp32_learned": ("k_pcg_spmv<float,float,%d,256,true,%d>", "PCG SpMV, FP32 blocks, FP32 vectors"),
           "mixed_learned_coarse": ("k_pcg_spmv<float,double,%d,256,true,%d>", "PCG SpMV, FP32 blocks, FP64 vectors"),

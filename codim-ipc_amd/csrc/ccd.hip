@@ -424,7 +424,7 @@ __global__ __launch_bounds__(kBlock) void k_ccd_walk(P T, int n, double alpha0, 
 
 // particle (boundary-node slot s >= codimBN1) against rod segments, IPC.h:2095-2133,
 // and particle pairs, IPC.h:2135-2162 (a pair is run with the lower slot first, as the
-// reference does); same voxel-overlap candidate rule and cell coverage as k_ccd_ee
+// reference does); same voxel-overlap candidate rule and cell coverage as the edge walk
 __device__ __forceinline__ void pe_ccd_candidate(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ bEdge,
                                                  int nBE, const uint8_t* __restrict__ dbc, const int* __restrict__ elo,
                                                  const int* __restrict__ ehi, int vI, const int* nlo, const int* nhi, d3 P, d3 dP, int e,

@@ -341,7 +341,8 @@ static auto spmv_kernel(int lanes, int unr, bool withP) -> decltype(&k_pcg_spmv<
 // per block cost more than the second launch.)
 // Partials: partS = [2][workgroups] of p.q, q.u; partU = [2][workgroups] of r.z, r.r,
 // double-buffered (an update reads the previous one's while it writes its own).
-template <class M, class V, int LANES, int BS, int UNR>
+// CON: whether there are contact blocks (without, their row bounds are not read).
+template <class M, class V, int LANES, int BS, bool CON, int UNR>
 __global__ __launch_bounds__(BS) void k_pcg_spmv_p(const int* __restrict__ erp, const int* __restrict__ ecol, const M* __restrict__ ev,
                                                    int enz, const int* __restrict__ crp, const int* __restrict__ ccol,
                                                    const M* __restrict__ cv, int cnz, int nrow, int rowsPerXcd,
@@ -358,7 +359,7 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv_p(const int* __restrict__ erp, 
     const bool live = g * RPG < rowsPerXcd && row < nrow;
     const int done = flags[F_DONE];
     int beg = live ? erp[row] : 0, end = live ? erp[row + 1] : 0;
-    int cbeg = live && cnz > 0 ? crp[row] : 0, cend = live && cnz > 0 ? crp[row + 1] : 0;
+    int cbeg = live && CON ? crp[row] : 0, cend = live && CON ? crp[row + 1] : 0;
     if (done) return;
     double sum[2] = {0, 0};
     for (; g * RPG < rowsPerXcd; g += nj) {
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv_p(const int* __restrict__ erp, 
         const int rowN = rowBase + gn * RPG;
         const bool liveN = gn * RPG < rowsPerXcd && rowN < nrow;
         const int begN = liveN ? erp[rowN] : 0, endN = liveN ? erp[rowN + 1] : 0;
-        const int cbegN = liveN && cnz > 0 ? crp[rowN] : 0, cendN = liveN && cnz > 0 ? crp[rowN + 1] : 0;
+        const int cbegN = liveN && CON ? crp[rowN] : 0, cendN = liveN && CON ? crp[rowN + 1] : 0;
         // lanes 0..2 own one component of the row each; their loads are in flight during
         // the row's products
         const bool owner = row < nrow && lane < 3;
@@ -413,9 +414,9 @@ __global__ __launch_bounds__(BS) void k_pcg_spmv_p(const int* __restrict__ erp, 
     }
 }
 template <class M, class V>
-static auto spmv_p_kernel(int lanes, int unr) -> decltype(&k_pcg_spmv_p<M, V, 16, kSpmvBlock, 1>) {
+static auto spmv_p_kernel(int lanes, int unr, bool con) -> decltype(&k_pcg_spmv_p<M, V, 16, kSpmvBlock, true, 1>) {
 #define CIPC_SPMV_P_PICK(L, U) \
-    if (lanes == L && unr == U) return k_pcg_spmv_p<M, V, L, kSpmvBlock, U>;
+    if (lanes == L && unr == U) return con ? k_pcg_spmv_p<M, V, L, kSpmvBlock, true, U> : k_pcg_spmv_p<M, V, L, kSpmvBlock, false, U>;
     CIPC_SPMV_P_PICK(8, 1)
     CIPC_SPMV_P_PICK(8, 2)
     CIPC_SPMV_P_PICK(4, 1)
@@ -840,7 +841,7 @@ static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V*
                 hipLaunchKernelGGL(kern, dim3(nS), dim3(kSpmvBlock), 0, c.s, args...);
         };
         if (!learned) {
-            go(spmv_p_kernel<M, V>(sLanes, sUnroll), (const int*)E.rowptr.p, (const int*)E.col.p, valE, E.nnzb, (const int*)K.rowptr.p,
+            go(spmv_p_kernel<M, V>(sLanes, sUnroll, K.nnzb > 0), (const int*)E.rowptr.p, (const int*)E.col.p, valE, E.nnzb, (const int*)K.rowptr.p,
                (const int*)K.col.p, valK, K.nnzb, nV, rpxS, (const V*)pbuf, dinv, q, partS, (const int*)flags);
             // the first update reads the init kernel's partials, the others the previous update's
             hipLaunchKernelGGL((updRows == kUpdRows ? k_pcg_update_p<V, kUpdRows> : k_pcg_update_p<V, kUpdRowsSmall>), dim3(nU),
