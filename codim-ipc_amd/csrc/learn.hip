@@ -320,12 +320,39 @@ __global__ void k_lp_scatter_lower(int nL, const int* __restrict__ lEdge, const 
 // The training form of the 64-wide layers on v_mfma_f32_16x16x4_f32: FP32 inputs, weights,
 // products and accumulation, so nothing is rounded that the vector form kept.  Lane l feeds
 // A row l % 16 and B column l % 16 at one k per instruction and holds D rows 4 (l / 16) + t,
-// column l % 16.  Which k a lane feeds in which step is free as long as A and B agree: over
-// 16 k's, lane group l / 16 takes k = 4 (l / 16) + step, so that both operands of four
-// steps are one 16-byte load.  The operand held in LDS has rows of 64 n + 4 floats: the 16
-// lanes of a group then read 16 different groups of four banks.
+// column l % 16.  An instruction adds its four products in k order, each by a fused
+// multiply-add (checked bit for bit against fmaf on the card, subnormal sums included).
+// The forward layers feed k in ascending order, lane group l / 16 at step s k = 4 s + l / 16,
+// and so round as a loop of fmaf over k does: a ReLU that stands within that rounding of
+// zero keeps its side, whereas one flipped mask moves a gradient by up to 5e-3 of its rms.
+// The input gradients have no such switch; there group l / 16 takes k = 4 (l / 16) + step,
+// so that both operands of four steps are one 16-byte load.  The operand held in LDS has
+// rows of 64 n + 4 floats: the 16 lanes of a group then read 16 different groups of four banks.
 typedef float lp_f4 __attribute__((ext_vector_type(4)));
 constexpr int kLpF32Pad = 4;
+// place of input k among the 16 of its group in LDS: lane group g finds k = g, 4 + g, 8 + g,
+// 12 + g side by side
+__device__ __forceinline__ constexpr int lp_place(int k) { return (k & ~15) | (k & 3) << 2 | (k >> 2 & 3); }
+// rows 4 g + t of lane group g -> rows 4 t + g: the 4 x 4 transposition of 16-lane groups and
+// registers, by swapping half waves, then rows of 16 lanes
+__device__ __forceinline__ void lp_swap32(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(a), __float_as_int(b), false, false);
+    a = __int_as_float((int)r[0]);
+    b = __int_as_float((int)r[1]);
+}
+__device__ __forceinline__ void lp_swap16(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(a), __float_as_int(b), false, false);
+    a = __int_as_float((int)r[0]);
+    b = __int_as_float((int)r[1]);
+}
+__device__ __forceinline__ lp_f4 lp_ascending(lp_f4 v) {
+    float a = v[0], b = v[1], c = v[2], d = v[3];
+    lp_swap32(a, c);
+    lp_swap32(b, d);
+    lp_swap16(a, b);
+    lp_swap16(c, d);
+    return lp_f4{a, b, c, d};
+}
 
 // out = act(b + [x0 x1 x2] W) (W [64 NSEG][nout], nout <= 16 NT), and sumOut = sumIn + out
 // when asked for.  A wave takes tiles of 16 rows.  Bound: the gathered rows (192 inputs per
@@ -346,14 +373,14 @@ __global__ __launch_bounds__(256, 3) void k_lp_dense_f32(int nrows, LpSeg s0, Lp
             const lp_f4 w = *reinterpret_cast<const lp_f4*>(W + 4 * t);
             const int k = t / 16, o = 4 * (t % 16);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) Wt[(o + i) * LD + k] = w[i];
+            for (int i = 0; i < 4; ++i) Wt[(o + i) * LD + lp_place(k)] = w[i];
         }
     } else {
 #pragma unroll 6
         for (int t = threadIdx.x; t < K * 16 * NT; t += 256) {
             const int k = t / (16 * NT), o = t % (16 * NT);
             const float w = W[o < nout ? k * nout + o : 0];
-            Wt[o * LD + k] = o < nout ? w : 0.f;
+            Wt[o * LD + lp_place(k)] = o < nout ? w : 0.f;
         }
     }
     __syncthreads();
@@ -368,6 +395,8 @@ __global__ __launch_bounds__(256, 3) void k_lp_dense_f32(int nrows, LpSeg s0, Lp
         for (int s = 0; s < NSEG; ++s)
 #pragma unroll
             for (int u = 0; u < 4; ++u) a[4 * s + u] = *reinterpret_cast<const lp_f4*>(row[s] + 16 * u + 4 * g);
+#pragma unroll
+        for (int u = 0; u < 4 * NSEG; ++u) a[u] = lp_ascending(a[u]);
         lp_f4 acc[NT];
 #pragma unroll
         for (int j = 0; j < NT; ++j) {

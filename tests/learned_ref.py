@@ -101,9 +101,9 @@ def contact_row_counts(nV, C, dbc=None):
     return np.array([len(r) for r in rows], dtype=float)
 
 
-def loss_and_grad(H, mass, dbc, tri, hinge, weights, nprobes, seed, contact_rows=None):
-    """H: scipy CSR (3n x 3n) of the assembled Hessian; contact_rows: per vertex number of
-    contact blocks in the row (None -> zeros).  Returns (loss, flat gradient float64)."""
+def features(H, mass, dbc, tri, hinge, contact_rows=None):
+    """Node and edge features (float64), the graph's edges, and the scaling S with the block
+    matrix they come from."""
     nV = H.shape[0] // 3
     B = H.tobsr(blocksize=(3, 3))
     B.sort_indices()
@@ -116,7 +116,6 @@ def loss_and_grad(H, mass, dbc, tri, hinge, weights, nprobes, seed, contact_rows
     d = H.diagonal()
     s = np.where(d > 0, 1.0 / np.sqrt(np.where(d > 0, d, 1.0)), 1.0).reshape(nV, 3)
     Hhat_full = torch.tensor(np.array([B.data[k] * s[i][:, None] * s[j][None, :] for k, (i, j) in enumerate(zip(brow, B.indices))]))
-    Hrow, Hcol = torch.tensor(brow), torch.tensor(B.indices.astype(np.int64))
     diagk = np.array([lut[(i, i)] for i in range(nV)])
     node = np.zeros((nV, 12))
     node[:, :9] = Hhat_full[diagk].reshape(nV, 9).numpy()
@@ -130,6 +129,16 @@ def loss_and_grad(H, mass, dbc, tri, hinge, weights, nprobes, seed, contact_rows
         k = lut.get((int(i), int(j)))
         if k is not None:
             ef[t] = (B.data[k] * s[i][:, None] * s[j][None, :]).ravel()
+    return node, ef, er, ec, s, B, brow
+
+
+def loss_and_grad(H, mass, dbc, tri, hinge, weights, nprobes, seed, contact_rows=None, relu=lambda z, layer: torch.relu(z)):
+    """H: scipy CSR (3n x 3n) of the assembled Hessian; contact_rows: per vertex number of
+    contact blocks in the row (None -> zeros); relu(z, layer): the activation of layer "h",
+    "e", "m0", "u0", ...  Returns (loss, flat gradient float64)."""
+    node, ef, er, ec, s, B, brow = features(H, mass, dbc, tri, hinge, contact_rows)
+    nV = len(node)
+    Hrow, Hcol = torch.tensor(brow), torch.tensor(B.indices.astype(np.int64))
 
     L, total = layout()
     wq = torch.tensor(bf16(weights).astype(np.float64), requires_grad=True)
@@ -145,12 +154,12 @@ def loss_and_grad(H, mass, dbc, tri, hinge, weights, nprobes, seed, contact_rows
     er_t, ec_t = torch.tensor(er), torch.tensor(ec)
     f = torch.tensor(node)
     a = torch.tensor(ef)
-    h = torch.relu(f @ W("we", 12, HID) + B_("be"))
-    e = torch.relu(a @ W("wx", 9, HID) + B_("bx"))
+    h = relu(f @ W("we", 12, HID) + B_("be"), "h")
+    e = relu(a @ W("wx", 9, HID) + B_("bx"), "e")
     for l in range(LAYERS):
-        m = torch.relu(torch.cat([h[er_t], h[ec_t], e], 1) @ W("wm%d" % l, 3 * HID, HID) + B_("bm%d" % l))
+        m = relu(torch.cat([h[er_t], h[ec_t], e], 1) @ W("wm%d" % l, 3 * HID, HID) + B_("bm%d" % l), "m%d" % l)
         agg = torch.zeros_like(h).index_add(0, er_t, m)
-        h = h + torch.relu(torch.cat([h, agg], 1) @ W("wu%d" % l, 2 * HID, HID) + B_("bu%d" % l))
+        h = h + relu(torch.cat([h, agg], 1) @ W("wu%d" % l, 2 * HID, HID) + B_("bu%d" % l), "u%d" % l)
         e = e + m
     low = torch.tensor(ec < er)
     lr_, lc_ = er_t[low], ec_t[low]
