@@ -106,10 +106,13 @@ static void upload_cs(cipc_ctx* ctx, const int32_t* cs, int32_t n) {
             if (cs[i] < -nV || cs[i] >= nV)
                 throw std::invalid_argument("constraint " + std::to_string(i / 4) + " has an entry outside [-n_vertices, n_vertices)");
     ctx->qC.ensure(std::max<size_t>(m, 4));
-    if (n == 0) return;
-    int* rows = ctx->qRows.ensure(m);
-    CIPC_HIP(hipMemcpyAsync(rows, cs, m * sizeof(int), hipMemcpyHostToDevice, ctx->c.s));
-    constraint_rows(ctx->c, ctx->qC.p, rows, n, false);
+    if (n > 0) {
+        int* rows = ctx->qRows.ensure(m);
+        CIPC_HIP(hipMemcpyAsync(rows, cs, m * sizeof(int), hipMemcpyHostToDevice, ctx->c.s));
+        constraint_rows(ctx->c, ctx->qC.p, rows, n, false);
+    }
+    // also for an empty set: the uploads before it (upload_x) may be in flight from the
+    // caller's pinned memory, and a call that has nothing to compute returns from here
     CIPC_HIP(hipStreamSynchronize(ctx->c.s));
 }
 
