@@ -17,6 +17,7 @@
 #pragma once
 #include "ctx.hpp"
 #include <algorithm>
+#include <stdexcept>
 
 namespace cipc {
 
@@ -28,7 +29,9 @@ inline int walk_grid(long n) { return (int)std::max(1l, std::min((long)kWalkGrid
 
 // A cell entry's value: the primitive and, per axis, whether the cell is the first one of
 // the primitive's box.  A cell is the first common one of two boxes when on every axis it
-// is the first of one of them.
+// is the first of one of them.  (Flags in the record's unused word, 32 bits for the primitive:
+// a fourth register per record read ahead, constraint set of 492,000 edges 5.10 -> 5.30 ms,
+// CCD of 129,000 edges 0.80 -> 0.83.)  More primitives than the 29 bits number are refused.
 constexpr int kWalkIdBits = 29;
 constexpr uint32_t kWalkId = (1u << kWalkIdBits) - 1;
 __device__ __forceinline__ uint32_t walk_entry(int prim, bool fx, bool fy, bool fz) {
@@ -72,6 +75,7 @@ __device__ __forceinline__ void for_prim_cells(const int* a, const int* b, const
 // per-cell counters cleared; room for the lists' starts
 inline void walk_cells_begin(Ctx& c, long nCells, int n, DevBuf<uint32_t>& start, DevBuf<uint32_t>& count, DevBuf<int>& box,
                              DevBuf<uint8_t>& lgFlag, DevBuf<int>& lgList) {
+    if ((uint32_t)n > kWalkId) throw std::length_error("more than 2^29 - 1 boundary triangles, edges or particles");
     start.ensure(nCells + 1);
     count.ensure(nCells);
     CIPC_HIP(hipMemsetAsync(count.p, 0, nCells * sizeof(uint32_t), c.s));
