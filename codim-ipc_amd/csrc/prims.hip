@@ -219,10 +219,17 @@ __global__ void k_rs_scatter(const uint64_t* __restrict__ kin, const uint32_t* _
 // Short inputs by counting: an element's place is the number of smaller keys plus the equal
 // ones before it.  64 elements per workgroup, each of its four waves compares them with a
 // quarter of the keys (uniform addresses: scalar loads); one launch instead of five per
-// digit.  kRankSort: from there on the quadratic work is longer than the passes of 20-bit
-// keys, the shortest in use (us, counting / passes of 20 bits / of 40 bits: 2,000 keys 13.5 /
-// 36.8 / 63, 8,000 keys 41.4 / 42.0 / 74, 16,000 keys 79 / 43 / 80).
-constexpr int kRankSort = 8192;
+// digit.  kRankSort: keys at most, by the number of digits that the passes would take: the
+// counting is quadratic in the keys and does not see their length.  The lines are those of
+// whole calls (us, counting / passes), where the card idles between calls:
+//   2 digits, gradient by vertex   1,600 slots 122 / 134   3,200 137 / 137   4,800 159 / 143   8,000 180 / 146
+//   3 digits, barrier Hessian      3,200 slots 581 / 630   6,400 745 / 746   8,000 813 / 794   16,000 1,229 / 1,094
+//   4 digits, constraint set, edge pairs 7,500 (2,400 point-triangle pairs)  338 / 426
+//             9,900 (3,100) 385 / 457   15,400 (4,900) 480 / 478   22,100 (7,000) 608 / 530:
+//             the edge pairs alone cross near 9,600
+// Back to back the counting is a third faster (2 digits cross at 5,000, 3 at 9,600, 4 at
+// 15,000, 1 at 1,900), which sets the lines for 1, 5 and 6 digits in proportion.
+constexpr long kRankSort[] = {0, 1200, 3200, 6400, 9600, 12800, 16000};
 __global__ __launch_bounds__(kBlock) void k_rank_sort(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                       uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, int n) {
     __shared__ uint32_t part[4][64];
@@ -250,13 +257,13 @@ SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, P
     if (n <= 0) return {keys, vals};
     uint64_t* k2 = w.keyAlt.ensure(n);
     uint32_t* v2 = w.valAlt.ensure(n);
-    if (n <= kRankSort) {
+    const int passes = (bits + kMaxDigit - 1) / kMaxDigit, rb = (bits + passes - 1) / passes;
+    if (n <= kRankSort[std::min(passes, 6)]) {
         hipLaunchKernelGGL(k_rank_sort, dim3((unsigned)((n + 63) / 64)), dim3(kBlock), 0, s, keys, iota ? nullptr : vals, k2, v2, (int)n);
         CIPC_LAUNCH_CHECK();
         return {k2, v2};
     }
     int nb = (int)((n + RS_TILE - 1) / RS_TILE);
-    const int passes = (bits + kMaxDigit - 1) / kMaxDigit, rb = (bits + passes - 1) / passes;
     uint32_t* hist = w.hist.ensure((size_t)nb << rb);
     uint32_t* hs = w.histScan.ensure((size_t)nb << rb);
     uint64_t *ka = keys, *kb = k2;
