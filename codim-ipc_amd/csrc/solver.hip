@@ -428,18 +428,19 @@ static auto spmv_p_kernel(int lanes, int unr, bool con) -> decltype(&k_pcg_spmv_
 }
 
 // Iteration `it` after its SpMV: convergence of r_it is decided first (its r.r was summed by
-// the previous update), then x, r, z and the next direction.  One thread per component:
-// consecutive lanes read consecutive addresses, where one thread per vertex took 33
-// accesses of stride 24 bytes each; r' crosses to the vertex's other components through
-// LDS.  Workgroups of VB = 128 vertices spread small systems over the CUs; large ones walk
-// several such groups (at most kUpdGrid workgroups, so that the partials every workgroup
-// adds up stay few).  Measured (us per iteration with groups of 64 / 128 / 256 vertices): 8.5 /
-// 9.1 / 10.7 on 4,247 vertices, 25.3 / 24.1 / 24.7 on 33,169 (FP64 blocks).
+// the previous update), then x, r and the next direction from z = Dinv r, which stays in
+// registers.  One thread per component: consecutive lanes read consecutive addresses, where
+// one thread per vertex took 33 accesses of stride 24 bytes each; r' crosses to the vertex's
+// other components through LDS.  Workgroups of VB vertices: 64 up to kSmallRows vertices, to
+// spread small systems over the CUs, 128 beyond; large systems walk several such groups (at
+// most kUpdGrid workgroups, so that the partials every workgroup adds up stay few).
+// Measured (us per iteration with groups of 64 / 128 / 256 vertices): 8.5 / 9.1 / 10.7 on
+// 4,247 vertices, 25.3 / 24.1 / 24.7 on 33,169 (FP64 blocks).
 template <class V, int VB>
 __global__ __launch_bounds__(3 * VB) void k_pcg_update_p(const int* __restrict__ itDev, int itArg, int maxIt, int nrow, int rowsPerXcd,
-                                                         V* __restrict__ x, V* __restrict__ r, V* __restrict__ z, V* __restrict__ p,
-                                                         const V* __restrict__ q, const V* __restrict__ dinv,
-                                                         const double* __restrict__ partS, int nS, const double* __restrict__ partU, int nIn,
+                                                         V* __restrict__ x, V* __restrict__ r, V* __restrict__ p, const V* __restrict__ q,
+                                                         const V* __restrict__ dinv, const double* __restrict__ partS, int nS,
+                                                         const double* __restrict__ partU, int nIn,
                                                          double* __restrict__ partUN, double* __restrict__ sc, int* __restrict__ flags) {
     constexpr int BS = 3 * VB, NW = BS / 64;
     __shared__ double lds[4][NW], ldsN[2][NW];
@@ -513,7 +514,6 @@ __global__ __launch_bounds__(3 * VB) void k_pcg_update_p(const int* __restrict__
         if (valid) {
             x[o] = xv + alpha * pv;
             r[o] = rv;
-            z[o] = zk;
             p[o] = zk + beta * pv;
         }
         srz += (double)rv * (double)zk;
@@ -635,12 +635,12 @@ __global__ __launch_bounds__(BS) void k_pcg_update_lower(const int* __restrict__
     if (threadIdx.x == 0) partRR[blockIdx.x] = brr;
 }
 
-// r = b, x = 0, z = Dinv r and, when p is given, p = z; partials of r.z and r.r in the
-// update kernel's layout; the solver flags are cleared.
+// r = b, x = 0 and, when p is given (block Jacobi), p = z = Dinv r; partials of r.z (then) and
+// r.r in the update kernel's layout; the solver flags are cleared.
 template <class V, int BS>
 __global__ __launch_bounds__(BS) void k_pcg_init(int nrow, int rowsPerXcd, const V* __restrict__ b, V* __restrict__ x, V* __restrict__ r,
-                                                 V* __restrict__ z, V* __restrict__ p, const V* __restrict__ dinv,
-                                                 double* __restrict__ partU, int* __restrict__ flags) {
+                                                 V* __restrict__ p, const V* __restrict__ dinv, double* __restrict__ partU,
+                                                 int* __restrict__ flags) {
     __shared__ double lds[BS / 64];
     const int row = (int)(blockIdx.x % kXcd) * rowsPerXcd + (int)(blockIdx.x / kXcd) * BS + (int)threadIdx.x;
     double rz = 0, rr = 0;
@@ -653,13 +653,13 @@ __global__ __launch_bounds__(BS) void k_pcg_init(int nrow, int rowsPerXcd, const
             x[3 * row + k] = 0;
             rr += (double)rv[k] * (double)rv[k];
         }
+        if (p)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const V zk = dinv[9l * row + 3 * k] * rv[0] + dinv[9l * row + 3 * k + 1] * rv[1] + dinv[9l * row + 3 * k + 2] * rv[2];
-            z[3 * row + k] = zk;
-            if (p) p[3 * row + k] = zk;
-            rz += (double)rv[k] * (double)zk;
-        }
+            for (int k = 0; k < 3; ++k) {
+                const V zk = dinv[9l * row + 3 * k] * rv[0] + dinv[9l * row + 3 * k + 1] * rv[1] + dinv[9l * row + 3 * k + 2] * rv[2];
+                p[3 * row + k] = zk;
+                rz += (double)rv[k] * (double)zk;
+            }
     }
     const double brz = block_allsum<BS>(rz, lds);
     const double brr = block_allsum<BS>(rr, lds);
@@ -760,7 +760,8 @@ __global__ void k_it_advance(int* itDev, int by) {
 }
 
 // ---- one preconditioned CG solve in precision V; returns 0 converged, 1 not SPD
-// (p^T A p <= 0), 2 iteration limit
+// (p^T A p <= 0), 2 iteration limit.  Block Jacobi keeps one direction in pbuf and no z; the
+// learned form alternates between the two halves of pbuf.
 template <class M, class V>
 static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V* r, V* z, V* pbuf, V* q, const V* dinv, double tol,
                    int maxIter, int* iters, double* relres, bool learned = false) {
@@ -793,7 +794,7 @@ static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V*
     V* ltmp = nullptr;
     V* rb[2] = {r, r};                        // learned form: r ping-pongs between r and a second buffer
 
-    hipLaunchKernelGGL((k_pcg_init<V, kInitBlock>), dim3(nI), dim3(kInitBlock), 0, c.s, nV, rpxI, b, xsol, r, z,
+    hipLaunchKernelGGL((k_pcg_init<V, kInitBlock>), dim3(nI), dim3(kInitBlock), 0, c.s, nV, rpxI, b, xsol, r,
                        learned ? (V*)nullptr : pbuf, dinv, partI, flags);
     CIPC_LAUNCH_CHECK();
     if (learned) {
@@ -845,8 +846,7 @@ static int pcg_run(Ctx& c, const M* valE, const M* valK, const V* b, V* xsol, V*
                (const int*)K.col.p, valK, K.nnzb, nV, rpxS, (const V*)pbuf, dinv, q, partS, (const int*)flags);
             // the first update reads the init kernel's partials, the others the previous update's
             hipLaunchKernelGGL((updRows == kUpdRows ? k_pcg_update_p<V, kUpdRows> : k_pcg_update_p<V, kUpdRowsSmall>), dim3(nU),
-                               dim3(3 * updRows), 0, c.s, itd, itArg, maxIter, nV, rpxU, xsol, r,
-                               z, pbuf, (const V*)q, dinv, (const double*)partS, nS,
+                               dim3(3 * updRows), 0, c.s, itd, itArg, maxIter, nV, rpxU, xsol, r, pbuf, (const V*)q, dinv, (const double*)partS, nS,
                                (const double*)(it == 0 ? partI : partU + 2l * (it & 1) * nU), it == 0 ? nI : nU,
                                partU + 2l * ((it + 1) & 1) * nU, sc, flags);
         } else {
