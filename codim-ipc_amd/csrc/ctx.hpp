@@ -155,9 +155,8 @@ struct Ctx {
     DevBuf<uint32_t> pcellStart, pcellCount;
     DevBuf<uint8_t> lgFlagP;
     DevBuf<int> lgListP;
-    DevBuf<int> ccdPlo, ccdPhi;
-    DevBuf<int> ccdTbox, ccdEbox, ccdPbox;   // the same voxel boxes as 32-byte records (lo xyz, hi xyz, 2 pad)
-    DevBuf<int> ccdTrec, ccdErec, ccdPrec;            // those records in cell order (third pad word = primitive)
+    DevBuf<int> ccdTbox, ccdEbox, ccdPbox;   // voxel boxes as 32-byte records (lo xyz, hi xyz, 2 unused)
+    DevBuf<int> ccdTrec, ccdErec, ccdPrec;   // those records in cell order (seventh word: primitive and flags)
 
     // device state
     DevBuf<double> x, xn, xt, v, xprev, X0, mass, p, g, rhs;
@@ -188,7 +187,6 @@ struct Ctx {
     DevBuf<uint32_t> csPos, csIdx, csHead;
     DevBuf<int> csBoxT, csBoxE, csBoxP;   // constraint-set grid: float boxes per primitive (32-byte records)
     DevBuf<int> csRecT, csRecE, csRecP;   // and in cell order
-    DevBuf<int> ccdTlo, ccdThi, ccdElo, ccdEhi;
     // primitives spanning more than kLargeCells grid cells are kept out of the cell
     // lists and tested by every query directly (flag per primitive + compact list)
     DevBuf<uint8_t> lgFlagT, lgFlagE;
