@@ -76,14 +76,14 @@ struct PrimWork {
 
 // exclusive prefix sum of n uint32 values; total (if not null) written to device memory
 void scan_exclusive(const uint32_t* in, uint32_t* out, long n, uint32_t* total, PrimWork& w, hipStream_t s);
-// stable sort of (key, value) pairs on the low `bits` bits of the keys, no bit set above them
-// (iota: the values are 0, 1, ... and `vals` is room for n of them).  The sorted pairs are
-// either where they were or in the work buffers, valid until the next sort.
+// stable sort of the keys with their positions 0, 1, ..., on the low `bits` bits of the keys,
+// no bit set above them; `vals` is room for n positions.  The sorted pairs are either in
+// `keys` and `vals` or in the work buffers, valid until the next sort.
 struct SortedPairs {
     uint64_t* keys;
     uint32_t* vals;
 };
-SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, PrimWork& w, hipStream_t s, bool iota);
+SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, PrimWork& w, hipStream_t s);
 // deterministic sums: chunks of 256 values folded by halving strides, chunk partials
 // added in chunk order by one thread; result written to device memory `out`
 void chunk_sum(const double* in, long n, double* out, PrimWork& w, hipStream_t s);

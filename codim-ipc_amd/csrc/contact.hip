@@ -594,7 +594,7 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
         uint32_t* si = c.csIdx.ensure((size_t)std::max<uint32_t>(std::max(std::max(nPT, nEE), nDup), 1));
         const uint64_t* dkey = nullptr;
         if (nDup) {
-            dkey = radix_sort_pairs(o.dkey, si, nDup, bits_for((uint64_t)c.nV * c.nV * (c.nV + 1)), c.pw, c.s, true).keys;
+            dkey = radix_sort_pairs(o.dkey, si, nDup, bits_for((uint64_t)c.nV * c.nV * (c.nV + 1)), c.pw, c.s).keys;
             uint32_t* h = c.csHead.ensure(nDup);
             hipLaunchKernelGGL(k_run_flags, dim3(nblocks(nDup)), dim3(kBlock), 0, c.s, dkey, (int)nDup, h);
             CIPC_LAUNCH_CHECK();
@@ -611,12 +611,12 @@ static void constraint_set_impl(Ctx& c, const double* x, DevBuf<int>& out, int& 
             CIPC_LAUNCH_CHECK();
         }
         if (nPT) {
-            const uint32_t* idx = radix_sort_pairs(o.key, si, nPT, bits_for((uint64_t)c.nBN * c.nBT), c.pw, c.s, true).vals;
+            const uint32_t* idx = radix_sort_pairs(o.key, si, nPT, bits_for((uint64_t)c.nBN * c.nBT), c.pw, c.s).vals;
             hipLaunchKernelGGL(k_gather_c4, dim3(nblocks(nPT)), dim3(kBlock), 0, c.s, idx, o.c4, (int)nPT, out.p, nC, 0);
             CIPC_LAUNCH_CHECK();
         }
         if (nEE) {
-            const uint32_t* idx = radix_sort_pairs(oEE.key, si, nEE, bits_for((uint64_t)c.nBE * c.nBE), c.pw, c.s, true).vals;
+            const uint32_t* idx = radix_sort_pairs(oEE.key, si, nEE, bits_for((uint64_t)c.nBE * c.nBE), c.pw, c.s).vals;
             hipLaunchKernelGGL(k_gather_c4, dim3(nblocks(nEE)), dim3(kBlock), 0, c.s, idx, oEE.c4, (int)nEE, out.p, nC, (int)nPT);
             CIPC_LAUNCH_CHECK();
         }
@@ -1118,7 +1118,7 @@ void scatter_local_gradient(Ctx& c, const double* gl, const int* gv, long ns, do
     uint32_t* slot = c.u32c.ensure(ns);
     hipLaunchKernelGGL(k_grad_keys, dim3(nblocks(ns)), dim3(kBlock), 0, c.s, gv, ns, c.nV, skip, key);
     CIPC_LAUNCH_CHECK();
-    const SortedPairs sorted = radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV + 1), c.pw, c.s, true);
+    const SortedPairs sorted = radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV + 1), c.pw, c.s);
     uint32_t* st = c.u32a.ensure(c.nV);
     uint32_t* en = c.u32b.ensure(c.nV);
     CIPC_HIP(hipMemsetAsync(st, 0, c.nV * sizeof(uint32_t), c.s));
@@ -1240,7 +1240,7 @@ void barrier_hessian(Ctx& c, const double* x, const int* C, int nC, double kappa
         friction_hess_local(c, x, fricXn, hl, 16l * nC);
         friction_hess_keys(c, key + 16l * nC);
     }
-    const SortedPairs sorted = radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV * c.nV + 1), c.pw, c.s, true);
+    const SortedPairs sorted = radix_sort_pairs(key, slot, ns, bits_for((uint64_t)c.nV * c.nV + 1), c.pw, c.s);
     const uint64_t* skey = sorted.keys;
     uint32_t* head = c.u32a.ensure(ns);
     uint32_t* pos = c.u32b.ensure(ns);

@@ -206,7 +206,7 @@ __global__ void k_fric_grad_local(const double* __restrict__ x, const double* __
     }
 }
 
-// Hessian blocks of stencil i at slots off + 16 i + 4 a + b of the SoA [9][ns] array
+// Hessian blocks of stencil i at slots off + 16 i + 4 a + b of the [slot][9] array
 __global__ void k_fric_hess_local(const double* __restrict__ x, const double* __restrict__ xn, const int* __restrict__ fC,
                                   const double* __restrict__ fI, int nF, double ev, double mu, double* __restrict__ hl,
                                   long off) {

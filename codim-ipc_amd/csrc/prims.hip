@@ -230,8 +230,8 @@ __global__ void k_rs_scatter(const uint64_t* __restrict__ kin, const uint32_t* _
 // Back to back the counting is a third faster (2 digits cross at 5,000, 3 at 9,600, 4 at
 // 15,000, 1 at 1,900), which sets the lines for 1, 5 and 6 digits in proportion.
 constexpr long kRankSort[] = {0, 1200, 3200, 6400, 9600, 12800, 16000};
-__global__ __launch_bounds__(kBlock) void k_rank_sort(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                      uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, int n) {
+__global__ __launch_bounds__(kBlock) void k_rank_sort(const uint64_t* __restrict__ kin, uint64_t* __restrict__ kout,
+                                                      uint32_t* __restrict__ vout, int n) {
     __shared__ uint32_t part[4][64];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int first = blockIdx.x * 64, i = first + lane;
@@ -250,16 +250,16 @@ __global__ __launch_bounds__(kBlock) void k_rank_sort(const uint64_t* __restrict
     if (w != 0 || i >= n) return;
     r = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
     kout[r] = mine;
-    vout[r] = vin ? vin[i] : (uint32_t)i;
+    vout[r] = (uint32_t)i;
 }
 
-SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, PrimWork& w, hipStream_t s, bool iota) {
+SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, PrimWork& w, hipStream_t s) {
     if (n <= 0) return {keys, vals};
     uint64_t* k2 = w.keyAlt.ensure(n);
     uint32_t* v2 = w.valAlt.ensure(n);
     const int passes = (bits + kMaxDigit - 1) / kMaxDigit, rb = (bits + passes - 1) / passes;
     if (n <= kRankSort[std::min(passes, 6)]) {
-        hipLaunchKernelGGL(k_rank_sort, dim3((unsigned)((n + 63) / 64)), dim3(kBlock), 0, s, keys, iota ? nullptr : vals, k2, v2, (int)n);
+        hipLaunchKernelGGL(k_rank_sort, dim3((unsigned)((n + 63) / 64)), dim3(kBlock), 0, s, keys, k2, v2, (int)n);
         CIPC_LAUNCH_CHECK();
         return {k2, v2};
     }
@@ -272,7 +272,7 @@ SortedPairs radix_sort_pairs(uint64_t* keys, uint32_t* vals, long n, int bits, P
         hipLaunchKernelGGL(k_rs_hist, dim3(nb), dim3(kBlock), 0, s, ka, n, rb * p, (1u << rb) - 1, hist, nb);
         CIPC_LAUNCH_CHECK();
         scan_exclusive(hist, hs, (long)nb << rb, nullptr, w, s);
-        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(kBlock), 0, s, ka, p == 0 && iota ? nullptr : va, kb, vb, n, rb * p, rb, hs, nb);
+        hipLaunchKernelGGL(k_rs_scatter, dim3(nb), dim3(kBlock), 0, s, ka, p == 0 ? nullptr : va, kb, vb, n, rb * p, rb, hs, nb);
         CIPC_LAUNCH_CHECK();
         std::swap(ka, kb);
         std::swap(va, vb);
