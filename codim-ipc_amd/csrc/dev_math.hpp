@@ -416,7 +416,8 @@ CIPC_DEV constexpr double tr_basis(int k, int a) {
 }
 
 // a <- V diag(max(lambda, 0)) V^T of the leading R x R part of a symmetric matrix (upper
-// triangle, a(i, j) at upk(N, i, j)): cyclic Jacobi in registers, off^2 <= 1e-24 ||.||_F^2.
+// triangle, a(i, j) at upk(N, i, j)): cyclic Jacobi in registers until off^2 <= 1e-24
+// ||.||_F^2 (FAST: 1e-26).
 // One matrix per thread holds R (R + 1) / 2 + R^2 doubles, which leaves one wave per SIMD
 // and nothing to hide the latency of a rotation's angle behind: three divisions and two
 // square roots one after the other, longer than the updates.  Rotations of zero entries are
@@ -426,14 +427,18 @@ CIPC_DEV constexpr double tr_basis(int k, int a) {
 // reciprocals and square roots (the matrix is scaled by a power of two first, so that its
 // entries are FP32 numbers), c from one cubic step on an FP32 reciprocal square root in FP64
 // (relative error 1e-20 before rounding), and the rotated pair keeps its true off-diagonal
-// entry (1e-7 of the old one, which the next sweep takes) instead of being set to zero.
+// entry (1e-7 of the old one, which the next sweep takes) instead of being set to zero.  What
+// is left out of the diagonal at the end bounds the error of the positive part (a projection
+// onto a convex cone), so FAST stops at a tenth of the other's rest: largest error of one
+// constraint against the oracle 1.7e-13 of its block, medians 0.8 to 1.6e-15, over every kind
+// of constraint and stiffnesses over 12 decades; FP64 angles at 1e-24 1.0e-12, 1.1 to 2.2e-15.
 // The contacts take it.  The hinges keep correctly rounded angles: on scenes without
 // contact a Newton step that stops near its tolerance turns the last bits of the Hessian
 // into differences of the size of that tolerance, so their results stay as they were (the
 // fused multiply-adds are written out for the same reason).
 // Measured: 480,000 hinges 1,089 -> 870 us without the branches and with block rows written
-// through LDS (below); of 400 spectra (indefinite, rank deficient, scales of 1e-9 to 1e9) the
-// FAST form's largest error against extended precision is 5.8e-13 ||.||, the other's 9.0e-13.
+// through LDS (below); contacts with FAST against FP64 angles 1,873 -> 1,353 us (1.25 million),
+// 328 -> 236 (184,000), 107 -> 71 (20 contacts); the tenth of the rest costs 2% of it.
 template <int R, int N, bool FAST>
 CIPC_DEV void jacobi_psd(double* a) {
     int ex = 0;
@@ -459,7 +464,7 @@ CIPC_DEV void jacobi_psd(double* a) {
     for (int i = 0; i < R; ++i)
 #pragma unroll
         for (int j = i; j < R; ++j) fro += (i == j ? 1.0 : 2.0) * a[upk(N, i, j)] * a[upk(N, i, j)];
-    const double tol = 1e-24 * fro;
+    const double tol = (FAST ? 1e-26 : 1e-24) * fro;
     for (int sweep = 0; sweep < 16; ++sweep) {
         double offd = 0;
 #pragma unroll
