@@ -92,7 +92,12 @@ static void upload_x(cipc_ctx* ctx, DevBuf<double>& b, const double* h, size_t n
     b.ensure(n);
     CIPC_HIP(hipMemcpyAsync(b.p, h, n * sizeof(double), hipMemcpyHostToDevice, ctx->c.s));
 }
-// constraints arrive as int4 rows; the device keeps them SoA [4][n]
+// constraints arrive as int4 rows; the device keeps them SoA [4][n].  Up to kHostRows rows the
+// host transposes: a kernel behind the copy costs the call up to 10 us, the host's pass 0.6 us
+// per 1,000 rows (barrier energy of 10 / 4,000 / 10,000 / 16,000 / 24,000 / 40,000 rows, us:
+// host 55 / 57 / 60 / 64 / 75 / 95, device 57 / 67 / 68 / 71 / 74 / 84; the gradient crosses
+// between 14,000 and 20,000).
+constexpr int kHostRows = 16384;
 // Every entry of the reference encoding is a vertex v, a -v-1, a -multiplicity or -1
 // (IPC.h:144-661), so all lie in [-nV, nV); anything else would be read out of bounds on
 // the device and is rejected here (CIPC_E_INVALID through guarded()).
@@ -110,10 +115,16 @@ static void upload_cs(cipc_ctx* ctx, const int32_t* cs, int32_t n) {
             if (cs[i] < -nV || cs[i] >= nV)
                 throw std::invalid_argument("constraint " + std::to_string(i / 4) + " has an entry outside [-n_vertices, n_vertices)");
     ctx->qC.ensure(std::max<size_t>(m, 4));
-    if (n > 0) {
+    std::vector<int> soa;   // must outlive the copy
+    if (n > kHostRows) {
         int* rows = ctx->qRows.ensure(m);
         CIPC_HIP(hipMemcpyAsync(rows, cs, m * sizeof(int), hipMemcpyHostToDevice, ctx->c.s));
         constraint_rows(ctx->c, ctx->qC.p, rows, n, false);
+    } else if (n > 0) {
+        soa.resize(m);
+        for (int i = 0; i < n; ++i)
+            for (int k = 0; k < 4; ++k) soa[(size_t)k * n + i] = cs[4 * (size_t)i + k];
+        CIPC_HIP(hipMemcpyAsync(ctx->qC.p, soa.data(), m * sizeof(int), hipMemcpyHostToDevice, ctx->c.s));
     }
     // also for an empty set: the uploads before it (upload_x) may be in flight from the
     // caller's pinned memory, and a call that has nothing to compute returns from here
