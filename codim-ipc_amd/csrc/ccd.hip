@@ -423,7 +423,7 @@ __global__ __launch_bounds__(kBlock) void k_ccd_walk(P T, int n, double alpha0, 
 // reference does); same voxel-overlap candidate rule and cell coverage as the edge walk.  One
 // particle per thread; the voxel box of an edge comes with its cell record.  CCD call of a
 // sheet with 1,680 / 4,800 rod segments and 441 / 3,600 particles, against six strided loads
-// of the box: 616 -> 541, 659 -> 568 us.
+// of the box: 616 -> 541, 659 -> 568 us (the kernel at the larger one 236 us).
 __device__ __forceinline__ void pe_ccd_candidate(const double* __restrict__ x, const double* __restrict__ p, const int* __restrict__ bEdge,
                                                  int nBE, const uint8_t* __restrict__ dbc, const int4& ba, const int4& bb, int vI,
                                                  const int4& qa, const int4& qb, d3 P, d3 dP, int e, double xi, double& largest) {

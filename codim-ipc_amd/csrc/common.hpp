@@ -121,8 +121,10 @@ __device__ __forceinline__ float dpp_move(float v) {
 }
 // sum over aligned groups of LANES (2, 4, 8 or 16) lanes, in every lane of the group.  A row
 // of 16: rotations by 8, 4, 2, 1 -- after the rotation by 8 the values repeat every 8 lanes,
-// so each next rotation meets the partner of an xor butterfly.  Shorter groups: the mirrored
-// half row, then quad permutations (lanes ^ 2, lanes ^ 1).
+// so each next rotation meets the partner of an xor butterfly.  Eight lanes start with the
+// mirrored half row (lane i and 7 - i, another association than lanes ^ 4), four and two with
+// the quad permutations (lanes ^ 2, lanes ^ 1).  Every lane of a group adds the same pairs in
+// every step, so all hold the same bits, and a launch shape gives the same bits every time.
 template <int LANES, class V>
 __device__ __forceinline__ V lane_sum(V v) {
     static_assert(LANES == 2 || LANES == 4 || LANES == 8 || LANES == 16, "");

@@ -341,7 +341,9 @@ static auto spmv_kernel(int lanes, int unr, bool withP) -> decltype(&k_pcg_spmv<
 // per block cost more than the second launch.)
 // Partials: partS = [2][workgroups] of p.q, q.u; partU = [2][workgroups] of r.z, r.r,
 // double-buffered (an update reads the previous one's while it writes its own).
-// CON: whether there are contact blocks (without, their row bounds are not read).
+// CON: whether there are contact blocks; without, their row bounds are not read, which is 1
+// to 2% of an iteration (us, with / without reading them: 4,247 vertices FP64 8.91 / 8.78,
+// 33,169 FP64 15.3 / 15.1, 164,170 FP32 blocks 33.2 / 32.5).
 template <class M, class V, int LANES, int BS, bool CON, int UNR>
 __global__ __launch_bounds__(BS) void k_pcg_spmv_p(const int* __restrict__ erp, const int* __restrict__ ecol, const M* __restrict__ ev,
                                                    int enz, const int* __restrict__ crp, const int* __restrict__ ccol,
